@@ -244,6 +244,27 @@ void svd_run(SvdPlan *plan, const float *A, const float *sketch, uint64_t seed, 
 // `minuend` is not null.
 void launch_reconstruct(const float *U, const float *S, const float *V, int m, int n, int k,
                         const float *minuend, float *out, hipStream_t stream);
+// Products of the range finder on the f16 matrix cores with every FP32 value
+// carried as two f16 pieces (gemm_h2.hip).  H2Scales: the exact power-of-two
+// scales of a matrix's rows, device memory (exponent, scale, inverse: one per
+// row; emax, common: one).
+struct H2Scales {
+    int *exponent = nullptr;
+    float *scale = nullptr;
+    float *inverse = nullptr;
+    int *emax = nullptr;
+    float *common = nullptr;
+};
+bool h2_supported(int K);
+uint64_t h2_workspace_bytes(int M, int N, int K);
+uint64_t h2_plane_units(int K, int N);
+void launch_h2_scales(const float *A, int m, int n, const H2Scales &s, hipStream_t stream);
+// C = A B (ta false: m x n times n x q) or A^T B (n x m times m x q), A
+// row-major m x n, B and C row-major with q columns; B's entries below 32 in
+// magnitude.
+void launch_h2_gemm(bool ta, int m, int n, int q, const float *A, const H2Scales &s, const float *B, uint16_t *planes,
+                    float *C, float *workspace, uint64_t workspace_bytes, hipStream_t stream);
+
 // N(0, 1) draws: Philox4x32-10 counter-based generator + Box-Muller.
 void launch_gaussian_fill(float *out, uint64_t n, uint64_t seed, hipStream_t stream);
 

@@ -6,9 +6,10 @@
 //     op(B) = B          (TB = false, B is K x N, ldb >= N)
 //           = B^T        (TB = true,  B is N x K, ldb >= K)
 //
-// Used for the randomised range finder (X = op(A) R, Y = op(A)^T X with the
-// big activation matrix read row-major in place, so no transposed copy is
-// ever made), the small basis rotations (X * W) and the low-rank
+// Used for the small basis rotations (X * W), for the range finder's product
+// with a caller's sketch and its products with matrices narrower than 64
+// (the others run in gemm_h2.hip; the big activation matrix is read row-major
+// in place, so no transposed copy is ever made), and for the low-rank
 // reconstruction U diag(S) V^T, which scales the A fragments by S (fetched a
 // slice ahead with the operand tiles) and can subtract from a minuend in the
 // epilogue (error = residual - U S V^T).

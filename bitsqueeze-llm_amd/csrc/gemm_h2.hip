@@ -1,0 +1,511 @@
+// Products with the big activation matrix on the f16 matrix cores, each FP32
+// operand value carried as two f16 pieces (v_mfma_f32_32x32x16_f16).
+//
+//   C[M x N] = op(A)[M x K] * B[K x N]     (row-major, FP32 in and out)
+//     op(A) = A    (TA = false, A is M x K)      the range finder's A_w B and
+//     op(A) = A^T  (TA = true,  A is K x M)      A_w^T B, A read in place
+//
+// Split.  A value x, scaled by an exact power of two s, is h + l 2^-11 with
+// h = f16(s x) and l = f16(2^11 (s x - h)): 22 bits and a sign, the rest at
+// most half a unit in the last place of FP32.  The product sums
+//     hi += h_a h_b          lo += h_a l_b + l_a h_b
+// in FP32 accumulators of their own and is hi + 2^-11 lo; the dropped
+// l_a l_b is 2^-24 of the product or less, with either sign.  Keeping the two
+// sums apart keeps l a normal f16 down to 2^-29 of the scaled maximum and
+// adds the small terms without rounding them into the large sum.  Against
+// 64-bit sums the error is 0.35 to 0.9 times that of a
+// v_mfma_f32_16x16x4f32 chain of the same length (K = 32 .. 11008; normal,
+// lognormal, one-signed and decaying operands, and a column 10^6 times the
+// others that B does not touch).
+// Three f16 products run at up to 5 times the FP32 matrix rate (2.5 / 3
+// against 0.157 PFLOP/s).  Measured, against the FP32 kernels with their
+// reductions: 4096 x 11008 with q = 128 101 -> 49 us (A^T B) and 98 -> 49 us
+// (A B); 16384 x 14336 with q = 512 1986 -> 1033 and 1590 -> 872 us (0.83
+// PFLOP/s of f16 products, two thirds of what a large library f16 product
+// reaches on this card: the staging's LDS traffic and the power limit are
+// what is left).
+//
+// Scales.  Row i of A is scaled so that its largest magnitude falls in
+// [2^14, 2^15) (row_scale_kernel, once per matrix).  With TA = false that is
+// a scale per row of C, undone with the partial sums' reduction.  With TA =
+// true the rows run along K: B's row i takes the inverse power times
+// 2^(E_max) (E_max the exponent of the largest entry of A), so the product
+// needs one common factor.  B (an orthonormal basis or the sketch, entries
+// below 32) is scaled by 2^11 and split ahead (split_b_kernel) into planes
+// [k / 8][column][8] whose 16-byte units go to LDS as they lie; A is split as
+// it is staged.  All scalings are exact.  Rows holding infinities or NaN give
+// NaN results, as sums over them do.
+#include "bsq_internal.hpp"
+#include "tile_map.hpp"
+
+#include <algorithm>
+
+namespace bsq {
+namespace {
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) void lds_void_t;
+typedef __attribute__((address_space(1))) void glb_void_t;
+
+constexpr int kThreads = 256;
+constexpr int T = 128;        // output tile
+constexpr int BK = 32;        // K slice
+constexpr int KG = BK / 8;    // groups of eight k per slice
+constexpr int kPitchA = 132;  // 16-byte units per k group of a staged A plane (128 rows, padded)
+constexpr int kScaleB = 11;   // B's scale, a power of two
+constexpr float kLo = 2048.0f, kLoInv = 1.0f / 2048.0f;
+
+// exponent of the largest magnitude of a row: in [-112, 127] (a zero row, or
+// one below 2^-112, takes -112; a row with infinities or NaN 127)
+__device__ __forceinline__ int row_exponent(float absmax) {
+    const int e = static_cast<int>(__float_as_uint(absmax) >> 23) - 127;
+    return min(max(e, -112), 127);
+}
+
+// 2^e, e in [-149, 127]
+__device__ __forceinline__ float pow2(int e) { return __builtin_ldexpf(1.0f, e); }
+
+// eight values to their f16 pieces: h the leading ones, l the scaled rests
+__device__ __forceinline__ void split8(const float (&y)[8], u32x4 &h, u32x4 &l) {
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+        const f16x2 hp{static_cast<_Float16>(y[2 * p]), static_cast<_Float16>(y[2 * p + 1])};
+        const f16x2 lp{static_cast<_Float16>((y[2 * p] - static_cast<float>(hp.x)) * kLo),
+                       static_cast<_Float16>((y[2 * p + 1] - static_cast<float>(hp.y)) * kLo)};
+        h[p] = __builtin_bit_cast(uint32_t, hp);
+        l[p] = __builtin_bit_cast(uint32_t, lp);
+    }
+}
+
+__device__ __forceinline__ void dma16(const u32x4 *g, const u32x4 *l) {
+    __builtin_amdgcn_global_load_lds((glb_void_t *)(g), (lds_void_t *)(reinterpret_cast<size_t>(l)), 16, 0, 0);
+}
+
+// all LDS operations of this wave and all but its PENDING newest vector
+// memory operations are done, then the workgroup barrier
+template <int PENDING>
+__device__ __forceinline__ void stage_barrier() {
+    static_assert(PENDING >= 0 && PENDING < 64, "vmcnt has six bits");
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0x070 | (PENDING & 15) | ((PENDING >> 4) << 14));
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+// Row exponents and scales of a row-major matrix: rs[i] = 2^(14 - E_i) scales
+// row i into f16's range, ri[i] = 2^(E_i - 14 - kScaleB) undoes it together
+// with B's scale.  One workgroup per row: the matrix is read once, at the
+// rate of a copy's reads.
+__global__ __launch_bounds__(kThreads) void row_scale_kernel(const float *__restrict__ A, int cols, int *__restrict__ E,
+                                                             float *__restrict__ rs, float *__restrict__ ri) {
+    __shared__ uint32_t wmax[kThreads / 64];
+    const int r = blockIdx.x, tid = threadIdx.x;
+    const float *row = A + static_cast<uint64_t>(r) * cols;
+    uint32_t m = 0;  // bit patterns of magnitudes order as the magnitudes do, NaN above infinity
+    const int head = min(cols, static_cast<int>((16 - (reinterpret_cast<uintptr_t>(row) & 15u)) & 15u) / 4);
+    if (tid < head) m = __float_as_uint(fabsf(row[tid]));
+    const float4 *q = reinterpret_cast<const float4 *>(row + head);
+    const int n4 = (cols - head) / 4;
+#pragma unroll 4
+    for (int i = tid; i < n4; i += kThreads) {
+        const float4 v = q[i];
+        m = max(max(m, __float_as_uint(fabsf(v.x))), __float_as_uint(fabsf(v.y)));
+        m = max(max(m, __float_as_uint(fabsf(v.z))), __float_as_uint(fabsf(v.w)));
+    }
+    const int t0 = head + 4 * n4;
+    if (tid < cols - t0) m = max(m, __float_as_uint(fabsf(row[t0 + tid])));
+    for (int off = 32; off >= 1; off >>= 1) m = max(m, static_cast<uint32_t>(__shfl_xor(static_cast<int>(m), off)));
+    if ((tid & 63) == 0) wmax[tid >> 6] = m;
+    __syncthreads();
+    if (tid == 0) {
+        m = max(max(wmax[0], wmax[1]), max(wmax[2], wmax[3]));
+        const int e = row_exponent(__uint_as_float(m));
+        E[r] = e;
+        rs[r] = pow2(14 - e);
+        ri[r] = pow2(e - 14 - kScaleB);
+    }
+}
+
+// emax[0] = max_i E[i], and pow2(emax - 14 - kScaleB) beside it (one workgroup)
+__global__ __launch_bounds__(1024) void scale_max_kernel(const int *__restrict__ E, int rows, int *__restrict__ emax,
+                                                         float *__restrict__ common) {
+    __shared__ int wmax[16];
+    int m = -112;
+    for (int i = threadIdx.x; i < rows; i += 1024) m = max(m, E[i]);
+    for (int off = 32; off >= 1; off >>= 1) m = max(m, __shfl_xor(m, off));
+    if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < 16; ++w) m = max(m, wmax[w]);
+        *emax = m;
+        *common = pow2(m - 14 - kScaleB);
+    }
+}
+
+// The first 8 kgroups rows of B (N columns, row-major) into its two planes,
+// [k / 8][np][8] f16 each, zero beyond column N: entry (k, n) times 2^kScaleB, and with E given also times
+// 2^(E[k] - *emax).  One lane per column and group of eight k.
+__global__ __launch_bounds__(kThreads) void split_b_kernel(const float *__restrict__ B, int N, int np, int kgroups,
+                                                           const int *__restrict__ E, const int *__restrict__ emax,
+                                                           u32x4 *__restrict__ hi, u32x4 *__restrict__ lo) {
+    const int t = blockIdx.x * kThreads + threadIdx.x;
+    const int kg = t / np, n = t - kg * np;
+    if (kg >= kgroups) return;
+    float y[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        y[i] = n < N ? B[static_cast<uint64_t>(8 * kg + i) * N + n] : 0.0f;
+    }
+    if (E) {
+        const int em = *emax;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) y[i] = __builtin_ldexpf(y[i], E[8 * kg + i] - em + kScaleB);
+    } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) y[i] *= static_cast<float>(1 << kScaleB);
+    }
+    u32x4 h, l;
+    split8(y, h, l);
+    hi[t] = h;
+    lo[t] = l;
+}
+
+struct H2Args {
+    const float *A;
+    const u32x4 *bh, *bl;  // B's planes
+    const float *rs;       // scales of A's rows
+    float *ws;             // partial tiles [tile][part][T][T]
+    int M, K, lda;
+    int np;                // columns of the planes (a multiple of 64)
+    int tiles_n;           // output tiles per row of tiles
+    int pairs;             // pairs of K slices per tile
+    int units;             // tiles x pairs
+    int maxparts;          // workspace slots per tile
+};
+
+// logical workgroup whose range holds unit u
+__host__ __device__ __forceinline__ int h2_owner(int64_t u, int64_t units, int G) {
+    return static_cast<int>(((u + 1) * G - 1) / units);
+}
+
+// Stream-K: G workgroups share the tiles' K slices in equal contiguous
+// ranges, one range a workgroup, laid so that an XCD runs a contiguous eighth
+// of them; each writes its partial sum of every tile it touches and
+// h2_reduce_kernel adds a tile's parts in order.  128 x 128 tiles, four waves
+// of 64 x 64 in 32 x 32 blocks with both sums in accumulator registers (128
+// of 256 a lane), so two workgroups share a CU and one's staging and barriers
+// run under the other's matrix instructions.  Slices of 32 k: B's pieces go
+// global -> LDS directly one slice ahead; A's values are fetched into
+// registers two slices ahead (row-major: a lane takes eight consecutive k of
+// two rows; A^T: eight k-rows of two columns, so the transposition is only a
+// choice of registers), then split and written to LDS in the same
+// [k group][row] units of 16 bytes that the fragments are read in.
+template <bool TA>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_h2_kernel(H2Args g) {
+    __shared__ u32x4 a0[2 * KG * kPitchA], a1[2 * KG * kPitchA];  // h plane, l plane
+    __shared__ __attribute__((aligned(1024))) u32x4 b0[2 * KG * T], b1[2 * KG * T];
+    constexpr int kLoadsA = TA ? 18 : 6;  // vector loads of one A slice and its scales, at least
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int wm0 = (wave >> 1) * 64, wn0 = (wave & 1) * 64;
+    const int G = static_cast<int>(gridDim.x), bid = static_cast<int>(blockIdx.x);
+    const int xcd = bid % kXcds, loc = bid / kXcds;
+    const int L = xcd * (G / kXcds) + min(xcd, G % kXcds) + loc;
+    const int p0 = static_cast<int>(static_cast<int64_t>(L) * g.units / G);
+    const int n = static_cast<int>(static_cast<int64_t>(L + 1) * g.units / G) - p0;  // slice pairs
+
+    // a position in the slices of the range (tile row, tile column, slice),
+    // `left` slices before its last
+    struct Cursor {
+        int tm, tn, ks, left;
+        __device__ __forceinline__ void next(int nk, int tiles_n) {
+            // by selects: branches here would split the accumulators' live ranges
+            const int step = left > 0 ? 1 : 0;
+            left -= step;
+            const int w = ks + step == nk ? 1 : 0;
+            ks = w ? 0 : ks + step;
+            const int w2 = tn + w == tiles_n ? 1 : 0;
+            tn = w2 ? 0 : tn + w;
+            tm += w2;
+        }
+    };
+    const int nk = 2 * g.pairs, tile0 = p0 / g.pairs;
+    Cursor ca{tile0 / g.tiles_n, tile0 % g.tiles_n, 2 * (p0 - tile0 * g.pairs), 2 * n - 1};  // next A slice to fetch
+    Cursor cb = ca;                                                                       // next B slice to fetch
+
+    float va[16];  // A values in flight
+    float vs[TA ? 8 : 2];
+    auto load_a = [&]() __attribute__((always_inline)) {
+        const int m0 = ca.tm * T, k0 = ca.ks * BK;
+        asm volatile("" ::: "memory");  // stays behind the DMA before it
+        if constexpr (!TA) {
+            const int r0 = min(m0 + (tid >> 2), g.M - 1), r1 = min(m0 + 64 + (tid >> 2), g.M - 1);
+            const int k = k0 + 8 * (tid & 3);
+            vs[0] = g.rs[r0];
+            vs[1] = g.rs[r1];
+            const float *p0 = g.A + static_cast<uint64_t>(r0) * g.lda + k, *p1 = g.A + static_cast<uint64_t>(r1) * g.lda + k;
+            // rows may start at any multiple of four bytes
+            __builtin_memcpy(&va[0], __builtin_assume_aligned(p0, 4), 32);
+            __builtin_memcpy(&va[8], __builtin_assume_aligned(p1, 4), 32);
+        } else {
+            const int c0 = min(m0 + lane, g.M - 1), c1 = min(m0 + 64 + lane, g.M - 1);
+            const int k = k0 + 8 * wave;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) vs[i] = g.rs[k + i];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const float *p = g.A + static_cast<uint64_t>(k + i) * g.lda;
+                va[i] = p[c0];
+                va[8 + i] = p[c1];
+            }
+        }
+        ca.next(nk, g.tiles_n);
+    };
+    auto stage_a = [&](u32x4 *as) __attribute__((always_inline)) {
+        const int row = TA ? lane : tid >> 2, kg = TA ? wave : tid & 3;
+        // the values are first touched here: their scaling, moved up past the
+        // barrier, would wait for them a slice early
+#pragma unroll
+        for (int i = 0; i < 16; ++i) asm volatile("" : "+v"(va[i]));
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+            float y[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) y[i] = va[8 * half + i] * (TA ? vs[i] : vs[half]);
+            u32x4 h, l;
+            split8(y, h, l);
+            as[kg * kPitchA + 64 * half + row] = h;
+            as[(KG + kg) * kPitchA + 64 * half + row] = l;
+        }
+    };
+    auto dma_b = [&](const u32x4 *bs) __attribute__((always_inline)) {  // wave w: k group w of both planes
+        const int n0 = cb.tn * T;
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+            const int nc = min(n0 + 64 * half, g.np - 64);  // beyond the planes: results not stored
+            const uint64_t src = static_cast<uint64_t>(cb.ks * KG + wave) * g.np + nc + lane;
+            dma16(g.bh + src, bs + wave * T + 64 * half);
+            dma16(g.bl + src, bs + (KG + wave) * T + 64 * half);
+        }
+        asm volatile("" ::: "memory");
+        cb.next(nk, g.tiles_n);
+    };
+
+    f32x16 hi[2][2], lo[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) hi[i][j] = lo[i][j] = f32x16{};
+
+    struct Frags {
+        f16x8 ah[2], al[2], bh[2], bl[2];
+    };
+    auto fetch = [&](Frags &f, const u32x4 *as, const u32x4 *bs, int s) __attribute__((always_inline)) {
+        const int kg = 2 * s + (lane >> 5), r = lane & 31;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            f.ah[i] = __builtin_bit_cast(f16x8, as[kg * kPitchA + wm0 + 32 * i + r]);
+            f.bh[i] = __builtin_bit_cast(f16x8, bs[kg * T + wn0 + 32 * i + r]);
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            f.al[i] = __builtin_bit_cast(f16x8, as[(KG + kg) * kPitchA + wm0 + 32 * i + r]);
+            f.bl[i] = __builtin_bit_cast(f16x8, bs[(KG + kg) * T + wn0 + 32 * i + r]);
+        }
+    };
+    auto multiply = [&](const Frags &f) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) hi[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.ah[i], f.bh[j], hi[i][j], 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) lo[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.ah[i], f.bl[j], lo[i][j], 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) lo[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.al[i], f.bh[j], lo[i][j], 0, 0, 0);
+    };
+
+    int c_tile = tile0, c_pr = p0 - tile0 * g.pairs;
+    // after a pair: at the tile's or the range's end the partial tile goes out
+    auto pair_done = [&](int j) __attribute__((always_inline)) {
+        ++c_pr;
+        const bool tile_end = c_pr == g.pairs;
+        if (tile_end || j + 1 == n) {  // uniform
+            const int first = h2_owner(static_cast<int64_t>(c_tile) * g.pairs, g.units, G);
+            // 16-byte units in accumulator order: [wave][i][jj][q / 4][lane]
+            uint32_t unit = static_cast<uint32_t>(wave) * 1024u + static_cast<uint32_t>(lane);
+            asm volatile("" : "+v"(unit));  // the addresses are formed here, not held through the loop
+            f32x4 *W = reinterpret_cast<f32x4 *>(g.ws) +
+                       (static_cast<uint64_t>(c_tile) * g.maxparts + (L - first)) * (T * T / 4) + unit;
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int jj = 0; jj < 2; ++jj) {
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        f32x4 v;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) v[e] = hi[i][jj][4 * q + e] + lo[i][jj][4 * q + e] * kLoInv;
+                        W[((2 * i + jj) * 4 + q) * 64] = v;
+                    }
+                    hi[i][jj] = lo[i][jj] = f32x16{};
+                }
+        }
+        c_pr = tile_end ? 0 : c_pr;
+        c_tile += tile_end ? 1 : 0;
+    };
+
+    // a slice: its A and B are in the current stage once every wave has
+    // passed the barrier, which also frees the other stage (read one slice
+    // ago); the next slice's A is in registers or in flight behind this
+    // slice's B (and is staged before B's next transfers are issued: the
+    // compiler's wait for it takes everything in flight).  Nothing in the loop is conditional but the partial tile's
+    // way out: past the range's end the fetches repeat its last slice.
+    auto slice = [&](u32x4 *ac, u32x4 *bc, u32x4 *an, u32x4 *bn) __attribute__((always_inline)) {
+        stage_barrier<kLoadsA>();
+        Frags f0, f1;
+        fetch(f0, ac, bc, 0);
+        stage_a(an);
+        dma_b(bn);
+        load_a();
+        fetch(f1, ac, bc, 1);
+        multiply(f0);
+        multiply(f1);
+    };
+    if (n <= 0) return;  // uniform (G <= units: does not occur)
+    load_a();
+    dma_b(b0);
+    stage_a(a0);
+    load_a();
+    for (int j = 0; j < n; ++j) {
+        slice(a0, b0, a1, b1);
+        slice(a1, b1, a0, b0);
+        pair_done(j);
+    }
+    // no transfer into LDS outlives the workgroup
+    stage_barrier<0>();
+}
+
+// C = the sum of each tile's parts in order, times the row's (ri) or the
+// common factor, plus the k past the last whole pair of slices (fewer than 64, summed
+// in FP32 from A and B themselves).  A lane takes one 16-byte unit of the
+// parts: four consecutive rows of a column, 32 lanes 32 columns.
+template <bool TA>
+__global__ __launch_bounds__(256) void h2_reduce_kernel(H2Args g, int G, int N, const float *__restrict__ B,
+                                                        const float *__restrict__ ri, const float *__restrict__ common,
+                                                        float *__restrict__ C) {
+    constexpr int kUnits = T * T / 4;
+    const int tile = static_cast<int>(blockIdx.x) / (kUnits / 256);
+    const int unit = (static_cast<int>(blockIdx.x) % (kUnits / 256)) * 256 + threadIdx.x;
+    const int64_t ub = static_cast<int64_t>(tile) * g.pairs;
+    const int parts = h2_owner(ub + g.pairs - 1, g.units, G) - h2_owner(ub, g.units, G) + 1;
+    const int tm = tile / g.tiles_n, tn = tile - tm * g.tiles_n;
+    const int lane = unit & 63, q = (unit >> 6) & 3, jj = (unit >> 8) & 1, i = (unit >> 9) & 1, wave = unit >> 10;
+    const int gi = tm * T + (wave >> 1) * 64 + 32 * i + 8 * q + 4 * (lane >> 5);
+    const int gj = tn * T + (wave & 1) * 64 + 32 * jj + (lane & 31);
+    if (gi >= g.M || gj >= N) return;
+    const f32x4 *W = reinterpret_cast<const f32x4 *>(g.ws) + static_cast<uint64_t>(tile) * g.maxparts * kUnits + unit;
+    f32x4 s = W[0];
+#pragma unroll 4
+    for (int p = 1; p < parts; ++p) s += W[static_cast<uint64_t>(p) * kUnits];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int r = min(gi + e, g.M - 1);
+        float v = s[e] * (TA ? *common : ri[r]);
+        for (int k = g.pairs * 2 * BK; k < g.K; ++k) {
+            const float a = TA ? g.A[static_cast<uint64_t>(k) * g.lda + r] : g.A[static_cast<uint64_t>(r) * g.lda + k];
+            v = fmaf(a, B[static_cast<uint64_t>(k) * N + gj], v);
+        }
+        if (gi + e < g.M) C[static_cast<uint64_t>(r) * N + gj] = v;
+    }
+}
+
+struct H2Plan {
+    int tiles, tiles_n, pairs, units, G, maxparts;
+    uint64_t bytes;  // partial tiles
+};
+
+// Two workgroups per CU share the slices, unless that leaves a workgroup
+// fewer than four pairs of them (256 k): the parts' traffic and the serial sum of
+// a tile's parts then cost more than the idle CUs.
+H2Plan h2_plan(int M, int N, int K) {
+    H2Plan p{};
+    p.tiles_n = static_cast<int>(ceil_div(N, T));
+    p.tiles = static_cast<int>(ceil_div(M, T)) * p.tiles_n;
+    p.pairs = K / (2 * BK);  // the rest of K goes with the reduction
+    p.units = p.tiles * p.pairs;
+    const int most = 2 * cu_count();
+    p.G = std::max(1, std::min(most, std::max(p.tiles, p.units / 4)));
+    p.G = std::min(p.G, p.units);
+    p.maxparts = 1;
+    for (int t = 0; t < p.tiles; ++t) {
+        const int64_t b = static_cast<int64_t>(t) * p.pairs;
+        p.maxparts = std::max(p.maxparts, h2_owner(b + p.pairs - 1, p.units, p.G) - h2_owner(b, p.units, p.G) + 1);
+    }
+    p.bytes = static_cast<uint64_t>(p.tiles) * p.maxparts * T * T * sizeof(float);
+    return p;
+}
+
+int pad64(int n) { return static_cast<int>(ceil_div(n, 64) * 64); }
+
+}  // namespace
+
+// Bytes of the partial tiles of an M x N x K product.
+uint64_t h2_workspace_bytes(int M, int N, int K) { return h2_plan(M, N, K).bytes; }
+
+// f16 values of the two planes of a K x N operand B.
+uint64_t h2_plane_units(int K, int N) { return static_cast<uint64_t>(K / (2 * BK)) * 2 * BK * pad64(N) * 2; }
+
+bool h2_supported(int K) { return K >= 2 * BK; }
+
+void launch_h2_scales(const float *A, int m, int n, const H2Scales &s, hipStream_t stream) {
+    BSQ_REQUIRE(A && m > 0 && n > 0 && s.exponent && s.scale && s.inverse && s.emax && s.common, "h2 scales: bad arguments");
+    row_scale_kernel<<<static_cast<unsigned>(m), kThreads, 0, stream>>>(A, n, s.exponent, s.scale, s.inverse);
+    BSQ_HIP(hipGetLastError());
+    scale_max_kernel<<<1, 1024, 0, stream>>>(s.exponent, m, s.emax, s.common);
+    BSQ_HIP(hipGetLastError());
+}
+
+void launch_h2_gemm(bool ta, int m, int n, int q, const float *A, const H2Scales &s, const float *B, uint16_t *planes,
+                    float *C, float *workspace, uint64_t workspace_bytes, hipStream_t stream) {
+    const int M = ta ? n : m, K = ta ? m : n;
+    BSQ_REQUIRE(M > 0 && q > 0 && h2_supported(K) && A && B && C && planes && workspace, "h2 gemm: bad arguments");
+    const H2Plan p = h2_plan(M, q, K);
+    BSQ_REQUIRE(p.bytes <= workspace_bytes, "h2 gemm: workspace too small");
+    H2Args g{};
+    const int np = pad64(q), kgroups = p.pairs * 2 * KG;
+    g.A = A;
+    auto *bh = reinterpret_cast<u32x4 *>(planes);
+    auto *bl = bh + static_cast<uint64_t>(kgroups) * np;
+    g.bh = bh;
+    g.bl = bl;
+    g.rs = s.scale;
+    g.ws = workspace;
+    g.M = M;
+    g.K = K;
+    g.lda = n;
+    g.np = np;
+    g.tiles_n = p.tiles_n;
+    g.pairs = p.pairs;
+    g.units = p.units;
+    g.maxparts = p.maxparts;
+    split_b_kernel<<<static_cast<unsigned>(ceil_div(static_cast<uint64_t>(kgroups) * np, kThreads)), kThreads, 0, stream>>>(
+        B, q, np, kgroups, ta ? s.exponent : nullptr, s.emax, bh, bl);
+    BSQ_HIP(hipGetLastError());
+    const dim3 grid(static_cast<unsigned>(p.G)), rgrid(static_cast<unsigned>(p.tiles * (T * T / 4 / 256)));
+    if (ta) gemm_h2_kernel<true><<<grid, kThreads, 0, stream>>>(g);
+    else gemm_h2_kernel<false><<<grid, kThreads, 0, stream>>>(g);
+    BSQ_HIP(hipGetLastError());
+    if (ta) h2_reduce_kernel<true><<<rgrid, 256, 0, stream>>>(g, p.G, q, B, nullptr, s.common, C);
+    else h2_reduce_kernel<false><<<rgrid, 256, 0, stream>>>(g, p.G, q, B, s.inverse, nullptr, C);
+    BSQ_HIP(hipGetLastError());
+}
+
+}  // namespace bsq

@@ -9,7 +9,8 @@
 //     B = Q^T A_w = U_hat S V_hat^T;  U_w = Q U_hat
 //     outputs (row-major): U = U_w, V = V_hat, or swapped when m < n.
 // Design on MI355X: the big matrix is read in place (row-major, as op(A) or
-// op(A)^T inside the MFMA GEMM, no transposed copy); orth() is CholeskyQR
+// op(A)^T inside the MFMA GEMM, no transposed copy, its values as two f16
+// pieces each: gemm_h2.hip); orth() is CholeskyQR
 // with the Gram matrix formed in FP64 (twice for the final basis); the SVD of
 // B is taken from the FP64 eigen-decomposition of B B^T = Y^T Y with
 // Y = A_w^T Q, so that U_hat comes from a k x k problem and
@@ -213,6 +214,9 @@ struct SvdPlan {
     double *gram_ws = nullptr;
     float *gemm_ws = nullptr;
     uint64_t gemm_ws_bytes = 0;
+    bool h2 = false;             // the products with A as two f16 pieces (gemm_h2.hip)
+    H2Scales h2s;                // of A's rows
+    uint16_t *planes = nullptr;  // the pieces of the other operand
     bool owns = true;  // buffers from hipMalloc (freed here), else carved from a caller's arena
 
     ~SvdPlan() {
@@ -240,6 +244,12 @@ struct SvdPlan {
         release(status);
         release(gram_ws);
         release(gemm_ws);
+        release(h2s.exponent);
+        release(h2s.scale);
+        release(h2s.inverse);
+        release(h2s.emax);
+        release(h2s.common);
+        release(planes);
     }
 };
 
@@ -291,11 +301,46 @@ void plan_buffers(SvdPlan &p, Get &&get) {
     uint64_t ws = 0;
     ws = std::max(ws, gemm_workspace_bytes(p.Mw, p.k, p.Nw));
     ws = std::max(ws, gemm_workspace_bytes(p.Nw, p.k, p.Mw));
+    if (p.h2) {
+        ws = std::max({ws, h2_workspace_bytes(p.Mw, p.k, p.Nw), h2_workspace_bytes(p.Nw, p.k, p.Mw)});
+        get(p.h2s.exponent, p.m);
+        get(p.h2s.scale, p.m);
+        get(p.h2s.inverse, p.m);
+        get(p.h2s.emax, 1);
+        get(p.h2s.common, 1);
+        get(p.planes, h2_plane_units(p.Mw, p.k));  // Mw >= Nw
+    }
     p.gemm_ws_bytes = ws;
     if (ws) get(p.gemm_ws, ws / sizeof(float));
 }
 
 constexpr uint64_t kArenaAlign = 256;
+constexpr uint64_t kNoAllocScratchBytes = 256ull << 20;  // see `scratch` below
+
+// Device bytes of a plan's buffers, each rounded up to kArenaAlign.
+uint64_t plan_bytes(int m, int n, int q, int niter, bool h2) {
+    SvdPlan p;
+    p.owns = false;
+    plan_shape(p, m, n, q, niter);
+    p.h2 = h2;
+    uint64_t total = 0;
+    plan_buffers(p, [&](auto *&ptr, uint64_t count) {
+        using T = std::remove_reference_t<decltype(*ptr)>;
+        total += ceil_div(count * sizeof(T), kArenaAlign) * kArenaAlign;
+        ptr = nullptr;
+    });
+    return total;
+}
+
+// Whether a plan's products with A run on the f16 matrix cores.  The fixed
+// scratch array of the no-allocation entry point holds every plan that it
+// held without the operand planes: one that would outgrow it only through
+// them keeps the FP32 products, in both entry points, so their results agree.
+bool plan_uses_h2(int m, int n, int q, int niter) {
+    if (!h2_supported(std::min(m, n))) return false;
+    return plan_bytes(m, n, q, niter, true) <= kNoAllocScratchBytes ||
+           plan_bytes(m, n, q, niter, false) > kNoAllocScratchBytes;
+}
 
 }  // namespace
 
@@ -303,6 +348,7 @@ SvdPlan *svd_plan_create(int m, int n, int q, int niter) {
     auto *p = new SvdPlan;
     try {
         plan_shape(*p, m, n, q, niter);
+        p->h2 = plan_uses_h2(m, n, q, niter);
         plan_buffers(*p, [](auto *&ptr, uint64_t count) {
             using T = std::remove_reference_t<decltype(*ptr)>;
             ptr = alloc<T>(count);
@@ -315,22 +361,14 @@ SvdPlan *svd_plan_create(int m, int n, int q, int niter) {
 }
 
 uint64_t svd_plan_arena_bytes(int m, int n, int q, int niter) {
-    SvdPlan p;
-    p.owns = false;
-    plan_shape(p, m, n, q, niter);
-    uint64_t total = 0;
-    plan_buffers(p, [&](auto *&ptr, uint64_t count) {
-        using T = std::remove_reference_t<decltype(*ptr)>;
-        total += ceil_div(count * sizeof(T), kArenaAlign) * kArenaAlign;
-        ptr = nullptr;
-    });
-    return total;
+    return plan_bytes(m, n, q, niter, plan_uses_h2(m, n, q, niter));
 }
 
 void svd_plan_init_arena(SvdPlan &p, int m, int n, int q, int niter, void *arena, uint64_t arena_bytes) {
     BSQ_REQUIRE(arena && (reinterpret_cast<uintptr_t>(arena) % kArenaAlign) == 0, "svd: arena not 256-byte aligned");
     p.owns = false;
     plan_shape(p, m, n, q, niter);
+    p.h2 = plan_uses_h2(m, n, q, niter);
     const uint64_t need = svd_plan_arena_bytes(m, n, q, niter);
     BSQ_REQUIRE(need <= arena_bytes, "svd: shape needs more scratch than the arena holds");
     auto *base = static_cast<uint8_t *>(arena);
@@ -355,24 +393,20 @@ void svd_run(SvdPlan *p, const float *A, const float *sketch, uint64_t seed, flo
         launch_gaussian_fill(p->R, static_cast<uint64_t>(Nw) * k, seed, st);
         R = p->R;
     }
-    // X (Mw x k) = A_w * B (B is Nw x k)
-    auto aw_times = [&](const float *Bm, float *out) {
+    if (p->h2) launch_h2_scales(A, m, n, p->h2s, st);
+    // out = A B (n x k, ta false) or A^T B (m x k)
+    auto times = [&](bool ta, const float *Bm, float *out) {
         timed_launch(kTimeRangeFinder, st, [&] {
-            if (!p->transposed) launch_gemm(false, false, m, k, n, A, n, Bm, k, out, k, nullptr, nullptr, p->gemm_ws,
-                                            p->gemm_ws_bytes, st);
-            else launch_gemm(true, false, n, k, m, A, n, Bm, k, out, k, nullptr, nullptr, p->gemm_ws,
-                             p->gemm_ws_bytes, st);
+            // a caller's sketch may hold anything: it takes the FP32 product
+            if (p->h2 && Bm != sketch)
+                launch_h2_gemm(ta, m, n, k, A, p->h2s, Bm, p->planes, out, p->gemm_ws, p->gemm_ws_bytes, st);
+            else
+                launch_gemm(ta, false, ta ? n : m, k, ta ? m : n, A, n, Bm, k, out, k, nullptr, nullptr, p->gemm_ws,
+                            p->gemm_ws_bytes, st);
         });
     };
-    // Y (Nw x k) = A_w^T * B (B is Mw x k)
-    auto awt_times = [&](const float *Bm, float *out) {
-        timed_launch(kTimeRangeFinder, st, [&] {
-            if (!p->transposed) launch_gemm(true, false, n, k, m, A, n, Bm, k, out, k, nullptr, nullptr, p->gemm_ws,
-                                            p->gemm_ws_bytes, st);
-            else launch_gemm(false, false, m, k, n, A, n, Bm, k, out, k, nullptr, nullptr, p->gemm_ws,
-                             p->gemm_ws_bytes, st);
-        });
-    };
+    auto aw_times = [&](const float *Bm, float *out) { times(p->transposed, Bm, out); };    // X (Mw x k) = A_w B
+    auto awt_times = [&](const float *Bm, float *out) { times(!p->transposed, Bm, out); };  // Y (Nw x k) = A_w^T B
     // one CholeskyQR pass: out = in * L^{-T}, G = in^T in = L L^T
     auto orth = [&](const float *in, float *out, int rows) {
         launch_gram(in, rows, k, k, p->G, p->gram_ws, st);
@@ -469,7 +503,6 @@ void launch_gaussian_fill(float *out, uint64_t n, uint64_t seed, hipStream_t str
 // SVD kernels write every scratch word before reading it (nothing needs to
 // start at zero), so the contents a previous call left behind do not matter.
 // ---------------------------------------------------------------------------
-constexpr uint64_t kNoAllocScratchBytes = 256ull << 20;
 static __device__ __align__(256) uint8_t scratch[kNoAllocScratchBytes];
 
 namespace {
