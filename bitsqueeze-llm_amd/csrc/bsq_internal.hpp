@@ -241,9 +241,11 @@ uint64_t svd_noalloc_scratch_bytes();
 void svd_run(SvdPlan *plan, const float *A, const float *sketch, uint64_t seed, float *U, float *S, float *V,
              hipStream_t stream);
 // out = U diag(S) V^T (m x n row-major), or minuend - U diag(S) V^T when
-// `minuend` is not null.
+// `minuend` is not null (recon.hip).  `exponents` (device, m + n ints of
+// scratch) saves every workgroup the search for its rows' largest magnitudes;
+// null gives the same bits.
 void launch_reconstruct(const float *U, const float *S, const float *V, int m, int n, int k,
-                        const float *minuend, float *out, hipStream_t stream);
+                        const float *minuend, float *out, int *exponents, hipStream_t stream);
 // Products of the range finder on the f16 matrix cores with every FP32 value
 // carried as two f16 pieces (gemm_h2.hip).  H2Scales: the exact power-of-two
 // scales of a matrix's rows, device memory (exponent, scale, inverse: one per
@@ -269,17 +271,6 @@ void launch_h2_gemm(bool ta, int m, int n, int q, const float *A, const H2Scales
 void launch_gaussian_fill(float *out, uint64_t n, uint64_t seed, hipStream_t stream);
 
 int cu_count();
-
-// Reconstruction from NF4 / NF4_DQ factors decoded inline (recon.hip): U
-// (m x k) and V (n x k) are packed nibbles with their block scales (and the
-// device dq of NF4_DQ), S is FP32; out = U diag(S) V^T, bit for bit what
-// decoding the factors and launch_reconstruct give.  Supported for
-// k % 64 == 0, 64 <= k <= kReconQMaxK and 16-byte aligned code arrays.
-constexpr int kReconQMaxK = 512;
-bool recon_q_supported(int m, int n, int k, const uint8_t *u_codes, const uint8_t *v_codes);
-void launch_recon_q(int method, const uint8_t *u_codes, const float *u_scales_f32, const uint8_t *u_scales_u8,
-                    const float *u_dq, const uint8_t *v_codes, const float *v_scales_f32, const uint8_t *v_scales_u8,
-                    const float *v_dq, const float *S, int m, int n, int k, float *out, hipStream_t stream);
 
 // Instrumentation (off unless started through the ABI): HIP events bracket
 // the launches of each class below inside the pipelines, on the stream they

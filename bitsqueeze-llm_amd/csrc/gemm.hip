@@ -6,13 +6,10 @@
 //     op(B) = B          (TB = false, B is K x N, ldb >= N)
 //           = B^T        (TB = true,  B is N x K, ldb >= K)
 //
-// Used for the small basis rotations (X * W), for the range finder's product
-// with a caller's sketch and its products with matrices narrower than 64
-// (the others run in gemm_h2.hip; the big activation matrix is read row-major
-// in place, so no transposed copy is ever made), and for the low-rank
-// reconstruction U diag(S) V^T, which scales the A fragments by S (fetched a
-// slice ahead with the operand tiles) and can subtract from a minuend in the
-// epilogue (error = residual - U S V^T).
+// Used for the small basis rotations (X * W), and for the range finder's
+// product with a caller's sketch and its products with matrices narrower than
+// 64 (the others run in gemm_h2.hip; the big activation matrix is read
+// row-major in place, so no transposed copy is ever made).
 //
 // Tiling: 256 threads = 4 waves in a 2 x 2 grid; workgroup tile 128 x 128,
 // BK = 16; each wave owns 64 x 64 as 4 x 4 MFMA 16x16 blocks (64 AGPRs).
@@ -45,9 +42,7 @@ constexpr int KS = BK / 4;  // k-values per lane per slice
 struct GemmArgs {
     const float *A;
     const float *B;
-    float *C;                 // output (or split-K workspace base)
-    const float *a_colscale;  // optional: op(A)[:, kk] *= a_colscale[kk]
-    const float *minuend;     // optional: C = minuend - acc (ldc layout)
+    float *C;             // output (or split-K workspace base)
     int M, N, K;
     int lda, ldb, ldc;
     int k_per_split;          // K range of one split (multiple of BK)
@@ -76,7 +71,7 @@ struct KContig {
     using Tile = float[R][PK];
     float4 v[N4];
     __device__ __forceinline__ void load(const float *__restrict__ P, int ld, int r0, int rows, int k0, int kend,
-                                         bool vec, const float *__restrict__ colscale) {
+                                         bool vec) {
         const int t = threadIdx.x;
 #pragma unroll
         for (int q = 0; q < N4; ++q) {
@@ -92,12 +87,6 @@ struct KContig {
                 x.y = (gr < rows && gk + 1 < kend) ? row[gk + 1] : 0.0f;
                 x.z = (gr < rows && gk + 2 < kend) ? row[gk + 2] : 0.0f;
                 x.w = (gr < rows && gk + 3 < kend) ? row[gk + 3] : 0.0f;
-            }
-            if (colscale) {
-                x.x *= (gk + 0 < kend) ? colscale[gk + 0] : 0.0f;
-                x.y *= (gk + 1 < kend) ? colscale[gk + 1] : 0.0f;
-                x.z *= (gk + 2 < kend) ? colscale[gk + 2] : 0.0f;
-                x.w *= (gk + 3 < kend) ? colscale[gk + 3] : 0.0f;
             }
             v[q] = x;
         }
@@ -127,7 +116,7 @@ struct KMajor {
     using Tile = float[BK][Cn + 4];
     float4 v[N4];
     __device__ __forceinline__ void load(const float *__restrict__ P, int ld, int c0, int cols, int k0, int kend,
-                                         bool vec, const float *__restrict__ rowscale) {
+                                         bool vec) {
         const int t = threadIdx.x;
         constexpr int C4 = Cn / 4;
 #pragma unroll
@@ -144,13 +133,6 @@ struct KMajor {
                 x.y = (gk < kend && gc + 1 < cols) ? row[gc + 1] : 0.0f;
                 x.z = (gk < kend && gc + 2 < cols) ? row[gc + 2] : 0.0f;
                 x.w = (gk < kend && gc + 3 < cols) ? row[gc + 3] : 0.0f;
-            }
-            if (rowscale) {
-                const float sc = (gk < kend) ? rowscale[gk] : 0.0f;
-                x.x *= sc;
-                x.y *= sc;
-                x.z *= sc;
-                x.w *= sc;
             }
             v[q] = x;
         }
@@ -170,22 +152,14 @@ struct KMajor {
     }
 };
 
-
-// RECON: the low-rank reconstruction form (column scale on op(A), optional
-// minuend), instantiated separately so the power-iteration GEMMs carry no
-// epilogue branches and profiles tell the two apart.
-template <bool TA, bool TB, bool RECON>
+template <bool TA, bool TB>
 __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(GemmArgs g) {
     constexpr int WM = BM / 2, WN = BN / 2;  // wave tile
     constexpr int FM = WM / 16, FN = WN / 16;
     using TileA = typename std::conditional<TA, KMajor<BM>, KContig<BM>>::type;
     using TileB = typename std::conditional<TB, KContig<BN>, KMajor<BN>>::type;
-    // one LDS block: the double-buffered operand tiles, reused by the
-    // reconstruction epilogue to stage the output tile
     constexpr size_t kABytes = 2 * sizeof(typename TileA::Tile), kBBytes = 2 * sizeof(typename TileB::Tile);
-    constexpr size_t kCBytes = RECON ? sizeof(float) * (BM / 2) * (BN + 4) : 0;
-    constexpr size_t kSmem = (kABytes + kBBytes > kCBytes) ? kABytes + kBBytes : kCBytes;
-    __shared__ __attribute__((aligned(16))) unsigned char smem[kSmem];
+    __shared__ __attribute__((aligned(16))) unsigned char smem[kABytes + kBBytes];
     typename TileA::Tile *As = reinterpret_cast<typename TileA::Tile *>(smem);
     typename TileB::Tile *Bs = reinterpret_cast<typename TileB::Tile *>(smem + kABytes);
 
@@ -206,27 +180,14 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(GemmArgs g) {
     TileA ta;
     TileB tb;
     auto load = [&](int k0) {
-        ta.load(g.A, g.lda, m0, g.M, k0, kend, g.vec_a, nullptr);
-        tb.load(g.B, g.ldb, n0, g.N, k0, kend, g.vec_b, nullptr);
+        ta.load(g.A, g.lda, m0, g.M, k0, kend, g.vec_a);
+        tb.load(g.B, g.ldb, n0, g.N, k0, kend, g.vec_b);
     };
 
     int buf = 0;
     const int kk = lane >> 4, cc = lane & 15;
-    // RECON: op(A)[:, k] *= colscale[k] on this lane's KS k-values
-    // (k = k0 + KS kk + s), fetched one slice ahead with the operand tiles
-    float sc[KS];
-    auto load_scale = [&](int k0) {
-        if constexpr (RECON) {
-#pragma unroll
-            for (int st = 0; st < KS; ++st) {
-                const int kx = k0 + KS * kk + st;
-                sc[st] = (g.a_colscale && kx < kend) ? g.a_colscale[kx] : 1.0f;
-            }
-        }
-    };
     if (kbeg < kend) {
         load(kbeg);
-        load_scale(kbeg);
         ta.store(As[0]);
         tb.store(Bs[0]);
     }
@@ -236,15 +197,8 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(GemmArgs g) {
         float a[FM][KS], b[FN][KS];
 #pragma unroll
         for (int i = 0; i < FM; ++i) TileA::frag(As[buf], wm0 + i * 16 + cc, kk, a[i]);
-        if constexpr (RECON) {
-#pragma unroll
-            for (int i = 0; i < FM; ++i)
-#pragma unroll
-                for (int st = 0; st < KS; ++st) a[i][st] *= sc[st];
-        }
         if (more) {
             load(k0 + BK);
-            load_scale(k0 + BK);
         }
 #pragma unroll
         for (int j = 0; j < FN; ++j) TileB::frag(Bs[buf], wn0 + j * 16 + cc, kk, b[j]);
@@ -265,60 +219,6 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(GemmArgs g) {
 
     // epilogue: fragment (i, j) register r holds row 4*(lane/16) + r, column lane % 16
     float *C = g.C + static_cast<uint64_t>(zs) * g.split_stride;
-    if constexpr (RECON) {
-        // the reconstruction writes (and may subtract from) a full m x n matrix:
-        // stage the tile through LDS (the operand buffers are free now) in two
-        // 64-row halves so that rows leave as 16-byte stores and the minuend
-        // arrives as 16-byte loads, issued before the staging
-        constexpr int CP = BN + 4, HM = BM / 2;
-        float(*Cs)[CP] = reinterpret_cast<float(*)[CP]>(smem);
-        constexpr int Q = HM * BN / 4 / kThreads;  // float4 per thread per half
-        const bool vec_c = ((g.ldc & 3) == 0) && ((reinterpret_cast<uintptr_t>(C) & 15u) == 0) &&
-                           (!g.minuend || (reinterpret_cast<uintptr_t>(g.minuend) & 15u) == 0);
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            float4 mv[Q];
-            if (g.minuend && vec_c) {
-#pragma unroll
-                for (int q = 0; q < Q; ++q) {
-                    const int lin = tid + q * kThreads, rr = h * HM + lin / (BN / 4), c4 = lin % (BN / 4);
-                    const int gi = m0 + rr, gj = n0 + 4 * c4;
-                    mv[q] = (gi < g.M && gj + 4 <= g.N)
-                                ? *reinterpret_cast<const float4 *>(g.minuend + static_cast<uint64_t>(gi) * g.ldc + gj)
-                                : float4{0.f, 0.f, 0.f, 0.f};
-                }
-            }
-            __syncthreads();  // the operand tiles (h = 0) or the previous half (h = 1) are consumed
-            if (wm0 == h * HM) {
-#pragma unroll
-                for (int i = 0; i < FM; ++i)
-#pragma unroll
-                    for (int j = 0; j < FN; ++j)
-#pragma unroll
-                        for (int r = 0; r < 4; ++r)
-                            Cs[i * 16 + 4 * (lane >> 4) + r][wn0 + j * 16 + (lane & 15)] = acc[i][j][r];
-            }
-            __syncthreads();
-#pragma unroll
-            for (int q = 0; q < Q; ++q) {
-                const int lin = tid + q * kThreads, rl = lin / (BN / 4), c4 = lin % (BN / 4);
-                const int gi = m0 + h * HM + rl, gj = n0 + 4 * c4;
-                if (gi >= g.M) continue;
-                float4 v = *reinterpret_cast<const float4 *>(&Cs[rl][4 * c4]);
-                const uint64_t e = static_cast<uint64_t>(gi) * g.ldc + gj;
-                if (vec_c && gj + 4 <= g.N) {
-                    if (g.minuend) v = float4{mv[q].x - v.x, mv[q].y - v.y, mv[q].z - v.z, mv[q].w - v.w};
-                    *reinterpret_cast<float4 *>(C + e) = v;
-                } else {
-                    const float vv[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-                    for (int u = 0; u < 4; ++u)
-                        if (gj + u < g.N) C[e + u] = g.minuend ? g.minuend[e + u] - vv[u] : vv[u];
-                }
-            }
-        }
-        return;
-    }
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
@@ -347,7 +247,6 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma_kernel(GemmArgs g) {
 typedef __attribute__((address_space(3))) void lds_void_t;
 typedef __attribute__((address_space(1))) void glb_void_t;
 constexpr int kStages = 4;
-constexpr int kDmaReconMaxK = 1024;  // RECON column scales staged in LDS
 
 __device__ __forceinline__ void dma16(const float *g, const float *l) {
     __builtin_amdgcn_global_load_lds((glb_void_t *)(g), (lds_void_t *)(reinterpret_cast<size_t>(l)), 16, 0, 0);
@@ -413,9 +312,9 @@ __device__ __forceinline__ void dma_frag(const float *S, int row, int kk, float 
 
 // T x T output tile (T = 128, or 64 for grids that 128-wide tiles would
 // leave short of the CU count); four waves of T/2 x T/2.
-template <bool TA, bool TB, bool RECON, int T>
+template <bool TA, bool TB, int T>
 __global__ __launch_bounds__(kThreads) void gemm_dma_kernel(GemmArgs g) {
-    static_assert(T == 128 || (T == 64 && !RECON), "gemm: tile size");
+    static_assert(T == 128 || T == 64, "gemm: tile size");
     constexpr int BM = T, BN = T;
     constexpr int kTileF = T * BK;     // floats per operand tile
     constexpr int kStageF = 2 * kTileF;  // A + B
@@ -430,7 +329,6 @@ __global__ __launch_bounds__(kThreads) void gemm_dma_kernel(GemmArgs g) {
     __shared__ __attribute__((aligned(1024))) float st1[kStageF];
     __shared__ __attribute__((aligned(1024))) float st2[kStageF];
     __shared__ __attribute__((aligned(1024))) float st3[kStageF];
-    __shared__ float scs[RECON ? kDmaReconMaxK : 1];  // RECON: the column scales of op(A)
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm0 = (wave >> 1) * WM, wn0 = (wave & 1) * WN;
@@ -447,10 +345,6 @@ __global__ __launch_bounds__(kThreads) void gemm_dma_kernel(GemmArgs g) {
 #pragma unroll
         for (int j = 0; j < FN; ++j) acc[i][j] = f32x4v{0.f, 0.f, 0.f, 0.f};
 
-    if constexpr (RECON) {
-        for (int t = tid; t < kend - kbeg; t += kThreads) scs[t] = g.a_colscale ? g.a_colscale[kbeg + t] : 1.0f;
-        // visible after the first barrier of the loop
-    }
     // each wave issues chunks kCpw w .. kCpw w + kCpw - 1 of A and of B
     auto issue = [&](const float *st, int j) {
         const int k0 = kbeg + j * BK;
@@ -462,54 +356,17 @@ __global__ __launch_bounds__(kThreads) void gemm_dma_kernel(GemmArgs g) {
         }
     };
     const int kk = lane >> 4, cc = lane & 15;
-    // RECON: the minuend of this wave's 64 x 64 output block (16 float4 per
-    // lane, in the layout the epilogue stores) is requested right after the
-    // last operand slice, so it arrives while the last slices are multiplied.
-    // Every lane issues all kMv loads (addresses clamped into the matrix), so
-    // the waits below can count them.
-    constexpr int kMv = RECON ? WM * WN / 4 / 64 : 0;
-    float4 mvall[RECON ? kMv : 1];
-    const bool vec_c = RECON && ((g.ldc & 3) == 0) &&
-                       ((reinterpret_cast<uintptr_t>(g.C + static_cast<uint64_t>(zs) * g.split_stride) & 15u) == 0) &&
-                       (!g.minuend || (reinterpret_cast<uintptr_t>(g.minuend) & 15u) == 0);
-    const bool mv_on = RECON && g.minuend && vec_c && g.N >= 4;
-    auto issue_minuend = [&]() {
-        asm volatile("" ::: "memory");  // stays behind the last slice's DMA
-#pragma unroll
-        for (int q = 0; q < kMv; ++q) {
-            const int gi = min(m0 + wm0 + 4 * q + (lane >> 4), g.M - 1), gj = min(n0 + wn0 + 4 * (lane & 15), g.N - 4);
-            mvall[q] = *reinterpret_cast<const float4 *>(g.minuend + static_cast<uint64_t>(gi) * g.ldc + gj);
-        }
-        asm volatile("" ::: "memory");
-    };
     // slice j sits in stage j % 4: cur holds it, nxt (= stage (j + 3) % 4, read
     // in iteration j - 1) receives slice j + 3
     auto body = [&](const float *cur, const float *nxt, int j) {
         const int ahead = min(kStages - 2, nk - 1 - j);  // slices issued after j
-        if (mv_on && j + kStages - 1 >= nk) {  // the minuend loads follow the last slice
-            if (ahead >= 2) dma_barrier<2 * kDmaPerSlice + kMv>();
-            else if (ahead == 1) dma_barrier<kDmaPerSlice + kMv>();
-            else dma_barrier<kMv>();
-        } else {
-            if (ahead >= 2) dma_barrier<2 * kDmaPerSlice>();
-            else if (ahead == 1) dma_barrier<kDmaPerSlice>();
-            else dma_barrier<0>();
-        }
-        if (j + kStages - 1 < nk) {
-            issue(nxt, j + kStages - 1);
-            if (mv_on && j + kStages - 1 == nk - 1) issue_minuend();
-        }
+        if (ahead >= 2) dma_barrier<2 * kDmaPerSlice>();
+        else if (ahead == 1) dma_barrier<kDmaPerSlice>();
+        else dma_barrier<0>();
+        if (j + kStages - 1 < nk) issue(nxt, j + kStages - 1);
         float a[FM][KS], b[FN][KS];
 #pragma unroll
         for (int i = 0; i < FM; ++i) dma_frag<TA, T>(cur, wm0 + i * 16 + cc, kk, a[i]);
-        if constexpr (RECON) {
-#pragma unroll
-            for (int s2 = 0; s2 < KS; ++s2) {
-                const float sc = scs[j * BK + KS * kk + s2];
-#pragma unroll
-                for (int i = 0; i < FM; ++i) a[i][s2] *= sc;
-            }
-        }
 #pragma unroll
         for (int jj = 0; jj < FN; ++jj) dma_frag<!TB, T>(cur + kTileF, wn0 + jj * 16 + cc, kk, b[jj]);
 #pragma unroll
@@ -523,7 +380,6 @@ __global__ __launch_bounds__(kThreads) void gemm_dma_kernel(GemmArgs g) {
     if (0 < nk) issue(st0, 0);
     if (1 < nk) issue(st1, 1);
     if (2 < nk) issue(st2, 2);
-    if (mv_on && nk <= kStages - 1) issue_minuend();
     for (int j = 0; j < nk; j += kStages) {
         body(st0, st3, j);
         if (j + 1 < nk) body(st1, st0, j + 1);
@@ -533,42 +389,6 @@ __global__ __launch_bounds__(kThreads) void gemm_dma_kernel(GemmArgs g) {
 
     float *C = g.C + static_cast<uint64_t>(zs) * g.split_stride;
     // fragment (i, j) register r holds row 4*(lane/16) + r, column lane % 16
-    if constexpr (RECON) {
-        // every wave leaves with its own 64 x 64 block through its own 16 KB
-        // of the ring, after one barrier (the ring is consumed): rows go out
-        // as 16-byte stores, the minuend comes in as 16-byte loads; columns
-        // are XOR-swizzled by 16 on alternate groups of four rows (the
-        // fragment writes of rows r and r + 4 then hit disjoint banks)
-        __syncthreads();
-        float *Cw = wave == 0 ? st0 : (wave == 1 ? st1 : (wave == 2 ? st2 : st3));
-#pragma unroll
-        for (int i = 0; i < FM; ++i)
-#pragma unroll
-            for (int j = 0; j < FN; ++j)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int rl = 16 * i + 4 * (lane >> 4) + r, col = 16 * j + (lane & 15);
-                    Cw[rl * WN + (col ^ (16 * ((rl >> 2) & 1)))] = acc[i][j][r];
-                }
-#pragma unroll
-        for (int q = 0; q < kMv; ++q) {
-            const int rl = 4 * q + (lane >> 4), c4 = 4 * (lane & 15);
-            const int gi = m0 + wm0 + rl, gj = n0 + wn0 + c4;
-            if (gi >= g.M) continue;
-            float4 v = *reinterpret_cast<const float4 *>(&Cw[rl * WN + (c4 ^ (16 * ((rl >> 2) & 1)))]);
-            const uint64_t e = static_cast<uint64_t>(gi) * g.ldc + gj;
-            if (vec_c && gj + 4 <= g.N) {
-                if (mv_on) v = float4{mvall[q].x - v.x, mvall[q].y - v.y, mvall[q].z - v.z, mvall[q].w - v.w};
-                *reinterpret_cast<float4 *>(C + e) = v;
-            } else {
-                const float vv[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-                for (int u = 0; u < 4; ++u)
-                    if (gj + u < g.N) C[e + u] = g.minuend ? g.minuend[e + u] - vv[u] : vv[u];
-            }
-        }
-        return;
-    }
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
@@ -884,17 +704,14 @@ uint64_t gemm_workspace_bytes(int M, int N, int K) {
 }
 
 void launch_gemm(bool ta, bool tb, int M, int N, int K, const float *A, int lda, const float *B, int ldb, float *C,
-                 int ldc, const float *a_colscale, const float *minuend, float *workspace, uint64_t workspace_bytes,
-                 hipStream_t stream) {
+                 int ldc, float *workspace, uint64_t workspace_bytes, hipStream_t stream) {
     BSQ_REQUIRE(M > 0 && N > 0 && K > 0 && A && B && C, "gemm: bad arguments");
-    int splits = (minuend || a_colscale) ? 1 : choose_splits(M, N, K);
+    int splits = choose_splits(M, N, K);
     if (splits > 1 && (!workspace || static_cast<uint64_t>(splits) * M * N * sizeof(float) > workspace_bytes))
         splits = 1;
     GemmArgs g{};
     g.A = A;
     g.B = B;
-    g.a_colscale = a_colscale;
-    g.minuend = minuend;
     g.M = M;
     g.N = N;
     g.K = K;
@@ -914,13 +731,12 @@ void launch_gemm(bool ta, bool tb, int M, int N, int K, const float *A, int lda,
     }
     g.splits = splits;
     dim3 grid(static_cast<unsigned>(ceil_div(N, BN) * ceil_div(M, BM) * splits));
-    const bool recon = a_colscale || minuend;
     // the DMA-pipelined kernel wherever its layout constraints hold, else the
     // register-staged one
     const bool dma = g.vec_a && g.vec_b && (K % BK == 0) && (!ta || M % 4 == 0) &&
-                     (tb || N % 4 == 0) && (!recon || K <= kDmaReconMaxK);
+                     (tb || N % 4 == 0);
     // the long-K products in stream-K form
-    if (dma && !recon && splits > 1) {
+    if (dma && splits > 1) {
         SkPlan pl = streamk_plan(M, N, K);
         if (pl.on && pl.bytes <= workspace_bytes) {
             pl.sk.ws = workspace;
@@ -943,29 +759,23 @@ void launch_gemm(bool ta, bool tb, int M, int N, int K, const float *A, int lda,
     }
     // 64 x 64 tiles when 128 x 128 ones (unsplit) would not give every CU two
     // workgroups: the short-K products of the orthonormalisation
-    const bool t64 = dma && !recon && splits == 1 &&
+    const bool t64 = dma && splits == 1 &&
                      ceil_div(M, BM) * ceil_div(N, BN) < 2 * static_cast<uint64_t>(cu_count());
     if (t64) {
         grid.x = static_cast<unsigned>(ceil_div(N, 64) * ceil_div(M, 64));  // unsplit
-        if (!ta && !tb) gemm_dma_kernel<false, false, false, 64><<<grid, kThreads, 0, stream>>>(g);
-        else if (ta && !tb) gemm_dma_kernel<true, false, false, 64><<<grid, kThreads, 0, stream>>>(g);
-        else if (!ta && tb) gemm_dma_kernel<false, true, false, 64><<<grid, kThreads, 0, stream>>>(g);
-        else gemm_dma_kernel<true, true, false, 64><<<grid, kThreads, 0, stream>>>(g);
+        if (!ta && !tb) gemm_dma_kernel<false, false, 64><<<grid, kThreads, 0, stream>>>(g);
+        else if (ta && !tb) gemm_dma_kernel<true, false, 64><<<grid, kThreads, 0, stream>>>(g);
+        else if (!ta && tb) gemm_dma_kernel<false, true, 64><<<grid, kThreads, 0, stream>>>(g);
+        else gemm_dma_kernel<true, true, 64><<<grid, kThreads, 0, stream>>>(g);
     } else if (dma) {
-        if (recon) {
-            BSQ_REQUIRE(!ta && tb, "gemm: column scale / minuend only in the A * B^T form");
-            gemm_dma_kernel<false, true, true, 128><<<grid, kThreads, 0, stream>>>(g);
-        } else if (!ta && !tb) gemm_dma_kernel<false, false, false, 128><<<grid, kThreads, 0, stream>>>(g);
-        else if (ta && !tb) gemm_dma_kernel<true, false, false, 128><<<grid, kThreads, 0, stream>>>(g);
-        else if (!ta && tb) gemm_dma_kernel<false, true, false, 128><<<grid, kThreads, 0, stream>>>(g);
-        else gemm_dma_kernel<true, true, false, 128><<<grid, kThreads, 0, stream>>>(g);
-    } else if (recon) {
-        BSQ_REQUIRE(!ta && tb, "gemm: column scale / minuend only in the A * B^T form");
-        gemm_mfma_kernel<false, true, true><<<grid, kThreads, 0, stream>>>(g);
-    } else if (!ta && !tb) gemm_mfma_kernel<false, false, false><<<grid, kThreads, 0, stream>>>(g);
-    else if (ta && !tb) gemm_mfma_kernel<true, false, false><<<grid, kThreads, 0, stream>>>(g);
-    else if (!ta && tb) gemm_mfma_kernel<false, true, false><<<grid, kThreads, 0, stream>>>(g);
-    else gemm_mfma_kernel<true, true, false><<<grid, kThreads, 0, stream>>>(g);
+        if (!ta && !tb) gemm_dma_kernel<false, false, 128><<<grid, kThreads, 0, stream>>>(g);
+        else if (ta && !tb) gemm_dma_kernel<true, false, 128><<<grid, kThreads, 0, stream>>>(g);
+        else if (!ta && tb) gemm_dma_kernel<false, true, 128><<<grid, kThreads, 0, stream>>>(g);
+        else gemm_dma_kernel<true, true, 128><<<grid, kThreads, 0, stream>>>(g);
+    } else if (!ta && !tb) gemm_mfma_kernel<false, false><<<grid, kThreads, 0, stream>>>(g);
+    else if (ta && !tb) gemm_mfma_kernel<true, false><<<grid, kThreads, 0, stream>>>(g);
+    else if (!ta && tb) gemm_mfma_kernel<false, true><<<grid, kThreads, 0, stream>>>(g);
+    else gemm_mfma_kernel<true, true><<<grid, kThreads, 0, stream>>>(g);
     BSQ_HIP(hipGetLastError());
     if (splits > 1) {
         const dim3 rgrid(static_cast<unsigned>(ceil_div(N, 256)),

@@ -5,18 +5,7 @@
 //     op(A) = A    (TA = false, A is M x K)      the range finder's A_w B and
 //     op(A) = A^T  (TA = true,  A is K x M)      A_w^T B, A read in place
 //
-// Split.  A value x, scaled by an exact power of two s, is h + l 2^-11 with
-// h = f16(s x) and l = f16(2^11 (s x - h)): 22 bits and a sign, the rest at
-// most half a unit in the last place of FP32.  The product sums
-//     hi += h_a h_b          lo += h_a l_b + l_a h_b
-// in FP32 accumulators of their own and is hi + 2^-11 lo; the dropped
-// l_a l_b is 2^-24 of the product or less, with either sign.  Keeping the two
-// sums apart keeps l a normal f16 down to 2^-29 of the scaled maximum and
-// adds the small terms without rounding them into the large sum.  Against
-// 64-bit sums the error is 0.35 to 0.9 times that of a
-// v_mfma_f32_16x16x4f32 chain of the same length (K = 32 .. 11008; normal,
-// lognormal, one-signed and decaying operands, and a column 10^6 times the
-// others that B does not touch).
+// The split and its error: h2_split.hpp.
 // Three f16 products run at up to 5 times the FP32 matrix rate (2.5 / 3
 // against 0.157 PFLOP/s).  Measured, against the FP32 kernels with their
 // reductions: 4096 x 11008 with q = 128 101 -> 49 us (A^T B) and 98 -> 49 us
@@ -36,6 +25,7 @@
 // it is staged.  All scalings are exact.  Rows holding infinities or NaN give
 // NaN results, as sums over them do.
 #include "bsq_internal.hpp"
+#include "h2_split.hpp"
 #include "tile_map.hpp"
 
 #include <algorithm>
@@ -43,10 +33,6 @@
 namespace bsq {
 namespace {
 
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) void lds_void_t;
 typedef __attribute__((address_space(1))) void glb_void_t;
 
@@ -56,29 +42,6 @@ constexpr int BK = 32;        // K slice
 constexpr int KG = BK / 8;    // groups of eight k per slice
 constexpr int kPitchA = 132;  // 16-byte units per k group of a staged A plane (128 rows, padded)
 constexpr int kScaleB = 11;   // B's scale, a power of two
-constexpr float kLo = 2048.0f, kLoInv = 1.0f / 2048.0f;
-
-// exponent of the largest magnitude of a row: in [-112, 127] (a zero row, or
-// one below 2^-112, takes -112; a row with infinities or NaN 127)
-__device__ __forceinline__ int row_exponent(float absmax) {
-    const int e = static_cast<int>(__float_as_uint(absmax) >> 23) - 127;
-    return min(max(e, -112), 127);
-}
-
-// 2^e, e in [-149, 127]
-__device__ __forceinline__ float pow2(int e) { return __builtin_ldexpf(1.0f, e); }
-
-// eight values to their f16 pieces: h the leading ones, l the scaled rests
-__device__ __forceinline__ void split8(const float (&y)[8], u32x4 &h, u32x4 &l) {
-#pragma unroll
-    for (int p = 0; p < 4; ++p) {
-        const f16x2 hp{static_cast<_Float16>(y[2 * p]), static_cast<_Float16>(y[2 * p + 1])};
-        const f16x2 lp{static_cast<_Float16>((y[2 * p] - static_cast<float>(hp.x)) * kLo),
-                       static_cast<_Float16>((y[2 * p + 1] - static_cast<float>(hp.y)) * kLo)};
-        h[p] = __builtin_bit_cast(uint32_t, hp);
-        l[p] = __builtin_bit_cast(uint32_t, lp);
-    }
-}
 
 __device__ __forceinline__ void dma16(const u32x4 *g, const u32x4 *l) {
     __builtin_amdgcn_global_load_lds((glb_void_t *)(g), (lds_void_t *)(reinterpret_cast<size_t>(l)), 16, 0, 0);
@@ -122,7 +85,7 @@ __global__ __launch_bounds__(kThreads) void row_scale_kernel(const float *__rest
     __syncthreads();
     if (tid == 0) {
         m = max(max(wmax[0], wmax[1]), max(wmax[2], wmax[3]));
-        const int e = row_exponent(__uint_as_float(m));
+        const int e = row_exponent(m);
         E[r] = e;
         rs[r] = pow2(14 - e);
         ri[r] = pow2(e - 14 - kScaleB);
@@ -295,15 +258,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         cb.next(nk, g.tiles_n);
     };
 
-    f32x16 hi[2][2], lo[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) hi[i][j] = lo[i][j] = f32x16{};
-
-    struct Frags {
-        f16x8 ah[2], al[2], bh[2], bl[2];
-    };
+    Sums acc;
+    acc.clear();
     auto fetch = [&](Frags &f, const u32x4 *as, const u32x4 *bs, int s) __attribute__((always_inline)) {
         const int kg = 2 * s + (lane >> 5), r = lane & 31;
 #pragma unroll
@@ -317,21 +273,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
             f.bl[i] = __builtin_bit_cast(f16x8, bs[(KG + kg) * T + wn0 + 32 * i + r]);
         }
     };
-    auto multiply = [&](const Frags &f) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int j = 0; j < 2; ++j) hi[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.ah[i], f.bh[j], hi[i][j], 0, 0, 0);
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int j = 0; j < 2; ++j) lo[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.ah[i], f.bl[j], lo[i][j], 0, 0, 0);
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int j = 0; j < 2; ++j) lo[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.al[i], f.bh[j], lo[i][j], 0, 0, 0);
-    };
-
     int c_tile = tile0, c_pr = p0 - tile0 * g.pairs;
     // after a pair: at the tile's or the range's end the partial tile goes out
     auto pair_done = [&](int j) __attribute__((always_inline)) {
@@ -352,11 +293,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
                     for (int q = 0; q < 4; ++q) {
                         f32x4 v;
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) v[e] = hi[i][jj][4 * q + e] + lo[i][jj][4 * q + e] * kLoInv;
+                        for (int e = 0; e < 4; ++e) v[e] = acc.hi[i][jj][4 * q + e] + acc.lo[i][jj][4 * q + e] * kLoInv;
                         W[((2 * i + jj) * 4 + q) * 64] = v;
                     }
-                    hi[i][jj] = lo[i][jj] = f32x16{};
                 }
+            acc.clear();
         }
         c_pr = tile_end ? 0 : c_pr;
         c_tile += tile_end ? 1 : 0;
@@ -376,8 +317,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         dma_b(bn);
         load_a();
         fetch(f1, ac, bc, 1);
-        multiply(f0);
-        multiply(f1);
+        acc.multiply(f0);
+        acc.multiply(f1);
     };
     if (n <= 0) return;  // uniform (G <= units: does not occur)
     load_a();

@@ -1,252 +1,284 @@
-// Reconstruction from NF4 / NF4_DQ factors on the gfx950 matrix cores
+// Low-rank reconstruction out = U diag(S) V^T, or minuend - U diag(S) V^T, on
+// the f16 matrix cores with every FP32 value as two f16 pieces (h2_split.hpp)
 // (reference modules/reconstruct_lowrank_cuda/src/reconstruct_lowrank_cuda.cu:
-// 21-62 with the decode of modules/quantization_cuda/src/
-// quantization_cuda.cu:287-341 inline): out = U diag(S) V^T from the packed
-// U (m x q) and V (n x q), the decompress side's reconstruction.
+// 21-62, 120-171; the subtraction of src/bitsqz_llm.cu:1141-1163).
 //
-// U and V stay in their packed form: one workgroup per 128 x 128 output tile
-// copies the nibbles of its 128 rows of U and of V (and their block scales)
-// into LDS once, and every slice of the K loop decodes its MFMA operand
-// fragments from there (two codes per 256-entry level-pair lookup), so the
-// main loop reads no global memory and needs no barrier.  Each value is
-// decoded exactly as the standalone decoder writes it (scale * L[code], the
-// scale guarded as there), then scaled by S[k], and the lane / k order of the
-// MFMA products is that of the FP32 reconstruction GEMM, so the output is
-// bit-identical to decoding U and V and reconstructing.  The top-k sets are
-// scatter-added afterwards by topk_scatter_kernel, error set first.
+// Each 128 x 128 tile of the output is one workgroup.  The rows of U diag(S)
+// and of V are scaled by powers of two that bring their largest magnitude into
+// [2^14, 2^15); their values are fetched a slice of 32 k ahead, split and
+// staged into LDS planes, and the tile leaves scaled back, straight from the
+// accumulators: 32 lanes write 128 contiguous bytes of a row.  The exponents
+// of the rows come from factor_exponent_kernel where the caller has room for
+// them, else each workgroup finds those of its own 256 rows first; the values
+// are the same, so the results are too.
+//
+// Measured against the FP32 matrix cores' kernels (which also decoded packed
+// factors inline on the decompress side): 4096 x 11008, rank 128 126 -> 96 us;
+// 8192 x 4096, rank 256 167 and 171 -> 110 us; 16384 x 14336, rank 512 2237
+// and 2553 -> 1234 us.
 #include "bsq_internal.hpp"
+#include "h2_split.hpp"
 #include "tile_map.hpp"
 
 namespace bsq {
 namespace {
 
-typedef float f32x4v __attribute__((ext_vector_type(4)));
-
 constexpr int kThreads = 256;
-constexpr int TT = 128, BK = 16, KS = 4;
+constexpr int T = 128, BK = 32, KG = BK / 8;
+constexpr int kPitch = 132;      // 16-byte units per k group of a plane (128 rows, padded)
+constexpr int kInfRow = 128;     // "exponent" of a row that holds infinities and no NaN
 
-struct QFactor {
-    const uint8_t *codes = nullptr;       // rows x K nibbles, two per byte, element 2j in the high nibble
-    const float *scales_f32 = nullptr;    // NF4: one per 64 elements
-    const uint8_t *scales_u8 = nullptr;   // NF4_DQ: E4M3 code per 64 elements
-    const float *dq = nullptr;            // NF4_DQ: the section's global scale
+struct ReconArgs {
+    const float *U, *S, *V;
+    const float *minuend;  // or null
+    float *out;
+    const int *eu, *ev;    // row exponents, or null
+    int m, n, k;
 };
 
-struct ReconQArgs {
-    QFactor u, v;
-    const float *s = nullptr;           // S (K), FP32
-    float *out = nullptr;               // M x N row-major
-    int M = 0, N = 0, K = 0;
-};
-
-__device__ __forceinline__ float e4m3_value(uint32_t v) {
-    // quantization_cuda.cu:111-128 (nf4_dq_impl.cpp:104-129)
-    const uint32_t ef = (v >> 3) & 15u, mf = v & 7u;
-    float r;
-    if (ef == 0) r = (static_cast<float>(mf) / 8.0f) * 0.015625f;
-    else r = (1.0f + static_cast<float>(mf) / 8.0f) * __builtin_ldexpf(1.0f, static_cast<int>(ef) - 7);
-    return (v & 0x80u) ? -r : r;
+__device__ __forceinline__ int factor_exponent(uint32_t bits) {
+    return bits == 0x7F800000u ? kInfRow : row_exponent(bits);
 }
+// scale of a row: its largest magnitude to [2^14, 2^15)
+__device__ __forceinline__ float factor_scale(int e) { return pow2(14 - min(e, 127)); }
 
-// Block scale b of a factor, as the decoder computes it (quantization_cuda.cu:
-// 300-305, 322-332): NF4 the stored scale, NF4_DQ dq * E4M3(code); 0 or a
-// non-finite value becomes 1.  `dq` is already guarded the same way.
-template <bool DQ>
-__device__ __forceinline__ float block_scale(const QFactor &f, uint64_t b, float dq) {
-    float s;
-    if constexpr (DQ) s = dq * e4m3_value(f.scales_u8[b]);
-    else s = f.scales_f32[b];
-    return (s == 0.0f || !__builtin_isfinite(s)) ? 1.0f : s;
-}
-
-__device__ __forceinline__ float guarded_dq(const float *p) {
-    const float dq = *p;
-    return (dq == 0.0f || !__builtin_isfinite(dq)) ? 1.0f : dq;
-}
-
-// LDS layout of one workgroup (bytes): codes of the tile's U rows and V rows
-// (row pitch K/2 + 16: 16-byte aligned rows that start four banks apart),
-// their block scales as floats, S, and the table of level pairs
-// L2[b] = (L[b >> 4], L[b & 15]).  The epilogue's staging of the output
-// (32 x 64 floats per wave) reuses the start of the block.
-struct Layout {
-    int pitch, cA, cB, sA, sB, sv, l2, bytes;
-    __host__ __device__ explicit Layout(int K) {
-        pitch = K / 2 + 16;
-        cA = 0;
-        cB = cA + TT * pitch;
-        sA = cB + TT * pitch;
-        sB = sA + TT * (K / 64) * 4;
-        sv = sB + TT * (K / 64) * 4;
-        l2 = sv + K * 4;
-        bytes = l2 + 256 * 8;
-        if (bytes < 4 * 32 * 64 * 4) bytes = 4 * 32 * 64 * 4;
+// eight values of a row from k on (rows may start at any multiple of four
+// bytes), zero past the row's end
+__device__ __forceinline__ void load_row8(const float *row, int k, int K, float (&v)[8]) {
+    if (k + 8 <= K) {
+        __builtin_memcpy(&v[0], __builtin_assume_aligned(row + k, 4), 32);
+    } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = k + i < K ? row[k + i] : 0.0f;
     }
-};
+}
 
-// Codes (uint4 chunks, row by row) and block scales of rows r0 .. r0 + rows - 1
-// of a factor into LDS; rows past the factor are left alone (their products
-// only reach output rows or columns that are never stored).
-template <bool DQ>
-__device__ __forceinline__ void stage_factor(const QFactor &f, int r0, int rows, int K, unsigned char *smem,
-                                             int c_off, int s_off, int pitch, float dq) {
-    const int chunks = K / 32;  // 16-byte chunks per row
-    const uint4 *src = reinterpret_cast<const uint4 *>(f.codes + static_cast<uint64_t>(r0) * (K / 2));
-    for (int i = threadIdx.x; i < rows * chunks; i += kThreads) {
-        const int r = i / chunks, c = i - r * chunks;
-        *reinterpret_cast<uint4 *>(smem + c_off + r * pitch + 16 * c) = src[static_cast<uint64_t>(r) * chunks + c];
+// exponents of the rows of U diag(S) (e[0 .. m)) and of V (e[m .. m + n)):
+// one wave per row
+__global__ __launch_bounds__(kThreads) void factor_exponent_kernel(const float *__restrict__ U,
+                                                                   const float *__restrict__ S,
+                                                                   const float *__restrict__ V, int m, int n, int k,
+                                                                   int *__restrict__ e) {
+    const int r = blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (r >= m + n) return;  // whole waves
+    const float *row = r < m ? U + static_cast<uint64_t>(r) * k : V + static_cast<uint64_t>(r - m) * k;
+    uint32_t bits = 0;
+#pragma unroll 4
+    for (int c = lane; c < k; c += 64) {
+        const float x = r < m ? row[c] * S[c] : row[c];
+        bits = max(bits, __float_as_uint(fabsf(x)));
     }
-    const int nb = K / 64;
-    float *sc = reinterpret_cast<float *>(smem + s_off);
-    const uint64_t b0 = static_cast<uint64_t>(r0) * nb;
-    for (int i = threadIdx.x; i < rows * nb; i += kThreads) sc[i] = block_scale<DQ>(f, b0 + i, dq);
+    for (int off = 32; off >= 1; off >>= 1)
+        bits = max(bits, static_cast<uint32_t>(__shfl_xor(static_cast<int>(bits), off)));
+    if (lane == 0) e[r] = factor_exponent(bits);
 }
 
-// Four consecutive elements k .. k + 3 (k % 4 == 0) of row `row`, decoded:
-// one 2-byte code read, two level-pair lookups, the block scale.
-__device__ __forceinline__ void decode4(const unsigned char *smem, int c_off, int s_off, int pitch, int K, int row,
-                                        int k, const float2 *L2, float (&o)[KS]) {
-    const uint32_t h = *reinterpret_cast<const uint16_t *>(smem + c_off + row * pitch + (k >> 1));
-    const float sc = reinterpret_cast<const float *>(smem + s_off)[row * (K / 64) + (k >> 6)];
-    const float2 l01 = L2[h & 0xFFu], l23 = L2[h >> 8];
-    o[0] = sc * l01.x;
-    o[1] = sc * l01.y;
-    o[2] = sc * l23.x;
-    o[3] = sc * l23.y;
-}
-
-template <bool DQ>
-__global__ __launch_bounds__(kThreads) void recon_q_kernel(ReconQArgs g) {
-    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    const int K = g.K;
-    const Layout lay(K);
+// (two waves per SIMD asked for: 128 accumulators and two slices' fragments)
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void recon_kernel(ReconArgs g) {
+    __shared__ u32x4 a0[2 * KG * kPitch], a1[2 * KG * kPitch];  // U diag(S): h plane, l plane
+    __shared__ u32x4 b0[2 * KG * kPitch], b1[2 * KG * kPitch];  // V
+    __shared__ int eu[T], ev[T];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm0 = (wave >> 1) * 64, wn0 = (wave & 1) * 64;
     int tile_m, tile_n, z;
-    const int ny = static_cast<int>(ceil_div(g.M, TT)), nx = static_cast<int>(ceil_div(g.N, TT));
-    xcd_tile(ny, nx, 1, tile_m, tile_n, z);
-    const int m0 = tile_m * TT, n0 = tile_n * TT;
+    xcd_tile(static_cast<int>(ceil_div(g.m, T)), static_cast<int>(ceil_div(g.n, T)), 1, tile_m, tile_n, z);
+    const int m0 = tile_m * T, n0 = tile_n * T, nk = static_cast<int>(ceil_div(g.k, BK));
 
-    float dqa = 1.0f, dqb = 1.0f;
-    if constexpr (DQ) {
-        dqa = guarded_dq(g.u.dq);
-        dqb = guarded_dq(g.v.dq);
-    }
-    stage_factor<DQ>(g.u, m0, min(TT, g.M - m0), K, smem, lay.cA, lay.sA, lay.pitch, dqa);
-    stage_factor<DQ>(g.v, n0, min(TT, g.N - n0), K, smem, lay.cB, lay.sB, lay.pitch, dqb);
-    float *Sv = reinterpret_cast<float *>(smem + lay.sv);
-    for (int k = tid; k < K; k += kThreads) Sv[k] = g.s[k];
-    float2 *L2 = reinterpret_cast<float2 *>(smem + lay.l2);
-    {
-        constexpr float Lc[16] = BSQ_NF4_LEVELS;
-        L2[tid] = float2{Lc[tid >> 4], Lc[tid & 15]};  // 256 threads, 256 pairs
-    }
-    __syncthreads();
-
-    f32x4v acc[4][4];
+    // a lane stages eight consecutive k (group kg of a slice) of rows r and
+    // r + 64 of each operand; rows past the factors repeat the last one
+    const int r = tid >> 2, kg = tid & 3;
+    const float *rows[4] = {g.U + static_cast<uint64_t>(min(m0 + r, g.m - 1)) * g.k,
+                            g.U + static_cast<uint64_t>(min(m0 + 64 + r, g.m - 1)) * g.k,
+                            g.V + static_cast<uint64_t>(min(n0 + r, g.n - 1)) * g.k,
+                            g.V + static_cast<uint64_t>(min(n0 + 64 + r, g.n - 1)) * g.k};
+    float v[4][8], s8[8];
+    auto load = [&](int j) __attribute__((always_inline)) {
+        const int k = j * BK + 8 * kg;
+        if ((j + 1) * BK <= g.k) {  // uniform: every slice but a ragged last one
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+            for (int h = 0; h < 4; ++h) __builtin_memcpy(&v[h][0], __builtin_assume_aligned(rows[h] + k, 4), 32);
+            __builtin_memcpy(&s8[0], __builtin_assume_aligned(g.S + k, 4), 32);
+        } else {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = f32x4v{0.f, 0.f, 0.f, 0.f};
-
-    const int kk = lane >> 4, cc = lane & 15;
-    for (int j = 0; j < K / BK; ++j) {
-        const int kb = j * BK + KS * kk;  // this lane's four k values
-        const float4 s4 = *reinterpret_cast<const float4 *>(Sv + kb);
-        float a[4][KS], b[4][KS];
+            for (int h = 0; h < 4; ++h) load_row8(rows[h], k, g.k, v[h]);
+            load_row8(g.S, k, g.k, s8);
+        }
+    };
+    if (g.eu) {  // uniform
+        if (tid < T) eu[tid] = g.eu[min(m0 + tid, g.m - 1)];
+        else ev[tid - T] = g.ev[min(n0 + tid - T, g.n - 1)];
+    } else {
+        uint32_t bits[4] = {0, 0, 0, 0};
+        for (int j = 0; j < nk; ++j) {
+            load(j);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            decode4(smem, lay.cA, lay.sA, lay.pitch, K, wm0 + i * 16 + cc, kb, L2, a[i]);
-            a[i][0] *= s4.x;
-            a[i][1] *= s4.y;
-            a[i][2] *= s4.z;
-            a[i][3] *= s4.w;
+            for (int h = 0; h < 4; ++h)
+#pragma unroll
+                for (int i = 0; i < 8; ++i)
+                    bits[h] = max(bits[h], __float_as_uint(fabsf(h < 2 ? v[h][i] * s8[i] : v[h][i])));
         }
 #pragma unroll
-        for (int jj = 0; jj < 4; ++jj) decode4(smem, lay.cB, lay.sB, lay.pitch, K, wn0 + jj * 16 + cc, kb, L2, b[jj]);
+        for (int h = 0; h < 4; ++h) {
+            for (int off = 1; off <= 2; off <<= 1)
+                bits[h] = max(bits[h], static_cast<uint32_t>(__shfl_xor(static_cast<int>(bits[h]), off)));
+            if (kg == 0) (h < 2 ? eu : ev)[64 * (h & 1) + r] = factor_exponent(bits[h]);
+        }
+    }
+    load(0);
+    __syncthreads();
+    float sc[4];
 #pragma unroll
-        for (int s2 = 0; s2 < KS; ++s2)
+    for (int h = 0; h < 4; ++h) sc[h] = factor_scale((h < 2 ? eu : ev)[64 * (h & 1) + r]);
+
+    auto stage = [&](u32x4 *as, u32x4 *bs) __attribute__((always_inline)) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+        for (int h = 0; h < 4; ++h) {
+            float y[8];
 #pragma unroll
-                for (int jj = 0; jj < 4; ++jj)
-                    acc[i][jj] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][s2], b[jj][s2], acc[i][jj], 0, 0, 0);
+            for (int i = 0; i < 8; ++i) y[i] = (h < 2 ? v[h][i] * s8[i] : v[h][i]) * sc[h];
+            u32x4 hp, lp;
+            split8(y, hp, lp);
+            u32x4 *dst = (h < 2 ? as : bs) + kg * kPitch + 64 * (h & 1) + r;
+            dst[0] = hp;
+            dst[KG * kPitch] = lp;
+        }
+    };
+    Sums acc;
+    acc.clear();
+    auto fetch = [&](Frags &f, const u32x4 *as, const u32x4 *bs, int s) __attribute__((always_inline)) {
+        const int o = (2 * s + (lane >> 5)) * kPitch + (lane & 31);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            f.ah[i] = __builtin_bit_cast(f16x8, as[o + wm0 + 32 * i]);
+            f.bh[i] = __builtin_bit_cast(f16x8, bs[o + wn0 + 32 * i]);
+            f.al[i] = __builtin_bit_cast(f16x8, as[KG * kPitch + o + wm0 + 32 * i]);
+            f.bl[i] = __builtin_bit_cast(f16x8, bs[KG * kPitch + o + wn0 + 32 * i]);
+        }
+    };
+    // slice j is in the current stage once every wave has passed the barrier;
+    // the next one goes to the other stage, read in slice j - 1, while this
+    // one is multiplied
+    auto slice = [&](u32x4 *ac, u32x4 *bc, u32x4 *an, u32x4 *bn, int j) __attribute__((always_inline)) {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the fetched values stay in flight
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (j + 1 < nk) {  // uniform
+            stage(an, bn);
+            load(min(j + 2, nk - 1));
+        }
+        Frags f;
+        fetch(f, ac, bc, 0);
+        acc.multiply(f);
+        fetch(f, ac, bc, 1);
+        acc.multiply(f);
+    };
+    stage(a0, b0);
+    load(min(1, nk - 1));
+    for (int j = 0; j < nk; j += 2) {
+        slice(a0, b0, a1, b1, j);
+        if (j + 1 < nk) slice(a1, b1, a0, b0, j + 1);
     }
 
-    // epilogue: every wave leaves with its own 64 x 64 block through its own
-    // 8 KB of LDS in two 32-row passes (16-byte stores; columns XOR-swizzled
-    // by 16 on alternate groups of four rows), after one barrier (the codes
-    // are consumed)
-    const bool vec_out = ((g.N & 3) == 0) && ((reinterpret_cast<uintptr_t>(g.out) & 15u) == 0);
-    __syncthreads();
-    float *Cw = reinterpret_cast<float *>(smem) + wave * (32 * 64);
+    const int g4 = 4 * (lane >> 5);
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int ii = 0; ii < 2; ++ii)
+        for (int jj = 0; jj < 2; ++jj) {
+            const int cl = wn0 + 32 * jj + (lane & 31), col = n0 + cl;
+            const int ec = ev[cl];
+            float mv[16];
+            if (g.minuend) {  // uniform
 #pragma unroll
-            for (int jj = 0; jj < 4; ++jj)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int rl = 16 * ii + 4 * (lane >> 4) + r, col = 16 * jj + (lane & 15);
-                    Cw[rl * 64 + (col ^ (16 * ((rl >> 2) & 1)))] = acc[2 * h + ii][jj][r];
+                for (int q = 0; q < 16; ++q) {
+                    const int row = min(m0 + wm0 + 32 * i + (q & 3) + 8 * (q >> 2) + g4, g.m - 1);
+                    mv[q] = g.minuend[static_cast<uint64_t>(row) * g.n + min(col, g.n - 1)];
                 }
+            }
 #pragma unroll
-        for (int q = 0; q < 8; ++q) {
-            const int rl = 4 * q + (lane >> 4), c4 = 4 * (lane & 15);
-            const int gi = m0 + wm0 + 32 * h + rl, gj = n0 + wn0 + c4;
-            if (gi >= g.M) continue;
-            const float4 v = *reinterpret_cast<const float4 *>(&Cw[rl * 64 + (c4 ^ (16 * ((rl >> 2) & 1)))]);
-            const uint64_t e = static_cast<uint64_t>(gi) * g.N + gj;
-            if (vec_out && gj + 4 <= g.N) {
-                *reinterpret_cast<float4 *>(g.out + e) = v;
-            } else {
-                const float vv[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-                for (int u = 0; u < 4; ++u)
-                    if (gj + u < g.N) g.out[e + u] = vv[u];
+            for (int q = 0; q < 16; ++q) {
+                const int rl = wm0 + 32 * i + (q & 3) + 8 * (q >> 2) + g4, row = m0 + rl;
+                const int er = eu[rl];
+                float x = __builtin_ldexpf(acc.hi[i][jj][q] + acc.lo[i][jj][q] * kLoInv,
+                                           min(er, 127) + min(ec, 127) - 28);
+                if (er == kInfRow || ec == kInfRow) {
+                    // an infinity has no second piece: these entries in FP32
+                    const float *u = g.U + static_cast<uint64_t>(min(row, g.m - 1)) * g.k;
+                    const float *w = g.V + static_cast<uint64_t>(min(col, g.n - 1)) * g.k;
+                    x = 0.0f;
+#pragma unroll 1
+                    for (int t = 0; t < g.k; ++t) x = fmaf(u[t] * g.S[t], w[t], x);
+                }
+                if (row < g.m && col < g.n)
+                    g.out[static_cast<uint64_t>(row) * g.n + col] = g.minuend ? mv[q] - x : x;
             }
         }
+}
+
+// Ranks below 32: FP32 sums over k.  There the two pieces' own rounding (7e-8
+// of the result) is no smaller than an FP32 chain's, and a full slice would be
+// mostly padding.  64 x 64 tiles, 4 x 4 outputs a lane, the factors in LDS.
+__global__ __launch_bounds__(kThreads) void recon_low_rank_kernel(ReconArgs g) {
+    constexpr int TS = 64;
+    __shared__ float us[BK][TS + 4], vs[BK][TS + 4];
+    int tile_m, tile_n, z;
+    xcd_tile(static_cast<int>(ceil_div(g.m, TS)), static_cast<int>(ceil_div(g.n, TS)), 1, tile_m, tile_n, z);
+    const int m0 = tile_m * TS, n0 = tile_n * TS, tid = threadIdx.x;
+    for (int e = tid; e < TS * g.k; e += kThreads) {
+        const int r = e / g.k, t = e - r * g.k;
+        us[t][r] = g.U[static_cast<uint64_t>(min(m0 + r, g.m - 1)) * g.k + t] * g.S[t];
+        vs[t][r] = g.V[static_cast<uint64_t>(min(n0 + r, g.n - 1)) * g.k + t];
+    }
+    __syncthreads();
+    const int r0 = 4 * (tid >> 4), c0 = 4 * (tid & 15);
+    float acc[4][4] = {};
+    for (int t = 0; t < g.k; ++t) {
+        const float4 u = *reinterpret_cast<const float4 *>(&us[t][r0]), w = *reinterpret_cast<const float4 *>(&vs[t][c0]);
+        const float uu[4] = {u.x, u.y, u.z, u.w}, ww[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(uu[i], ww[j], acc[i][j]);
+    }
+    const bool vec = g.n % 4 == 0 && (reinterpret_cast<uintptr_t>(g.out) & 15u) == 0 &&
+                     (reinterpret_cast<uintptr_t>(g.minuend) & 15u) == 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int row = m0 + r0 + i, col = n0 + c0;
+        if (row >= g.m || col >= g.n) continue;
+        const uint64_t e = static_cast<uint64_t>(row) * g.n + col;
+        if (vec) {  // whole quads: n % 4 == 0
+            float4 x{acc[i][0], acc[i][1], acc[i][2], acc[i][3]};
+            if (g.minuend) {
+                const float4 mv = *reinterpret_cast<const float4 *>(g.minuend + e);
+                x = float4{mv.x - x.x, mv.y - x.y, mv.z - x.z, mv.w - x.w};
+            }
+            *reinterpret_cast<float4 *>(g.out + e) = x;
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (col + j < g.n) g.out[e + j] = g.minuend ? g.minuend[e + j] - acc[i][j] : acc[i][j];
+        }
     }
 }
-
-template <bool DQ>
-void launch_q(const ReconQArgs &g, size_t lds, hipStream_t stream) {
-    auto kern = recon_q_kernel<DQ>;
-    BSQ_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                static_cast<int>(lds)));
-    const unsigned grid = static_cast<unsigned>(ceil_div(g.M, TT) * ceil_div(g.N, TT));
-    kern<<<grid, kThreads, lds, stream>>>(g);
-}
-
-bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 }  // namespace
 
-bool recon_q_supported(int m, int n, int k, const uint8_t *u_codes, const uint8_t *v_codes) {
-    return m > 0 && n > 0 && k >= 64 && k <= kReconQMaxK && k % 64 == 0 && aligned16(u_codes) &&
-           aligned16(v_codes);
-}
-
-void launch_recon_q(int method, const uint8_t *u_codes, const float *u_scales_f32, const uint8_t *u_scales_u8,
-                    const float *u_dq, const uint8_t *v_codes, const float *v_scales_f32, const uint8_t *v_scales_u8,
-                    const float *v_dq, const float *S, int m, int n, int k, float *out, hipStream_t stream) {
-    BSQ_REQUIRE(recon_q_supported(m, n, k, u_codes, v_codes) && S && out, "packed reconstruct: bad arguments");
-    BSQ_REQUIRE(method == kMethodNF4 || method == kMethodNF4DQ, "packed reconstruct: factors are not NF4 / NF4_DQ");
-    const bool dq = method == kMethodNF4DQ;
-    BSQ_REQUIRE(dq ? (u_scales_u8 && v_scales_u8 && u_dq && v_dq) : (u_scales_f32 && v_scales_f32),
-                "packed reconstruct: missing block scales");
-    ReconQArgs g;
-    g.u = QFactor{u_codes, u_scales_f32, u_scales_u8, u_dq};
-    g.v = QFactor{v_codes, v_scales_f32, v_scales_u8, v_dq};
-    g.s = S;
-    g.out = out;
-    g.M = m;
-    g.N = n;
-    g.K = k;
-    const size_t lds = static_cast<size_t>(Layout(k).bytes);
-    if (dq) launch_q<true>(g, lds, stream);
-    else launch_q<false>(g, lds, stream);
+void launch_reconstruct(const float *U, const float *S, const float *V, int m, int n, int k, const float *minuend,
+                        float *out, int *exponents, hipStream_t stream) {
+    BSQ_REQUIRE(m > 0 && n > 0 && k > 0 && U && S && V && out, "reconstruct: bad arguments");
+    ReconArgs g{U, S, V, minuend, out, exponents, exponents ? exponents + m : nullptr, m, n, k};
+    if (k < BK) {
+        recon_low_rank_kernel<<<static_cast<unsigned>(ceil_div(m, 64) * ceil_div(n, 64)), kThreads, 0, stream>>>(g);
+        BSQ_HIP(hipGetLastError());
+        return;
+    }
+    if (exponents) {
+        factor_exponent_kernel<<<static_cast<unsigned>(ceil_div(static_cast<uint64_t>(m) + n, kThreads / 64)), kThreads,
+                                 0, stream>>>(U, S, V, m, n, k, exponents);
+        BSQ_HIP(hipGetLastError());
+    }
+    recon_kernel<<<static_cast<unsigned>(ceil_div(m, T) * ceil_div(n, T)), kThreads, 0, stream>>>(g);
     BSQ_HIP(hipGetLastError());
 }
 

@@ -299,6 +299,7 @@ struct Runtime {
     TopkBuf topk[2];
     Meta *meta = nullptr;
     SvdPlan *svd = nullptr;
+    int *recon_exp = nullptr;       // row exponents of the factors (launch_reconstruct)
     const float *sketch = nullptr;  // injected Gaussian sketch (test hook)
     // decompress-side staging for quantised sections (shared, like the reference's buffers)
     float *q_scales_f32 = nullptr;
@@ -323,6 +324,7 @@ struct Runtime {
         dev_free(d_err);
         dev_free(d_row_gmax);
         dev_free(meta);
+        dev_free(recon_exp);
         dev_free(q_scales_f32);
         dev_free(q_scales_u8);
         dev_free(q_codes);
@@ -516,7 +518,10 @@ void compress_init(Runtime &rt, uint16_t rows, uint16_t cols, float r_out, float
             if (sc.method != kMethodNone) sc.alloc_quant();
         }
         rt.reconstruct_initialized = true;
-        if (rt.topk[TK_ERROR].capacity > 0) rt.d_err = dev_alloc<float>(N);
+        if (rt.topk[TK_ERROR].capacity > 0) {
+            rt.d_err = dev_alloc<float>(N);
+            rt.recon_exp = dev_alloc<int>(static_cast<uint64_t>(rows) + cols);
+        }
     } else {
         Section &sc = rt.sec[SEC_DIRECT];
         sc.method = direct;
@@ -556,6 +561,7 @@ void decompress_init(Runtime &rt, uint16_t rows, uint16_t cols, float r_out, flo
             rt.sec[i].dense = dev_alloc<float>(counts[i]);
             rt.sec[i].own_dense = true;
         }
+        rt.recon_exp = dev_alloc<int>(static_cast<uint64_t>(rows) + cols);
         rt.reconstruct_initialized = true;
     }
     if (uses_quant(rt)) {
@@ -679,7 +685,7 @@ void compress_device(Runtime &rt, const float *d_in, bsq_device_packed_t *out, c
         if (te.capacity > 0) {
             // reconstruct + subtract fused (src/bitsqz_llm.cu:1141-1163)
             timed_launch(kTimeReconstruct, st, [&] {
-                launch_reconstruct(U.dense, S.dense, V.dense, rows, cols, rt.q, residual, rt.d_err, st);
+                launch_reconstruct(U.dense, S.dense, V.dense, rows, cols, rt.q, residual, rt.d_err, rt.recon_exp, st);
             });
             mark(5);
             TopkArgs a;
@@ -849,33 +855,21 @@ void decompress_device(Runtime &rt, const bsq_device_packed_t &P, const bool has
     const uint32_t ke = has_error ? P.topk_k[1] : 0, ko = has_outlier ? P.topk_k[0] : 0;
     if (H.flags & kFlagSvd) {
         const int q = static_cast<uint16_t>(H.effective_rank);
-        // packed U and V: the reconstruction decodes them inline
-        const bool fused = H.svd_uv_format != kMethodNone && !P.d_dense[SEC_U] && !P.d_dense[SEC_V] &&
-                           recon_q_supported(rows, cols, q, P.d_codes[SEC_U], P.d_codes[SEC_V]);
         const float *dense[3];
         for (int i = 0; i < 3; ++i) {
             if (P.d_dense[i]) {
                 dense[i] = P.d_dense[i];
-            } else if (!(fused && i != SEC_S)) {
-                Section &sc = rt.sec[i];  // decompress runtime's dense U / S / V
-                const int method = (i == SEC_S) ? H.svd_s_format : H.svd_uv_format;
-                launch_quant_decode(P.count[i], method, P.d_scales_f32[i], P.d_scales_u8[i], P.d_dq_scale[i],
-                                    P.d_codes[i], sc.dense, st);
-                dense[i] = sc.dense;
-            } else {
-                dense[i] = nullptr;
+                continue;
             }
+            Section &sc = rt.sec[i];  // decompress runtime's dense U / S / V
+            const int method = (i == SEC_S) ? H.svd_s_format : H.svd_uv_format;
+            launch_quant_decode(P.count[i], method, P.d_scales_f32[i], P.d_scales_u8[i], P.d_dq_scale[i],
+                                P.d_codes[i], sc.dense, st);
+            dense[i] = sc.dense;
         }
-        if (fused) {
-            timed_launch(kTimeReconstruct, st, [&] {
-                launch_recon_q(H.svd_uv_format, P.d_codes[SEC_U], P.d_scales_f32[SEC_U], P.d_scales_u8[SEC_U],
-                               P.d_dq_scale[SEC_U], P.d_codes[SEC_V], P.d_scales_f32[SEC_V], P.d_scales_u8[SEC_V],
-                               P.d_dq_scale[SEC_V], dense[SEC_S], rows, cols, q, d_dst, st);
-            });
-        } else {
-            timed_launch(kTimeReconstruct, st,
-                       [&] { launch_reconstruct(dense[0], dense[1], dense[2], rows, cols, q, nullptr, d_dst, st); });
-        }
+        timed_launch(kTimeReconstruct, st, [&] {
+            launch_reconstruct(dense[0], dense[1], dense[2], rows, cols, q, nullptr, d_dst, rt.recon_exp, st);
+        });
     } else {
         const uint64_t N = static_cast<uint64_t>(rows) * cols;
         if (P.d_dense[SEC_DIRECT]) {
@@ -1233,24 +1227,8 @@ void decompress_host(Runtime &rt, const bitsqz_llm_array_t *c, float *d_dst) {
         P.topk_k[t] = h.num_topk_columns;
     }
 
-    // Packed U and V of the SVD path stay packed for the reconstruction, which
-    // decodes them inline, when both fit the shared staging side by side;
-    // otherwise every section is decoded as soon as it arrives (the staging
-    // is then shared).
-    const uint64_t uq = (c->flags & kFlagSvd) ? static_cast<uint64_t>(rows) * static_cast<uint16_t>(c->effective_rank) : 0;
-    const uint64_t vq = (c->flags & kFlagSvd) ? static_cast<uint64_t>(cols) * static_cast<uint16_t>(c->effective_rank) : 0;
-    const uint64_t v_code_off = ceil_div(uq / 2, 256) * 256, v_scale_off = ceil_div(uq / kQuantBlock, 64) * 64;
-    // a packed S is decoded at once, from behind V (U and V must stay intact)
-    const uint64_t s_code_off = ceil_div(v_code_off + vq / 2, 256) * 256,
-                   s_scale_off = ceil_div(v_scale_off + vq / kQuantBlock, 64) * 64;
-    const uint64_t sq = (c->flags & kFlagSvd) ? static_cast<uint16_t>(c->effective_rank) : 0;
-    const bool keep_packed = (c->flags & kFlagSvd) && c->svd_uv_format != kMethodNone && rt.quant_initialized &&
-                             c->section_u.storage == BITSQZ_SECTION_QUANT &&
-                             c->section_v.storage == BITSQZ_SECTION_QUANT &&
-                             recon_q_supported(rows, cols, static_cast<uint16_t>(c->effective_rank), rt.q_codes,
-                                               rt.q_codes + v_code_off) &&
-                             s_code_off + (sq + 1) / 2 <= (N + 1) / 2 &&
-                             s_scale_off + ceil_div(sq, kQuantBlock) <= ceil_div(N, kQuantBlock);
+    // Every section is decoded as soon as it arrives (the staging of packed
+    // sections is shared).
     auto stage_section = [&](int i, const bitsqz_section_t &s, int method, uint64_t count, float *dense_dst) {
         if (s.storage == BITSQZ_SECTION_FP32) {
             BSQ_REQUIRE(s.size == count * 4, "FP32 section size mismatch");
@@ -1268,26 +1246,14 @@ void decompress_host(Runtime &rt, const bitsqz_llm_array_t *c, float *d_dst) {
         // the header and block scales staged at once, the codes piecewise
         const bitsqz_section_t head{s.offset, 48 + ssz, s.storage};
         const uint8_t *pl = staged(head);
-        // packed U at the start of the staging, packed V after it
-        const bool packed = keep_packed && (i == SEC_U || i == SEC_V);
-        const uint64_t coff = !keep_packed ? 0 : (i == SEC_V ? v_code_off : (i == SEC_S ? s_code_off : 0));
-        const uint64_t soff = !keep_packed ? 0 : (i == SEC_V ? v_scale_off : (i == SEC_S ? s_scale_off : 0));
-        float *sc_f32 = rt.q_scales_f32 + soff;
-        uint8_t *sc_u8 = rt.q_scales_u8 + soff, *codes = rt.q_codes + coff;
+        float *sc_f32 = rt.q_scales_f32;
+        uint8_t *sc_u8 = rt.q_scales_u8, *codes = rt.q_codes;
         void *sdst = method == kMethodNF4 ? static_cast<void *>(sc_f32) : static_cast<void *>(sc_u8);
         BSQ_HIP(hipMemcpyAsync(sdst, pl + s.offset + 48, ssz, hipMemcpyHostToDevice, st));
         h2d_pieces(codes, s.offset + 48 + ssz, (count + 1) / 2, st);
         if (method == kMethodNF4DQ)
             BSQ_HIP(hipMemcpyAsync(&rt.meta->dq[i], pl + s.offset + 40, 4, hipMemcpyHostToDevice, st));
         P.count[i] = count;
-        if (packed) {
-            P.d_dense[i] = nullptr;
-            P.d_codes[i] = codes;
-            P.d_scales_f32[i] = method == kMethodNF4 ? sc_f32 : nullptr;
-            P.d_scales_u8[i] = method == kMethodNF4DQ ? sc_u8 : nullptr;
-            P.d_dq_scale[i] = method == kMethodNF4DQ ? &rt.meta->dq[i] : nullptr;
-            return;
-        }
         // decode now (the staging buffers are shared between sections)
         launch_quant_decode(count, method, sc_f32, sc_u8, &rt.meta->dq[i], codes, dense_dst, st);
         P.d_dense[i] = dense_dst;
@@ -1788,7 +1754,7 @@ int bsq_reconstruct_lowrank(const float *d_U, const float *d_S, const float *d_V
                             void *stream) {
     return guarded([&] {
         BSQ_REQUIRE(m > 0 && n > 0 && k > 0, "reconstruct: bad shape");
-        launch_reconstruct(d_U, d_S, d_V, m, n, k, nullptr, d_out, static_cast<hipStream_t>(stream));
+        launch_reconstruct(d_U, d_S, d_V, m, n, k, nullptr, d_out, nullptr, static_cast<hipStream_t>(stream));
     });
 }
 

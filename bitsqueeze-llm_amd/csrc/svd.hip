@@ -1,5 +1,5 @@
-// Randomised rank-q SVD (range finder with power iterations), the low-rank
-// reconstruction and the Gaussian sketch generator.
+// Randomised rank-q SVD (range finder with power iterations) and the Gaussian
+// sketch generator.
 //
 // Algorithm (reference modules/svd_lowrank_cuda/src/svd_lowrank_cuda.cu:
 // 129-137, 284-426, 478-524): with A_w = A (m >= n) or A^T (m < n), of size
@@ -28,8 +28,7 @@ namespace bsq {
 // launchers from gemm.hip / linalg.hip
 uint64_t gemm_workspace_bytes(int M, int N, int K);
 void launch_gemm(bool ta, bool tb, int M, int N, int K, const float *A, int lda, const float *B, int ldb, float *C,
-                 int ldc, const float *a_colscale, const float *minuend, float *workspace, uint64_t workspace_bytes,
-                 hipStream_t stream);
+                 int ldc, float *workspace, uint64_t workspace_bytes, hipStream_t stream);
 uint64_t gram_workspace_bytes(int M, int k);
 void launch_gram(const float *X, int M, int k, int ld, double *G, double *workspace, hipStream_t stream,
                  double *rowsq = nullptr);
@@ -401,7 +400,7 @@ void svd_run(SvdPlan *p, const float *A, const float *sketch, uint64_t seed, flo
             if (p->h2 && Bm != sketch)
                 launch_h2_gemm(ta, m, n, k, A, p->h2s, Bm, p->planes, out, p->gemm_ws, p->gemm_ws_bytes, st);
             else
-                launch_gemm(ta, false, ta ? n : m, k, ta ? m : n, A, n, Bm, k, out, k, nullptr, nullptr, p->gemm_ws,
+                launch_gemm(ta, false, ta ? n : m, k, ta ? m : n, A, n, Bm, k, out, k, p->gemm_ws,
                             p->gemm_ws_bytes, st);
         });
     };
@@ -418,7 +417,7 @@ void svd_run(SvdPlan *p, const float *A, const float *sketch, uint64_t seed, flo
             launch_chol_inv_2x2(p->G, k, p->scratch, p->Linv, p->status, st);
         else
             launch_chol_inv(p->G, k, p->W, p->Linv, p->status, p->scratch, st);
-        launch_gemm(false, true, rows, k, k, in, k, p->Linv, k, out, k, nullptr, nullptr, p->gemm_ws,
+        launch_gemm(false, true, rows, k, k, in, k, p->Linv, k, out, k, p->gemm_ws,
                     p->gemm_ws_bytes, st);
     };
     float *Xa = p->X, *Xb = p->X2, *Ya = p->Y, *Yb = p->Y2;
@@ -438,7 +437,7 @@ void svd_run(SvdPlan *p, const float *A, const float *sketch, uint64_t seed, flo
     if (p->Lbuf) {
         launch_gram(Xa, Mw, k, k, p->G, p->gram_ws, st, p->rowsq);
         launch_orth_refine(p->G, p->rowsq, k, p->Lbuf, p->Linv, p->status, p->status + 1, st);
-        launch_gemm(false, false, Mw, k, k, Xa, k, p->Linv, k, Xb, k, nullptr, nullptr, p->gemm_ws,
+        launch_gemm(false, false, Mw, k, k, Xa, k, p->Linv, k, Xb, k, p->gemm_ws,
                     p->gemm_ws_bytes, st);
     } else {
         orth(Xa, Xb, Mw);
@@ -452,9 +451,9 @@ void svd_run(SvdPlan *p, const float *A, const float *sketch, uint64_t seed, flo
     BSQ_HIP(hipGetLastError());
     float *Uw_out = p->transposed ? V : U;  // Mw x k
     float *Vh_out = p->transposed ? U : V;  // Nw x k
-    launch_gemm(false, false, Mw, k, k, Xa, k, p->Uh, k, Uw_out, k, nullptr, nullptr, p->gemm_ws, p->gemm_ws_bytes,
+    launch_gemm(false, false, Mw, k, k, Xa, k, p->Uh, k, Uw_out, k, p->gemm_ws, p->gemm_ws_bytes,
                 st);
-    launch_gemm(false, false, Nw, k, k, Ya, k, p->Uh, k, Vh_out, k, nullptr, nullptr, p->gemm_ws, p->gemm_ws_bytes,
+    launch_gemm(false, false, Nw, k, k, Ya, k, p->Uh, k, Vh_out, k, p->gemm_ws, p->gemm_ws_bytes,
                 st);
     // V_hat = Y U_hat / S (columns normalised), then the sign convention: the
     // first largest-|.| entry of every column of U is non-negative (U and V
@@ -474,13 +473,6 @@ void svd_run(SvdPlan *p, const float *A, const float *sketch, uint64_t seed, flo
                                                                      p->csign + k);
         BSQ_HIP(hipGetLastError());
     }
-}
-
-void launch_reconstruct(const float *U, const float *S, const float *V, int m, int n, int k, const float *minuend,
-                        float *out, hipStream_t stream) {
-    BSQ_REQUIRE(m > 0 && n > 0 && k > 0 && U && S && V && out, "reconstruct: bad arguments");
-    // out = (minuend -) (U diag(S)) V^T: A = U with columns scaled by S, B = V^T
-    launch_gemm(false, true, m, n, k, U, k, V, k, out, n, S, minuend, nullptr, 0, stream);
 }
 
 void launch_gaussian_fill(float *out, uint64_t n, uint64_t seed, hipStream_t stream) {
