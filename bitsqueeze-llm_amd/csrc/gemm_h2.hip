@@ -40,7 +40,7 @@ constexpr int kThreads = 256;
 constexpr int T = 128;        // output tile
 constexpr int BK = 32;        // K slice
 constexpr int KG = BK / 8;    // groups of eight k per slice
-constexpr int kPitchA = 132;  // 16-byte units per k group of a staged A plane (128 rows, padded)
+constexpr int kPitchA = 130;  // 16-byte units per k group of a staged A plane (128 rows, padded)
 constexpr int kScaleB = 11;   // B's scale, a power of two
 
 __device__ __forceinline__ void dma16(const u32x4 *g, const u32x4 *l) {
@@ -122,16 +122,16 @@ __global__ __launch_bounds__(kThreads) void split_b_kernel(const float *__restri
     for (int i = 0; i < 8; ++i) {
         y[i] = n < N ? B[static_cast<uint64_t>(8 * kg + i) * N + n] : 0.0f;
     }
+    float f[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) f[i] = static_cast<float>(1 << kScaleB);
     if (E) {
         const int em = *emax;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) y[i] = __builtin_ldexpf(y[i], E[8 * kg + i] - em + kScaleB);
-    } else {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) y[i] *= static_cast<float>(1 << kScaleB);
+        for (int i = 0; i < 8; ++i) f[i] = pow2(max(E[8 * kg + i] - em, -138) + kScaleB);
     }
     u32x4 h, l;
-    split8(y, h, l);
+    split8(y, [&](int i) { return f[i]; }, h, l);
     hi[t] = h;
     lo[t] = l;
 }
@@ -214,15 +214,17 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
             __builtin_memcpy(&va[0], __builtin_assume_aligned(p0, 4), 32);
             __builtin_memcpy(&va[8], __builtin_assume_aligned(p1, 4), 32);
         } else {
-            const int c0 = min(m0 + lane, g.M - 1), c1 = min(m0 + 64 + lane, g.M - 1);
-            const int k = k0 + 8 * wave;
+            // k-rows are the wave's own: scalar bases, one 32-bit offset a column
+            const uint32_t c0 = 4u * static_cast<uint32_t>(min(m0 + lane, g.M - 1));
+            const uint32_t c1 = 4u * static_cast<uint32_t>(min(m0 + 64 + lane, g.M - 1));
 #pragma unroll
-            for (int i = 0; i < 8; ++i) vs[i] = g.rs[k + i];
+            for (int i = 0; i < 8; ++i) vs[i] = g.rs[k0 + 8 * wave + i];
+            const char *p = reinterpret_cast<const char *>(g.A) +
+                            4u * static_cast<uint64_t>(k0 + 8 * __builtin_amdgcn_readfirstlane(wave)) * g.lda;
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const float *p = g.A + static_cast<uint64_t>(k + i) * g.lda;
-                va[i] = p[c0];
-                va[8 + i] = p[c1];
+            for (int i = 0; i < 8; ++i, p += 4u * static_cast<uint64_t>(g.lda)) {
+                va[i] = *reinterpret_cast<const float *>(p + c0);
+                va[8 + i] = *reinterpret_cast<const float *>(p + c1);
             }
         }
         ca.next(nk, g.tiles_n);
@@ -235,11 +237,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         for (int i = 0; i < 16; ++i) asm volatile("" : "+v"(va[i]));
 #pragma unroll
         for (int half = 0; half < 2; ++half) {
-            float y[8];
+            float x[8];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) y[i] = va[8 * half + i] * (TA ? vs[i] : vs[half]);
+            for (int i = 0; i < 8; ++i) x[i] = va[8 * half + i];
             u32x4 h, l;
-            split8(y, h, l);
+            split8(x, [&](int i) { return TA ? vs[i] : vs[half]; }, h, l);
             as[kg * kPitchA + 64 * half + row] = h;
             as[(KG + kg) * kPitchA + 64 * half + row] = l;
         }
@@ -374,7 +376,7 @@ struct H2Plan {
 };
 
 // Two workgroups per CU share the slices, unless that leaves a workgroup
-// fewer than four pairs of them (256 k): the parts' traffic and the serial sum of
+// fewer than two pairs of them (128 k): the parts' traffic and the serial sum of
 // a tile's parts then cost more than the idle CUs.
 H2Plan h2_plan(int M, int N, int K) {
     H2Plan p{};
@@ -383,7 +385,7 @@ H2Plan h2_plan(int M, int N, int K) {
     p.pairs = K / (2 * BK);  // the rest of K goes with the reduction
     p.units = p.tiles * p.pairs;
     const int most = 2 * cu_count();
-    p.G = std::max(1, std::min(most, std::max(p.tiles, p.units / 4)));
+    p.G = std::max(1, std::min(most, std::max(p.tiles, p.units / 2)));
     p.G = std::min(p.G, p.units);
     p.maxparts = 1;
     for (int t = 0; t < p.tiles; ++t) {

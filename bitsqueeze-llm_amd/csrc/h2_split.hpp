@@ -40,15 +40,27 @@ __device__ __forceinline__ int row_exponent(uint32_t bits) {
 // 2^e, e in [-149, 127]
 __device__ __forceinline__ float pow2(int e) { return __builtin_ldexpf(1.0f, e); }
 
-// eight scaled values to their pieces
-__device__ __forceinline__ void split8(const float (&y)[8], u32x4 &h, u32x4 &l) {
+// eight values x, scaled by f, to their pieces.  Three mixed-precision FMAs a
+// value write the pieces into their halves (h = f16(f x), f x - h exactly,
+// l = f16 of 2^11 times that); left to the compiler it is five instructions,
+// with the products and the packing of their own.
+template <class F>
+__device__ __forceinline__ void split8(const float (&x)[8], F &&f, u32x4 &h, u32x4 &l) {
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
-        const f16x2 hp{static_cast<_Float16>(y[2 * p]), static_cast<_Float16>(y[2 * p + 1])};
-        const f16x2 lp{static_cast<_Float16>((y[2 * p] - static_cast<float>(hp.x)) * kLo),
-                       static_cast<_Float16>((y[2 * p + 1] - static_cast<float>(hp.y)) * kLo)};
-        h[p] = __builtin_bit_cast(uint32_t, hp);
-        l[p] = __builtin_bit_cast(uint32_t, lp);
+        const float x0 = x[2 * p], x1 = x[2 * p + 1], f0 = f(2 * p), f1 = f(2 * p + 1);
+        uint32_t hp, lp;
+        float r0, r1;
+        asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "=v"(hp) : "v"(x0), "v"(f0));
+        asm("v_fma_mixhi_f16 %0, %1, %2, 0" : "+v"(hp) : "v"(x1), "v"(f1));
+        asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel_hi:[0,0,1]" : "=v"(r0) : "v"(x0), "v"(f0), "v"(hp));
+        asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel:[0,0,1] op_sel_hi:[0,0,1]"
+            : "=v"(r1)
+            : "v"(x1), "v"(f1), "v"(hp));
+        asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "=v"(lp) : "v"(r0), "s"(kLo));
+        asm("v_fma_mixhi_f16 %0, %1, %2, 0" : "+v"(lp) : "v"(r1), "s"(kLo));
+        h[p] = hp;
+        l[p] = lp;
     }
 }
 

@@ -25,7 +25,7 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int T = 128, BK = 32, KG = BK / 8;
-constexpr int kPitch = 132;      // 16-byte units per k group of a plane (128 rows, padded)
+constexpr int kPitch = 130;      // 16-byte units per k group of a plane (128 rows, padded)
 constexpr int kInfRow = 128;     // "exponent" of a row that holds infinities and no NaN
 
 struct ReconArgs {
@@ -133,11 +133,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     auto stage = [&](u32x4 *as, u32x4 *bs) __attribute__((always_inline)) {
 #pragma unroll
         for (int h = 0; h < 4; ++h) {
-            float y[8];
+            float x[8];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) y[i] = (h < 2 ? v[h][i] * s8[i] : v[h][i]) * sc[h];
+            for (int i = 0; i < 8; ++i) x[i] = h < 2 ? v[h][i] * s8[i] : v[h][i];
             u32x4 hp, lp;
-            split8(y, hp, lp);
+            split8(x, [&](int) { return sc[h]; }, hp, lp);
             u32x4 *dst = (h < 2 ? as : bs) + kg * kPitch + 64 * (h & 1) + r;
             dst[0] = hp;
             dst[KG * kPitch] = lp;
