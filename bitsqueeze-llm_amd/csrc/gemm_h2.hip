@@ -8,11 +8,10 @@
 // The split and its error: h2_split.hpp.
 // Three f16 products run at up to 5 times the FP32 matrix rate (2.5 / 3
 // against 0.157 PFLOP/s).  Measured, against the FP32 kernels with their
-// reductions: 4096 x 11008 with q = 128 101 -> 49 us (A^T B) and 98 -> 49 us
-// (A B); 16384 x 14336 with q = 512 1986 -> 1033 and 1590 -> 872 us (0.83
-// PFLOP/s of f16 products, two thirds of what a large library f16 product
-// reaches on this card: the staging's LDS traffic and the power limit are
-// what is left).
+// reductions: 4096 x 11008 with q = 128 101 -> 47 us (A^T B) and 98 -> 47 us
+// (A B); 16384 x 14336 with q = 512 1986 -> 838 and 1590 -> 825 us, 0.86
+// PFLOP/s of f16 products (a large library bf16 product reaches 1.2 on this
+// card; the clock falls to 1.9 GHz under the matrix cores' power).
 //
 // Scales.  Row i of A is scaled so that its largest magnitude falls in
 // [2^14, 2^15) (row_scale_kernel, once per matrix).  With TA = false that is
@@ -40,7 +39,6 @@ constexpr int kThreads = 256;
 constexpr int T = 128;        // output tile
 constexpr int BK = 32;        // K slice
 constexpr int KG = BK / 8;    // groups of eight k per slice
-constexpr int kPitchA = 130;  // 16-byte units per k group of a staged A plane (128 rows, padded)
 constexpr int kScaleB = 11;   // B's scale, a power of two
 
 __device__ __forceinline__ void dma16(const u32x4 *g, const u32x4 *l) {
@@ -140,34 +138,44 @@ struct H2Args {
     const float *A;
     const u32x4 *bh, *bl;  // B's planes
     const float *rs;       // scales of A's rows
-    float *ws;             // partial tiles [tile][part][T][T]
+    float *ws;             // partial tiles [tile row][tile column][part][tile]
     int M, K, lda;
     int np;                // columns of the planes (a multiple of 64)
     int tiles_n;           // output tiles per row of tiles
     int pairs;             // pairs of K slices per tile
-    int units;             // tiles x pairs
+    int units;             // tile rows x pairs
+    int ranges;            // contiguous shares of the units
     int maxparts;          // workspace slots per tile
 };
 
-// logical workgroup whose range holds unit u
-__host__ __device__ __forceinline__ int h2_owner(int64_t u, int64_t units, int G) {
-    return static_cast<int>(((u + 1) * G - 1) / units);
+// range that holds unit u
+__host__ __device__ __forceinline__ int h2_owner(int64_t u, int64_t units, int ranges) {
+    return static_cast<int>(((u + 1) * ranges - 1) / units);
 }
 
-// Stream-K: G workgroups share the tiles' K slices in equal contiguous
-// ranges, one range a workgroup, laid so that an XCD runs a contiguous eighth
-// of them; each writes its partial sum of every tile it touches and
-// h2_reduce_kernel adds a tile's parts in order.  128 x 128 tiles, four waves
-// of 64 x 64 in 32 x 32 blocks with both sums in accumulator registers (128
-// of 256 a lane), so two workgroups share a CU and one's staging and barriers
-// run under the other's matrix instructions.  Slices of 32 k: B's pieces go
-// global -> LDS directly one slice ahead; A's values are fetched into
-// registers two slices ahead (row-major: a lane takes eight consecutive k of
-// two rows; A^T: eight k-rows of two columns, so the transposition is only a
-// choice of registers), then split and written to LDS in the same
-// [k group][row] units of 16 bytes that the fragments are read in.
+// Stream-K: the K slices of all tile rows, in pairs, are cut into equal
+// contiguous ranges; the tiles_n workgroups of a range run the same slices of
+// A against their own columns of B, side by side on one XCD, so A comes from
+// HBM once (with ranges cut over the tiles themselves the workgroups of a tile
+// row drift apart: 6.9 GB instead of 2.2 GB through the L2s' misses at
+// 14336 x 16384 x 512).  Each workgroup writes its partial sum of every tile
+// it touches and h2_reduce_kernel adds a tile's parts in order.
+//
+// 128 x 128 tiles, four waves of 64 x 64 in 32 x 32 blocks with both sums in
+// accumulator registers (128 of 256 a lane), so two workgroups share a CU and
+// one's staging and barriers run under the other's matrix instructions.
+// 128 x 256 and 256 x 128 tiles (one workgroup a CU, three quarters of the
+// operand bytes per product) measured the same within 3 %, as one 128 x 128
+// workgroup a CU does: the matrix cores' power, not the operands' way, sets
+// the rate.  Slices of 32 k: B's pieces go global -> LDS directly one slice
+// ahead; A's values are fetched into registers two slices ahead (row-major: a
+// lane takes eight consecutive k of two rows; A^T: eight k-rows of two
+// columns, so the transposition is only a choice of registers), then split and
+// written to LDS in the same [k group][row] units of 16 bytes that the
+// fragments are read in.
 template <bool TA>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_h2_kernel(H2Args g) {
+    constexpr int kPitchA = T + 2;  // 16-byte units per k group of a staged A plane: +2 spreads the writes' banks
     __shared__ u32x4 a0[2 * KG * kPitchA], a1[2 * KG * kPitchA];  // h plane, l plane
     __shared__ __attribute__((aligned(1024))) u32x4 b0[2 * KG * T], b1[2 * KG * T];
     constexpr int kLoadsA = TA ? 18 : 6;  // vector loads of one A slice and its scales, at least
@@ -177,140 +185,128 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     const int G = static_cast<int>(gridDim.x), bid = static_cast<int>(blockIdx.x);
     const int xcd = bid % kXcds, loc = bid / kXcds;
     const int L = xcd * (G / kXcds) + min(xcd, G % kXcds) + loc;
-    const int p0 = static_cast<int>(static_cast<int64_t>(L) * g.units / G);
-    const int n = static_cast<int>(static_cast<int64_t>(L + 1) * g.units / G) - p0;  // slice pairs
+    const int range = L / g.tiles_n, tn = L - range * g.tiles_n;
+    const int p0 = static_cast<int>(static_cast<int64_t>(range) * g.units / g.ranges);
+    const int n = static_cast<int>(static_cast<int64_t>(range + 1) * g.units / g.ranges) - p0;  // slice pairs
 
-    // a position in the slices of the range (tile row, tile column, slice),
-    // `left` slices before its last
+    // a position in the slices of the range (tile row, slice), `left` slices
+    // before its last
     struct Cursor {
-        int tm, tn, ks, left;
-        __device__ __forceinline__ void next(int nk, int tiles_n) {
+        int tm, ks, left;
+        __device__ __forceinline__ void next(int nk) {
             // by selects: branches here would split the accumulators' live ranges
             const int step = left > 0 ? 1 : 0;
             left -= step;
             const int w = ks + step == nk ? 1 : 0;
             ks = w ? 0 : ks + step;
-            const int w2 = tn + w == tiles_n ? 1 : 0;
-            tn = w2 ? 0 : tn + w;
-            tm += w2;
+            tm += w;
         }
     };
     const int nk = 2 * g.pairs, tile0 = p0 / g.pairs;
-    Cursor ca{tile0 / g.tiles_n, tile0 % g.tiles_n, 2 * (p0 - tile0 * g.pairs), 2 * n - 1};  // next A slice to fetch
-    Cursor cb = ca;                                                                       // next B slice to fetch
+    Cursor ca{tile0, 2 * (p0 - tile0 * g.pairs), 2 * n - 1};  // next A slice to fetch
+    Cursor cb = ca;                                           // next B slice to fetch
 
-    float va[16];  // A values in flight
+    float va[2][8];  // A values in flight
     float vs[TA ? 8 : 2];
     auto load_a = [&]() __attribute__((always_inline)) {
         const int m0 = ca.tm * T, k0 = ca.ks * BK;
         asm volatile("" ::: "memory");  // stays behind the DMA before it
         if constexpr (!TA) {
-            const int r0 = min(m0 + (tid >> 2), g.M - 1), r1 = min(m0 + 64 + (tid >> 2), g.M - 1);
             const int k = k0 + 8 * (tid & 3);
-            vs[0] = g.rs[r0];
-            vs[1] = g.rs[r1];
-            const float *p0 = g.A + static_cast<uint64_t>(r0) * g.lda + k, *p1 = g.A + static_cast<uint64_t>(r1) * g.lda + k;
-            // rows may start at any multiple of four bytes
-            __builtin_memcpy(&va[0], __builtin_assume_aligned(p0, 4), 32);
-            __builtin_memcpy(&va[8], __builtin_assume_aligned(p1, 4), 32);
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int r = min(m0 + 64 * h + (tid >> 2), g.M - 1);
+                vs[h] = g.rs[r];
+                // rows may start at any multiple of four bytes
+                __builtin_memcpy(&va[h][0], __builtin_assume_aligned(g.A + static_cast<uint64_t>(r) * g.lda + k, 4), 32);
+            }
         } else {
             // k-rows are the wave's own: scalar bases, one 32-bit offset a column
-            const uint32_t c0 = 4u * static_cast<uint32_t>(min(m0 + lane, g.M - 1));
-            const uint32_t c1 = 4u * static_cast<uint32_t>(min(m0 + 64 + lane, g.M - 1));
+            uint32_t c[2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) c[h] = 4u * static_cast<uint32_t>(min(m0 + 64 * h + lane, g.M - 1));
 #pragma unroll
             for (int i = 0; i < 8; ++i) vs[i] = g.rs[k0 + 8 * wave + i];
             const char *p = reinterpret_cast<const char *>(g.A) +
                             4u * static_cast<uint64_t>(k0 + 8 * __builtin_amdgcn_readfirstlane(wave)) * g.lda;
 #pragma unroll
-            for (int i = 0; i < 8; ++i, p += 4u * static_cast<uint64_t>(g.lda)) {
-                va[i] = *reinterpret_cast<const float *>(p + c0);
-                va[8 + i] = *reinterpret_cast<const float *>(p + c1);
-            }
+            for (int i = 0; i < 8; ++i, p += 4u * static_cast<uint64_t>(g.lda))
+#pragma unroll
+                for (int h = 0; h < 2; ++h) va[h][i] = *reinterpret_cast<const float *>(p + c[h]);
         }
-        ca.next(nk, g.tiles_n);
+        ca.next(nk);
     };
     auto stage_a = [&](u32x4 *as) __attribute__((always_inline)) {
         const int row = TA ? lane : tid >> 2, kg = TA ? wave : tid & 3;
         // the values are first touched here: their scaling, moved up past the
         // barrier, would wait for them a slice early
 #pragma unroll
-        for (int i = 0; i < 16; ++i) asm volatile("" : "+v"(va[i]));
+        for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int half = 0; half < 2; ++half) {
-            float x[8];
+            for (int i = 0; i < 8; ++i) asm volatile("" : "+v"(va[h][i]));
 #pragma unroll
-            for (int i = 0; i < 8; ++i) x[i] = va[8 * half + i];
-            u32x4 h, l;
-            split8(x, [&](int i) { return TA ? vs[i] : vs[half]; }, h, l);
-            as[kg * kPitchA + 64 * half + row] = h;
-            as[(KG + kg) * kPitchA + 64 * half + row] = l;
+        for (int h = 0; h < 2; ++h) {
+            u32x4 hp, lp;
+            split8(va[h], [&](int i) { return TA ? vs[i] : vs[h]; }, hp, lp);
+            as[kg * kPitchA + 64 * h + row] = hp;
+            as[(KG + kg) * kPitchA + 64 * h + row] = lp;
         }
     };
     auto dma_b = [&](const u32x4 *bs) __attribute__((always_inline)) {  // wave w: k group w of both planes
-        const int n0 = cb.tn * T;
         asm volatile("" ::: "memory");
 #pragma unroll
-        for (int half = 0; half < 2; ++half) {
-            const int nc = min(n0 + 64 * half, g.np - 64);  // beyond the planes: results not stored
+        for (int h = 0; h < 2; ++h) {
+            const int nc = min(tn * T + 64 * h, g.np - 64);  // beyond the planes: results not stored
             const uint64_t src = static_cast<uint64_t>(cb.ks * KG + wave) * g.np + nc + lane;
-            dma16(g.bh + src, bs + wave * T + 64 * half);
-            dma16(g.bl + src, bs + (KG + wave) * T + 64 * half);
+            dma16(g.bh + src, bs + wave * T + 64 * h);
+            dma16(g.bl + src, bs + (KG + wave) * T + 64 * h);
         }
         asm volatile("" ::: "memory");
-        cb.next(nk, g.tiles_n);
+        cb.next(nk);
     };
 
     Sums acc;
-    acc.clear();
     auto fetch = [&](Frags &f, const u32x4 *as, const u32x4 *bs, int s) __attribute__((always_inline)) {
         const int kg = 2 * s + (lane >> 5), r = lane & 31;
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            f.ah[i] = __builtin_bit_cast(f16x8, as[kg * kPitchA + wm0 + 32 * i + r]);
-            f.bh[i] = __builtin_bit_cast(f16x8, bs[kg * T + wn0 + 32 * i + r]);
-        }
+        for (int i = 0; i < 2; ++i) f.ah[i] = __builtin_bit_cast(f16x8, as[kg * kPitchA + wm0 + 32 * i + r]);
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            f.al[i] = __builtin_bit_cast(f16x8, as[(KG + kg) * kPitchA + wm0 + 32 * i + r]);
-            f.bl[i] = __builtin_bit_cast(f16x8, bs[(KG + kg) * T + wn0 + 32 * i + r]);
-        }
+        for (int j = 0; j < 2; ++j) f.bh[j] = __builtin_bit_cast(f16x8, bs[kg * T + wn0 + 32 * j + r]);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) f.bl[j] = __builtin_bit_cast(f16x8, bs[(KG + kg) * T + wn0 + 32 * j + r]);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) f.al[i] = __builtin_bit_cast(f16x8, as[(KG + kg) * kPitchA + wm0 + 32 * i + r]);
     };
-    int c_tile = tile0, c_pr = p0 - tile0 * g.pairs;
-    // after a pair: at the tile's or the range's end the partial tile goes out
-    auto pair_done = [&](int j) __attribute__((always_inline)) {
-        ++c_pr;
-        const bool tile_end = c_pr == g.pairs;
-        if (tile_end || j + 1 == n) {  // uniform
-            const int first = h2_owner(static_cast<int64_t>(c_tile) * g.pairs, g.units, G);
-            // 16-byte units in accumulator order: [wave][i][jj][q / 4][lane]
-            uint32_t unit = static_cast<uint32_t>(wave) * 1024u + static_cast<uint32_t>(lane);
-            asm volatile("" : "+v"(unit));  // the addresses are formed here, not held through the loop
-            f32x4 *W = reinterpret_cast<f32x4 *>(g.ws) +
-                       (static_cast<uint64_t>(c_tile) * g.maxparts + (L - first)) * (T * T / 4) + unit;
+
+    // the partial tile of tile row t goes out, in 16-byte units in accumulator
+    // order: [wave][i][j][q / 4][lane]
+    auto flush = [&](int t) __attribute__((always_inline)) {
+        const int first = h2_owner(static_cast<int64_t>(t) * g.pairs, g.units, g.ranges);
+        uint32_t unit = static_cast<uint32_t>(wave) * (T * T / 16) + static_cast<uint32_t>(lane);
+        asm volatile("" : "+v"(unit));  // the addresses are formed here, not held through the loop
+        f32x4 *W = reinterpret_cast<f32x4 *>(g.ws) +
+                   ((static_cast<uint64_t>(t) * g.tiles_n + tn) * g.maxparts + (range - first)) * (T * T / 4) + unit;
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < 2; ++i)
 #pragma unroll
-                for (int jj = 0; jj < 2; ++jj) {
+            for (int jj = 0; jj < 2; ++jj)
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        f32x4 v;
+                for (int q = 0; q < 4; ++q) {
+                    f32x4 v;
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) v[e] = acc.hi[i][jj][4 * q + e] + acc.lo[i][jj][4 * q + e] * kLoInv;
-                        W[((2 * i + jj) * 4 + q) * 64] = v;
-                    }
+                    for (int e = 0; e < 4; ++e)
+                        v[e] = acc.hi[i][jj][4 * q + e] + acc.lo[i][jj][4 * q + e] * kLoInv;
+                    W[((2 * i + jj) * 4 + q) * 64] = v;
                 }
-            acc.clear();
-        }
-        c_pr = tile_end ? 0 : c_pr;
-        c_tile += tile_end ? 1 : 0;
     };
 
     // a slice: its A and B are in the current stage once every wave has
     // passed the barrier, which also frees the other stage (read one slice
     // ago); the next slice's A is in registers or in flight behind this
     // slice's B (and is staged before B's next transfers are issued: the
-    // compiler's wait for it takes everything in flight).  Nothing in the loop is conditional but the partial tile's
-    // way out: past the range's end the fetches repeat its last slice.
+    // compiler's wait for it takes everything in flight).  Nothing in a
+    // slice is conditional, which would split the accumulators' live ranges:
+    // past the range's end the fetches repeat its last slice.
     auto slice = [&](u32x4 *ac, u32x4 *bc, u32x4 *an, u32x4 *bn) __attribute__((always_inline)) {
         stage_barrier<kLoadsA>();
         Frags f0, f1;
@@ -322,39 +318,45 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         acc.multiply(f0);
         acc.multiply(f1);
     };
-    if (n <= 0) return;  // uniform (G <= units: does not occur)
+    if (n <= 0 || range >= g.ranges) return;  // uniform (ranges <= units and grid = ranges x tiles_n: does not occur)
     load_a();
     dma_b(b0);
     stage_a(a0);
     load_a();
-    for (int j = 0; j < n; ++j) {
-        slice(a0, b0, a1, b1);
-        slice(a1, b1, a0, b0);
-        pair_done(j);
+    int left = n, c_pr = p0 - tile0 * g.pairs;
+    for (int t = tile0; left > 0; ++t, c_pr = 0) {  // the range's tile rows
+        const int here = min(g.pairs - c_pr, left);
+        acc.clear();
+        for (int j = 0; j < here; ++j) {
+            slice(a0, b0, a1, b1);
+            slice(a1, b1, a0, b0);
+        }
+        flush(t);
+        left -= here;
     }
     // no transfer into LDS outlives the workgroup
     stage_barrier<0>();
 }
 
 // C = the sum of each tile's parts in order, times the row's (ri) or the
-// common factor, plus the k past the last whole pair of slices (fewer than 64, summed
-// in FP32 from A and B themselves).  A lane takes one 16-byte unit of the
-// parts: four consecutive rows of a column, 32 lanes 32 columns.
+// common factor, plus the k past the last whole pair of slices (fewer than 64,
+// summed in FP32 from A and B themselves).  A lane takes one 16-byte unit of
+// the parts: four consecutive rows of a column, 32 lanes 32 columns.
 template <bool TA>
-__global__ __launch_bounds__(256) void h2_reduce_kernel(H2Args g, int G, int N, const float *__restrict__ B,
+__global__ __launch_bounds__(256) void h2_reduce_kernel(H2Args g, int N, const float *__restrict__ B,
                                                         const float *__restrict__ ri, const float *__restrict__ common,
                                                         float *__restrict__ C) {
     constexpr int kUnits = T * T / 4;
     const int tile = static_cast<int>(blockIdx.x) / (kUnits / 256);
     const int unit = (static_cast<int>(blockIdx.x) % (kUnits / 256)) * 256 + threadIdx.x;
-    const int64_t ub = static_cast<int64_t>(tile) * g.pairs;
-    const int parts = h2_owner(ub + g.pairs - 1, g.units, G) - h2_owner(ub, g.units, G) + 1;
     const int tm = tile / g.tiles_n, tn = tile - tm * g.tiles_n;
+    const int64_t ub = static_cast<int64_t>(tm) * g.pairs;
+    const int parts = h2_owner(ub + g.pairs - 1, g.units, g.ranges) - h2_owner(ub, g.units, g.ranges) + 1;
+    const f32x4 *W = reinterpret_cast<const f32x4 *>(g.ws) + static_cast<uint64_t>(tile) * g.maxparts * kUnits + unit;
     const int lane = unit & 63, q = (unit >> 6) & 3, jj = (unit >> 8) & 1, i = (unit >> 9) & 1, wave = unit >> 10;
     const int gi = tm * T + (wave >> 1) * 64 + 32 * i + 8 * q + 4 * (lane >> 5);
     const int gj = tn * T + (wave & 1) * 64 + 32 * jj + (lane & 31);
     if (gi >= g.M || gj >= N) return;
-    const f32x4 *W = reinterpret_cast<const f32x4 *>(g.ws) + static_cast<uint64_t>(tile) * g.maxparts * kUnits + unit;
     f32x4 s = W[0];
 #pragma unroll 4
     for (int p = 1; p < parts; ++p) s += W[static_cast<uint64_t>(p) * kUnits];
@@ -371,28 +373,29 @@ __global__ __launch_bounds__(256) void h2_reduce_kernel(H2Args g, int G, int N, 
 }
 
 struct H2Plan {
-    int tiles, tiles_n, pairs, units, G, maxparts;
+    int tiles_m, tiles_n, pairs, units, ranges, maxparts;
     uint64_t bytes;  // partial tiles
 };
 
 // Two workgroups per CU share the slices, unless that leaves a workgroup
-// fewer than two pairs of them (128 k): the parts' traffic and the serial sum of
-// a tile's parts then cost more than the idle CUs.
+// fewer than two pairs of them (128 k): the parts' traffic and the serial sum
+// of a tile's parts then cost more than the idle CUs (512 x 1024, rank 64:
+// 488 us a round trip with two, 494 with one and 508 with four).
 H2Plan h2_plan(int M, int N, int K) {
     H2Plan p{};
+    p.tiles_m = static_cast<int>(ceil_div(M, T));
     p.tiles_n = static_cast<int>(ceil_div(N, T));
-    p.tiles = static_cast<int>(ceil_div(M, T)) * p.tiles_n;
     p.pairs = K / (2 * BK);  // the rest of K goes with the reduction
-    p.units = p.tiles * p.pairs;
-    const int most = 2 * cu_count();
-    p.G = std::max(1, std::min(most, std::max(p.tiles, p.units / 2)));
-    p.G = std::min(p.G, p.units);
+    p.units = p.tiles_m * p.pairs;
+    const int most = std::max(1, 2 * cu_count() / p.tiles_n);
+    p.ranges = std::max(1, std::min({most, std::max(p.tiles_m, p.units / 2), p.units}));
     p.maxparts = 1;
-    for (int t = 0; t < p.tiles; ++t) {
+    for (int t = 0; t < p.tiles_m; ++t) {
         const int64_t b = static_cast<int64_t>(t) * p.pairs;
-        p.maxparts = std::max(p.maxparts, h2_owner(b + p.pairs - 1, p.units, p.G) - h2_owner(b, p.units, p.G) + 1);
+        p.maxparts =
+            std::max(p.maxparts, h2_owner(b + p.pairs - 1, p.units, p.ranges) - h2_owner(b, p.units, p.ranges) + 1);
     }
-    p.bytes = static_cast<uint64_t>(p.tiles) * p.maxparts * T * T * sizeof(float);
+    p.bytes = static_cast<uint64_t>(p.tiles_m) * p.tiles_n * p.maxparts * T * T * sizeof(float);
     return p;
 }
 
@@ -438,16 +441,18 @@ void launch_h2_gemm(bool ta, int m, int n, int q, const float *A, const H2Scales
     g.tiles_n = p.tiles_n;
     g.pairs = p.pairs;
     g.units = p.units;
+    g.ranges = p.ranges;
     g.maxparts = p.maxparts;
     split_b_kernel<<<static_cast<unsigned>(ceil_div(static_cast<uint64_t>(kgroups) * np, kThreads)), kThreads, 0, stream>>>(
         B, q, np, kgroups, ta ? s.exponent : nullptr, s.emax, bh, bl);
     BSQ_HIP(hipGetLastError());
-    const dim3 grid(static_cast<unsigned>(p.G)), rgrid(static_cast<unsigned>(p.tiles * (T * T / 4 / 256)));
+    const dim3 grid(static_cast<unsigned>(p.ranges * p.tiles_n)),
+        rgrid(static_cast<unsigned>(p.tiles_m * p.tiles_n * (T * T / 4 / 256)));
     if (ta) gemm_h2_kernel<true><<<grid, kThreads, 0, stream>>>(g);
     else gemm_h2_kernel<false><<<grid, kThreads, 0, stream>>>(g);
     BSQ_HIP(hipGetLastError());
-    if (ta) h2_reduce_kernel<true><<<rgrid, 256, 0, stream>>>(g, p.G, q, B, nullptr, s.common, C);
-    else h2_reduce_kernel<false><<<rgrid, 256, 0, stream>>>(g, p.G, q, B, s.inverse, nullptr, C);
+    if (ta) h2_reduce_kernel<true><<<rgrid, 256, 0, stream>>>(g, q, B, nullptr, s.common, C);
+    else h2_reduce_kernel<false><<<rgrid, 256, 0, stream>>>(g, q, B, s.inverse, nullptr, C);
     BSQ_HIP(hipGetLastError());
 }
 
