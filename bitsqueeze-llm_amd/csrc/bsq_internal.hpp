@@ -241,11 +241,23 @@ uint64_t svd_noalloc_scratch_bytes();
 void svd_run(SvdPlan *plan, const float *A, const float *sketch, uint64_t seed, float *U, float *S, float *V,
              hipStream_t stream);
 // out = U diag(S) V^T (m x n row-major), or minuend - U diag(S) V^T when
-// `minuend` is not null (recon.hip).  `exponents` (device, m + n ints of
-// scratch) saves every workgroup the search for its rows' largest magnitudes;
-// null gives the same bits.
+// `minuend` is not null (recon.hip).
 void launch_reconstruct(const float *U, const float *S, const float *V, int m, int n, int k,
-                        const float *minuend, float *out, int *exponents, hipStream_t stream);
+                        const float *minuend, float *out, hipStream_t stream);
+// The same bits with scratch of factor_plane_bytes (16-byte aligned) and each
+// factor in FP32 (dense) or as NF4 / NF4_DQ codes with their block scales (and
+// NF4_DQ's global scale); ranks from 32.
+struct FactorSource {
+    const float *dense = nullptr;
+    const uint8_t *codes = nullptr;
+    const float *scales_f32 = nullptr;
+    const uint8_t *scales_u8 = nullptr;
+    const float *dq = nullptr;
+};
+bool reconstruct_planes_supported(int k);
+uint64_t factor_plane_bytes(int m, int n, int k);
+void launch_reconstruct_planes(const FactorSource &U, const float *S, const FactorSource &V, int m, int n, int k,
+                               const float *minuend, float *out, void *planes, hipStream_t stream);
 // Products of the range finder on the f16 matrix cores with every FP32 value
 // carried as two f16 pieces (gemm_h2.hip).  H2Scales: the exact power-of-two
 // scales of a matrix's rows, device memory (exponent, scale, inverse: one per

@@ -5,19 +5,27 @@
 //
 // Each 128 x 128 tile of the output is one workgroup.  The rows of U diag(S)
 // and of V are scaled by powers of two that bring their largest magnitude into
-// [2^14, 2^15); their values are fetched a slice of 32 k ahead, split and
-// staged into LDS planes, and the tile leaves scaled back, straight from the
-// accumulators: 32 lanes write 128 contiguous bytes of a row.  The exponents
-// of the rows come from factor_exponent_kernel where the caller has room for
-// them, else each workgroup finds those of its own 256 rows first; the values
-// are the same, so the results are too.
+// [2^14, 2^15), and the tile leaves scaled back, straight from the
+// accumulators: 32 lanes write 128 contiguous bytes of a row.  Two forms, with
+// the same pieces summed in the same order, so with the same results:
+//   recon_planes_kernel  where the caller has room for the pieces
+//                        (FactorPlanes): factor_planes_kernel splits each
+//                        factor once, from FP32 or straight from its NF4 /
+//                        NF4_DQ codes, and the tiles fetch whole 16-byte units
+//                        from the planes into LDS;
+//   recon_kernel         without scratch: each workgroup finds the exponents
+//                        of its own 256 rows, then fetches their values a
+//                        slice of 32 k ahead and splits them as it stages
+//                        them.
 //
-// Measured against the FP32 matrix cores' kernels (which also decoded packed
-// factors inline on the decompress side): 4096 x 11008, rank 128 126 -> 96 us;
-// 8192 x 4096, rank 256 167 and 171 -> 110 us; 16384 x 14336, rank 512 2237
-// and 2553 -> 1234 us.
+// Measured against the FP32 matrix cores' kernels (whose decompress side
+// decoded packed factors inline), planes included: 4096 x 11008, rank 128
+// 126 -> 81 us; 8192 x 4096, rank 256 167 and 171 -> 93 us; 16384 x 14336,
+// rank 512 2237 and 2553 -> 890 us.  Splitting while staging in every tile
+// took 96, 110 and 1182 us: twelve VALU instructions per matrix instruction.
 #include "bsq_internal.hpp"
 #include "h2_split.hpp"
+#include "scalar_codecs.hpp"
 #include "tile_map.hpp"
 
 namespace bsq {
@@ -32,7 +40,6 @@ struct ReconArgs {
     const float *U, *S, *V;
     const float *minuend;  // or null
     float *out;
-    const int *eu, *ev;    // row exponents, or null
     int m, n, k;
 };
 
@@ -53,24 +60,52 @@ __device__ __forceinline__ void load_row8(const float *row, int k, int K, float 
     }
 }
 
-// exponents of the rows of U diag(S) (e[0 .. m)) and of V (e[m .. m + n)):
-// one wave per row
-__global__ __launch_bounds__(kThreads) void factor_exponent_kernel(const float *__restrict__ U,
-                                                                   const float *__restrict__ S,
-                                                                   const float *__restrict__ V, int m, int n, int k,
-                                                                   int *__restrict__ e) {
-    const int r = blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (r >= m + n) return;  // whole waves
-    const float *row = r < m ? U + static_cast<uint64_t>(r) * k : V + static_cast<uint64_t>(r - m) * k;
-    uint32_t bits = 0;
-#pragma unroll 4
-    for (int c = lane; c < k; c += 64) {
-        const float x = r < m ? row[c] * S[c] : row[c];
-        bits = max(bits, __float_as_uint(fabsf(x)));
+// The tile's way out: exponents eu, ev (LDS) of its rows and columns undo the
+// scales; entries of a row or column with infinities are summed in FP32, since
+// an infinity has no second piece.
+template <class FU, class FV>
+__device__ __forceinline__ void store_tile(const ReconArgs &g, const Sums &acc, const int *eu, const int *ev, int m0,
+                                           int n0, int wave, int lane, FU &&u_at, FV &&v_at) {
+    const int wm0 = (wave >> 1) * 64, wn0 = (wave & 1) * 64;
+    const int g4 = 4 * (lane >> 5);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int jj = 0; jj < 2; ++jj) {
+            const int cl = wn0 + 32 * jj + (lane & 31), col = n0 + cl;
+            const int ec = ev[cl];
+            float mv[16];
+            if (g.minuend) {  // uniform
+#pragma unroll
+                for (int q = 0; q < 16; ++q) {
+                    const int row = min(m0 + wm0 + 32 * i + (q & 3) + 8 * (q >> 2) + g4, g.m - 1);
+                    mv[q] = g.minuend[static_cast<uint64_t>(row) * g.n + min(col, g.n - 1)];
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < 16; ++q) {
+                const int rl = wm0 + 32 * i + (q & 3) + 8 * (q >> 2) + g4, row = m0 + rl;
+                const int er = eu[rl];
+                const float x = __builtin_ldexpf(acc.hi[i][jj][q] + acc.lo[i][jj][q] * kLoInv,
+                                                 min(er, 127) + min(ec, 127) - 28);
+                if (row < g.m && col < g.n && er != kInfRow && ec != kInfRow)
+                    g.out[static_cast<uint64_t>(row) * g.n + col] = g.minuend ? mv[q] - x : x;
+            }
+        }
+    // the entries left out above, if any
+    bool inf = ev[wn0 + (lane & 31)] == kInfRow || ev[wn0 + 32 + (lane & 31)] == kInfRow || eu[wm0 + lane] == kInfRow;
+    if (!__any(inf)) return;
+#pragma unroll 1
+    for (int s = 0; s < 64; ++s) {
+        const int q = s & 15, rl = wm0 + 32 * (s >> 5) + (q & 3) + 8 * (q >> 2) + g4;
+        const int cl = wn0 + 32 * ((s >> 4) & 1) + (lane & 31), row = m0 + rl, col = n0 + cl;
+        if (row >= g.m || col >= g.n || (eu[rl] != kInfRow && ev[cl] != kInfRow)) continue;
+        float x = 0.0f;
+#pragma unroll 1
+        for (int t = 0; t < g.k; ++t) x = fmaf(u_at(row, t) * g.S[t], v_at(col, t), x);
+        const uint64_t e = static_cast<uint64_t>(row) * g.n + col;
+        g.out[e] = g.minuend ? g.minuend[e] - x : x;
     }
-    for (int off = 32; off >= 1; off >>= 1)
-        bits = max(bits, static_cast<uint32_t>(__shfl_xor(static_cast<int>(bits), off)));
-    if (lane == 0) e[r] = factor_exponent(bits);
 }
 
 // (two waves per SIMD asked for: 128 accumulators and two slices' fragments)
@@ -104,25 +139,20 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
             load_row8(g.S, k, g.k, s8);
         }
     };
-    if (g.eu) {  // uniform
-        if (tid < T) eu[tid] = g.eu[min(m0 + tid, g.m - 1)];
-        else ev[tid - T] = g.ev[min(n0 + tid - T, g.n - 1)];
-    } else {
-        uint32_t bits[4] = {0, 0, 0, 0};
-        for (int j = 0; j < nk; ++j) {
-            load(j);
+    uint32_t bits[4] = {0, 0, 0, 0};
+    for (int j = 0; j < nk; ++j) {
+        load(j);
 #pragma unroll
-            for (int h = 0; h < 4; ++h)
+        for (int h = 0; h < 4; ++h)
 #pragma unroll
-                for (int i = 0; i < 8; ++i)
-                    bits[h] = max(bits[h], __float_as_uint(fabsf(h < 2 ? v[h][i] * s8[i] : v[h][i])));
-        }
+            for (int i = 0; i < 8; ++i)
+                bits[h] = max(bits[h], __float_as_uint(fabsf(h < 2 ? v[h][i] * s8[i] : v[h][i])));
+    }
 #pragma unroll
-        for (int h = 0; h < 4; ++h) {
-            for (int off = 1; off <= 2; off <<= 1)
-                bits[h] = max(bits[h], static_cast<uint32_t>(__shfl_xor(static_cast<int>(bits[h]), off)));
-            if (kg == 0) (h < 2 ? eu : ev)[64 * (h & 1) + r] = factor_exponent(bits[h]);
-        }
+    for (int h = 0; h < 4; ++h) {
+        for (int off = 1; off <= 2; off <<= 1)
+            bits[h] = max(bits[h], static_cast<uint32_t>(__shfl_xor(static_cast<int>(bits[h]), off)));
+        if (kg == 0) (h < 2 ? eu : ev)[64 * (h & 1) + r] = factor_exponent(bits[h]);
     }
     load(0);
     __syncthreads();
@@ -180,39 +210,226 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         if (j + 1 < nk) slice(a1, b1, a0, b0, j + 1);
     }
 
-    const int g4 = 4 * (lane >> 5);
+    auto at = [&](const float *f) {
+        return [=](int row, int t) { return f[static_cast<uint64_t>(row) * g.k + t]; };
+    };
+    store_tile(g, acc, eu, ev, m0, n0, wave, lane, at(g.U), at(g.V));
+}
+
+// ---------------------------------------------------------------------------
+// A factor as pieces: planes [k / 8][padded rows][8] of f16, h then l, zero
+// past k and past the rows, and the exponent of each row.
+struct PlaneSource {
+    const float *dense;       // FP32 values, or null
+    const uint8_t *codes;     // NF4 / NF4_DQ nibbles, element 2 j in the high one
+    const float *scales_f32;  // NF4 block scales
+    const uint8_t *scales_u8; // NF4_DQ block scale codes
+    const float *dq;          // NF4_DQ global scale
+    const float *S;           // values times S[k], or null
+    u32x4 *h, *l;
+    int *e;
+    int rows, padded;
+};
+
+// scale of block b, as the decoder computes it (quantization_cuda.cu:300-305,
+// 322-332)
+__device__ __forceinline__ float block_scale(const PlaneSource &p, uint64_t b, float dq) {
+    const float s = p.scales_u8 ? dq * e4m3_decode(p.scales_u8[b]) : p.scales_f32[b];
+    return (s == 0.0f || !__builtin_isfinite(s)) ? 1.0f : s;
+}
+
+// One workgroup per 16 rows (the first `groups_u` of U, the others of V); the
+// sixteen groups of sixteen lanes share a row's groups of eight k.  Exponents
+// first, then the pieces, the values of up to 512 k held in registers between
+// (64 rows a workgroup, each value read twice, took 22 us instead of 8 at
+// 8192 x 4096, rank 256: too few loads in flight).  Quantised factors are
+// decoded here, element by element as the decoder does.
+constexpr int kPlaneRows = 16;
+__global__ __launch_bounds__(kThreads) void factor_planes_kernel(PlaneSource u, PlaneSource v, int groups_u, int k,
+                                                                 int kgroups) {
+    constexpr float Lc[16] = BSQ_NF4_LEVELS;
+    __shared__ float levels[16];
+    __shared__ uint32_t wbits[kThreads / 64][kPlaneRows];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const bool is_u = static_cast<int>(blockIdx.x) < groups_u;  // uniform
+    const PlaneSource p = is_u ? u : v;
+    const int row = (static_cast<int>(blockIdx.x) - (is_u ? 0 : groups_u)) * kPlaneRows + (lane & 15);
+    const int kg0 = 4 * wave + (lane >> 4);
+    if (tid < 16) levels[tid] = Lc[tid];
+    __syncthreads();
+    const uint64_t base = static_cast<uint64_t>(min(row, p.rows - 1)) * k;
+    float dq = 1.0f;
+    if (p.scales_u8) {
+        dq = *p.dq;
+        if (dq == 0.0f || !__builtin_isfinite(dq)) dq = 1.0f;
+    }
+    const bool quick = k % 8 == 0;  // a group of eight in one 64-element block, its codes in one aligned word
+    auto values = [&](int kg, float (&x)[8]) {
+        const int k0 = 8 * kg;
+        const uint64_t e0 = base + k0;
+        if (p.dense) {
+            load_row8(p.dense + base, k0, k, x);
+        } else if (quick && k0 < k) {
+            const uint32_t w = *reinterpret_cast<const uint32_t *>(p.codes + e0 / 2);
+            const float s = block_scale(p, e0 / kQuantBlock, dq);
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+            for (int i = 0; i < 8; ++i) x[i] = s * levels[(w >> (8 * (i / 2) + (i % 2 ? 0 : 4))) & 15u];
+        } else {
 #pragma unroll
-        for (int jj = 0; jj < 2; ++jj) {
-            const int cl = wn0 + 32 * jj + (lane & 31), col = n0 + cl;
-            const int ec = ev[cl];
-            float mv[16];
-            if (g.minuend) {  // uniform
-#pragma unroll
-                for (int q = 0; q < 16; ++q) {
-                    const int row = min(m0 + wm0 + 32 * i + (q & 3) + 8 * (q >> 2) + g4, g.m - 1);
-                    mv[q] = g.minuend[static_cast<uint64_t>(row) * g.n + min(col, g.n - 1)];
+            for (int i = 0; i < 8; ++i) {
+                const uint64_t e = e0 + i;
+                x[i] = 0.0f;
+                if (k0 + i < k) {
+                    const uint32_t byte = p.codes[e >> 1];
+                    x[i] = block_scale(p, e / kQuantBlock, dq) * levels[(e & 1) ? (byte & 15u) : (byte >> 4)];
                 }
-            }
-#pragma unroll
-            for (int q = 0; q < 16; ++q) {
-                const int rl = wm0 + 32 * i + (q & 3) + 8 * (q >> 2) + g4, row = m0 + rl;
-                const int er = eu[rl];
-                float x = __builtin_ldexpf(acc.hi[i][jj][q] + acc.lo[i][jj][q] * kLoInv,
-                                           min(er, 127) + min(ec, 127) - 28);
-                if (er == kInfRow || ec == kInfRow) {
-                    // an infinity has no second piece: these entries in FP32
-                    const float *u = g.U + static_cast<uint64_t>(min(row, g.m - 1)) * g.k;
-                    const float *w = g.V + static_cast<uint64_t>(min(col, g.n - 1)) * g.k;
-                    x = 0.0f;
-#pragma unroll 1
-                    for (int t = 0; t < g.k; ++t) x = fmaf(u[t] * g.S[t], w[t], x);
-                }
-                if (row < g.m && col < g.n)
-                    g.out[static_cast<uint64_t>(row) * g.n + col] = g.minuend ? mv[q] - x : x;
             }
         }
+        if (p.S) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                if (k0 + i < k) x[i] *= p.S[k0 + i];
+        }
+    };
+    constexpr int kKeep = 4, kStep = 16;  // groups of eight k held per lane, and their distance
+    float x[kKeep][8];
+    uint32_t bits = 0;
+    auto largest = [&](const float (&y)[8]) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) bits = max(bits, __float_as_uint(fabsf(y[i])));
+    };
+#pragma unroll
+    for (int n = 0; n < kKeep; ++n)
+        if (kg0 + kStep * n < kgroups) values(kg0 + kStep * n, x[n]);
+#pragma unroll
+    for (int n = 0; n < kKeep; ++n)
+        if (kg0 + kStep * n < kgroups) largest(x[n]);
+    for (int kg = kg0 + kStep * kKeep; kg < kgroups; kg += kStep) {
+        float y[8];
+        values(kg, y);
+        largest(y);
+    }
+    for (int off = 16; off <= 32; off <<= 1)
+        bits = max(bits, static_cast<uint32_t>(__shfl_xor(static_cast<int>(bits), off)));
+    if (lane < kPlaneRows) wbits[wave][lane] = bits;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < kThreads / 64; ++w) bits = max(bits, wbits[w][lane & 15]);
+    const int e = factor_exponent(bits);
+    if (tid < kPlaneRows && row < p.rows) p.e[row] = e;
+    const float sc = row < p.rows ? factor_scale(e) : 0.0f;
+    auto put = [&](int kg, const float (&y)[8]) {
+        u32x4 h, l;
+        split8(y, [&](int) { return sc; }, h, l);
+        const uint64_t unit = static_cast<uint64_t>(kg) * p.padded + row;
+        p.h[unit] = h;
+        p.l[unit] = l;
+    };
+#pragma unroll
+    for (int n = 0; n < kKeep; ++n)
+        if (kg0 + kStep * n < kgroups) put(kg0 + kStep * n, x[n]);
+    for (int kg = kg0 + kStep * kKeep; kg < kgroups; kg += kStep) {
+        float y[8];
+        values(kg, y);
+        put(kg, y);
+    }
+}
+
+// element (row, t) of a factor, without S
+__device__ float factor_value(const PlaneSource &p, int row, int t, int k) {
+    constexpr float Lc[16] = BSQ_NF4_LEVELS;
+    const uint64_t e = static_cast<uint64_t>(row) * k + t;
+    if (p.dense) return p.dense[e];
+    float dq = 1.0f;
+    if (p.scales_u8) {
+        dq = *p.dq;
+        if (dq == 0.0f || !__builtin_isfinite(dq)) dq = 1.0f;
+    }
+    const uint32_t byte = p.codes[e >> 1];
+    return block_scale(p, e / kQuantBlock, dq) * Lc[(e & 1) ? (byte & 15u) : (byte >> 4)];
+}
+
+struct PlaneArgs {
+    PlaneSource u, v;
+    int slices;  // 16-deep slices (a multiple of two)
+};
+
+typedef __attribute__((address_space(3))) void lds_void_t;
+typedef __attribute__((address_space(1))) void glb_void_t;
+
+// Slices of 16 k through a ring of four LDS stages, three in flight: wave 0
+// fetches U's h units, wave 1 its l units, waves 2 and 3 V's.  One LDS object
+// per stage, so that no wait is inserted for another stage's transfers.
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void recon_planes_kernel(
+    ReconArgs g, PlaneArgs pl) {
+    constexpr int kStage = 4 * 2 * T;  // units: planes uh, ul, vh, vl of two k groups x 128 rows
+    constexpr int kDma = 4;            // transfers of a wave per slice
+    __shared__ __attribute__((aligned(1024))) u32x4 st0[kStage], st1[kStage], st2[kStage], st3[kStage];
+    __shared__ int eu[T], ev[T];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int wm0 = (wave >> 1) * 64, wn0 = (wave & 1) * 64;
+    int tile_m, tile_n, z;
+    xcd_tile(static_cast<int>(ceil_div(g.m, T)), static_cast<int>(ceil_div(g.n, T)), 1, tile_m, tile_n, z);
+    const int m0 = tile_m * T, n0 = tile_n * T;
+    if (tid < T) eu[tid] = pl.u.e[min(m0 + tid, g.m - 1)];
+    else ev[tid - T] = pl.v.e[min(n0 + tid - T, g.n - 1)];  // both visible after the loop's barriers
+
+    // this wave's plane, from its first row; rows past the planes repeat the
+    // last 64 (their results are not stored)
+    const u32x4 *src = wave == 0 ? pl.u.h : (wave == 1 ? pl.u.l : (wave == 2 ? pl.v.h : pl.v.l));
+    const int rows = wave < 2 ? pl.u.padded : pl.v.padded, r0 = wave < 2 ? m0 : n0;
+    const int c0 = min(r0, rows - 64) + lane, c1 = min(r0 + 64, rows - 64) + lane;
+    auto issue = [&](const u32x4 *st, int j) __attribute__((always_inline)) {
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int kg = 0; kg < 2; ++kg) {
+            const u32x4 *p = src + static_cast<uint64_t>(2 * j + kg) * rows;
+            const u32x4 *dst = st + (2 * wave + kg) * T;
+            __builtin_amdgcn_global_load_lds((glb_void_t *)(p + c0), (lds_void_t *)(reinterpret_cast<size_t>(dst)), 16,
+                                             0, 0);
+            __builtin_amdgcn_global_load_lds((glb_void_t *)(p + c1),
+                                             (lds_void_t *)(reinterpret_cast<size_t>(dst + 64)), 16, 0, 0);
+        }
+        asm volatile("" ::: "memory");
+    };
+    Sums acc;
+    acc.clear();
+    // slice j from `cur`; slice j + 3 goes to `nxt`, read in slice j - 1.
+    // Past the last slice the transfers repeat it, so the count of those in
+    // flight is the same in every slice.
+    auto slice = [&](const u32x4 *cur, const u32x4 *nxt, int j) __attribute__((always_inline)) {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(0x070 | (2 * kDma));  // lgkmcnt(0), vmcnt(8): slice j has landed
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        issue(nxt, min(j + 3, pl.slices - 1));
+        Frags f;
+        const int o = (lane >> 5) * T + (lane & 31);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            f.ah[i] = __builtin_bit_cast(f16x8, cur[o + wm0 + 32 * i]);
+            f.bh[i] = __builtin_bit_cast(f16x8, cur[4 * T + o + wn0 + 32 * i]);
+            f.al[i] = __builtin_bit_cast(f16x8, cur[2 * T + o + wm0 + 32 * i]);
+            f.bl[i] = __builtin_bit_cast(f16x8, cur[6 * T + o + wn0 + 32 * i]);
+        }
+        acc.multiply(f);
+    };
+    issue(st0, 0);
+    issue(st1, min(1, pl.slices - 1));
+    issue(st2, min(2, pl.slices - 1));
+    for (int j = 0; j < pl.slices; j += 4) {
+        slice(st0, st3, j);
+        slice(st1, st0, j + 1);
+        if (j + 2 < pl.slices) {  // uniform; the slices come in pairs
+            slice(st2, st1, j + 2);
+            slice(st3, st2, j + 3);
+        }
+    }
+    // no transfer into LDS outlives the workgroup
+    __builtin_amdgcn_s_waitcnt(0x070);
+    store_tile(
+        g, acc, eu, ev, m0, n0, wave, lane, [&](int row, int t) { return factor_value(pl.u, row, t, g.k); },
+        [&](int row, int t) { return factor_value(pl.v, row, t, g.k); });
 }
 
 // Ranks below 32: FP32 sums over k.  There the two pieces' own rounding (7e-8
@@ -264,21 +481,48 @@ __global__ __launch_bounds__(kThreads) void recon_low_rank_kernel(ReconArgs g) {
 
 }  // namespace
 
+namespace {
+int padded_rows(int rows) { return static_cast<int>(ceil_div(rows, 64) * 64); }
+int plane_groups(int k) { return static_cast<int>(ceil_div(k, BK) * KG); }
+}  // namespace
+
+uint64_t factor_plane_bytes(int m, int n, int k) {
+    if (k < BK) return 0;
+    return 2ull * 16 * plane_groups(k) * (static_cast<uint64_t>(padded_rows(m)) + padded_rows(n)) +
+           sizeof(int) * (static_cast<uint64_t>(m) + n);
+}
+
 void launch_reconstruct(const float *U, const float *S, const float *V, int m, int n, int k, const float *minuend,
-                        float *out, int *exponents, hipStream_t stream) {
+                        float *out, hipStream_t stream) {
     BSQ_REQUIRE(m > 0 && n > 0 && k > 0 && U && S && V && out, "reconstruct: bad arguments");
-    ReconArgs g{U, S, V, minuend, out, exponents, exponents ? exponents + m : nullptr, m, n, k};
-    if (k < BK) {
+    const ReconArgs g{U, S, V, minuend, out, m, n, k};
+    if (k < BK)
         recon_low_rank_kernel<<<static_cast<unsigned>(ceil_div(m, 64) * ceil_div(n, 64)), kThreads, 0, stream>>>(g);
-        BSQ_HIP(hipGetLastError());
-        return;
-    }
-    if (exponents) {
-        factor_exponent_kernel<<<static_cast<unsigned>(ceil_div(static_cast<uint64_t>(m) + n, kThreads / 64)), kThreads,
-                                 0, stream>>>(U, S, V, m, n, k, exponents);
-        BSQ_HIP(hipGetLastError());
-    }
-    recon_kernel<<<static_cast<unsigned>(ceil_div(m, T) * ceil_div(n, T)), kThreads, 0, stream>>>(g);
+    else
+        recon_kernel<<<static_cast<unsigned>(ceil_div(m, T) * ceil_div(n, T)), kThreads, 0, stream>>>(g);
+    BSQ_HIP(hipGetLastError());
+}
+
+bool reconstruct_planes_supported(int k) { return k >= BK; }
+
+void launch_reconstruct_planes(const FactorSource &U, const float *S, const FactorSource &V, int m, int n, int k,
+                               const float *minuend, float *out, void *planes, hipStream_t stream) {
+    BSQ_REQUIRE(m > 0 && n > 0 && reconstruct_planes_supported(k) && S && out && planes, "reconstruct: bad arguments");
+    for (const FactorSource *f : {&U, &V})
+        BSQ_REQUIRE(f->dense || (f->codes && (f->scales_f32 || (f->scales_u8 && f->dq))), "reconstruct: missing factor");
+    const int kgroups = plane_groups(k), up = padded_rows(m), vp = padded_rows(n);
+    auto *uh = static_cast<u32x4 *>(planes);
+    u32x4 *ul = uh + static_cast<uint64_t>(kgroups) * up, *vh = ul + static_cast<uint64_t>(kgroups) * up,
+          *vl = vh + static_cast<uint64_t>(kgroups) * vp;
+    int *eu = reinterpret_cast<int *>(vl + static_cast<uint64_t>(kgroups) * vp), *ev = eu + m;
+    const PlaneSource pu{U.dense, U.codes, U.scales_f32, U.scales_u8, U.dq, S, uh, ul, eu, m, up};
+    const PlaneSource pv{V.dense, V.codes, V.scales_f32, V.scales_u8, V.dq, nullptr, vh, vl, ev, n, vp};
+    factor_planes_kernel<<<static_cast<unsigned>((up + vp) / kPlaneRows), kThreads, 0, stream>>>(
+        pu, pv, up / kPlaneRows, k, kgroups);
+    BSQ_HIP(hipGetLastError());
+    const ReconArgs g{nullptr, S, nullptr, minuend, out, m, n, k};
+    const PlaneArgs pl{pu, pv, kgroups / 2};
+    recon_planes_kernel<<<static_cast<unsigned>(ceil_div(m, T) * ceil_div(n, T)), kThreads, 0, stream>>>(g, pl);
     BSQ_HIP(hipGetLastError());
 }
 

@@ -299,7 +299,7 @@ struct Runtime {
     TopkBuf topk[2];
     Meta *meta = nullptr;
     SvdPlan *svd = nullptr;
-    int *recon_exp = nullptr;       // row exponents of the factors (launch_reconstruct)
+    uint8_t *planes = nullptr;      // the factors' pieces (launch_reconstruct_planes)
     const float *sketch = nullptr;  // injected Gaussian sketch (test hook)
     // decompress-side staging for quantised sections (shared, like the reference's buffers)
     float *q_scales_f32 = nullptr;
@@ -324,7 +324,7 @@ struct Runtime {
         dev_free(d_err);
         dev_free(d_row_gmax);
         dev_free(meta);
-        dev_free(recon_exp);
+        dev_free(planes);
         dev_free(q_scales_f32);
         dev_free(q_scales_u8);
         dev_free(q_codes);
@@ -520,7 +520,7 @@ void compress_init(Runtime &rt, uint16_t rows, uint16_t cols, float r_out, float
         rt.reconstruct_initialized = true;
         if (rt.topk[TK_ERROR].capacity > 0) {
             rt.d_err = dev_alloc<float>(N);
-            rt.recon_exp = dev_alloc<int>(static_cast<uint64_t>(rows) + cols);
+            rt.planes = dev_alloc<uint8_t>(factor_plane_bytes(rows, cols, q));
         }
     } else {
         Section &sc = rt.sec[SEC_DIRECT];
@@ -561,7 +561,7 @@ void decompress_init(Runtime &rt, uint16_t rows, uint16_t cols, float r_out, flo
             rt.sec[i].dense = dev_alloc<float>(counts[i]);
             rt.sec[i].own_dense = true;
         }
-        rt.recon_exp = dev_alloc<int>(static_cast<uint64_t>(rows) + cols);
+        rt.planes = dev_alloc<uint8_t>(factor_plane_bytes(rows, cols, svd_ranks));
         rt.reconstruct_initialized = true;
     }
     if (uses_quant(rt)) {
@@ -665,9 +665,8 @@ void compress_device(Runtime &rt, const float *d_in, bsq_device_packed_t *out, c
         Section &U = rt.sec[SEC_U], &S = rt.sec[SEC_S], &V = rt.sec[SEC_V];
         svd_run(rt.svd, residual, rt.sketch, 1241ULL, U.dense, S.dense, V.dense, st);
         mark(2);
-        // quantise U, S, V, each dequantised in place afterwards
-        // (append_quantized_section with d_dequantized_dst = the source,
-        // src/bitsqz_llm.cu:1078-1139)
+        // quantise U, S, V (append_quantized_section, src/bitsqz_llm.cu:
+        // 1078-1139); only the error set needs their decoded values
         for (int i = 0; i < 3; ++i) {
             Section &sc = rt.sec[i];
             if (sc.method == kMethodNone) continue;
@@ -675,9 +674,12 @@ void compress_device(Runtime &rt, const float *d_in, bsq_device_packed_t *out, c
                                 sc.codes, &rt.meta->gmax, st);
         }
         mark(3);
+        // the reconstruction decodes U and V as it splits them; S, and all
+        // three at ranks outside that form, are decoded in place
+        const bool planes = reconstruct_planes_supported(rt.q);
         for (int i = 0; i < 3; ++i) {
             Section &sc = rt.sec[i];
-            if (sc.method == kMethodNone) continue;
+            if (sc.method == kMethodNone || te.capacity == 0 || (planes && i != SEC_S)) continue;
             launch_quant_decode(sc.count, sc.method, sc.scales_f32, sc.scales_u8, &rt.meta->dq[i], sc.codes,
                                 sc.dense, st);
         }
@@ -685,7 +687,16 @@ void compress_device(Runtime &rt, const float *d_in, bsq_device_packed_t *out, c
         if (te.capacity > 0) {
             // reconstruct + subtract fused (src/bitsqz_llm.cu:1141-1163)
             timed_launch(kTimeReconstruct, st, [&] {
-                launch_reconstruct(U.dense, S.dense, V.dense, rows, cols, rt.q, residual, rt.d_err, rt.recon_exp, st);
+                auto factor = [&](int i) {
+                    const Section &sc = rt.sec[i];
+                    if (sc.method == kMethodNone) return FactorSource{sc.dense};
+                    return FactorSource{nullptr, sc.codes, sc.scales_f32, sc.scales_u8, &rt.meta->dq[i]};
+                };
+                if (planes)
+                    launch_reconstruct_planes(factor(SEC_U), S.dense, factor(SEC_V), rows, cols, rt.q, residual,
+                                              rt.d_err, rt.planes, st);
+                else
+                    launch_reconstruct(U.dense, S.dense, V.dense, rows, cols, rt.q, residual, rt.d_err, st);
             });
             mark(5);
             TopkArgs a;
@@ -855,12 +866,11 @@ void decompress_device(Runtime &rt, const bsq_device_packed_t &P, const bool has
     const uint32_t ke = has_error ? P.topk_k[1] : 0, ko = has_outlier ? P.topk_k[0] : 0;
     if (H.flags & kFlagSvd) {
         const int q = static_cast<uint16_t>(H.effective_rank);
+        const bool planes = reconstruct_planes_supported(q);  // U and V are decoded as they are split
         const float *dense[3];
         for (int i = 0; i < 3; ++i) {
-            if (P.d_dense[i]) {
-                dense[i] = P.d_dense[i];
-                continue;
-            }
+            dense[i] = P.d_dense[i];
+            if (dense[i] || (planes && i != SEC_S)) continue;
             Section &sc = rt.sec[i];  // decompress runtime's dense U / S / V
             const int method = (i == SEC_S) ? H.svd_s_format : H.svd_uv_format;
             launch_quant_decode(P.count[i], method, P.d_scales_f32[i], P.d_scales_u8[i], P.d_dq_scale[i],
@@ -868,7 +878,18 @@ void decompress_device(Runtime &rt, const bsq_device_packed_t &P, const bool has
             dense[i] = sc.dense;
         }
         timed_launch(kTimeReconstruct, st, [&] {
-            launch_reconstruct(dense[0], dense[1], dense[2], rows, cols, q, nullptr, d_dst, rt.recon_exp, st);
+            if (!planes) {
+                launch_reconstruct(dense[SEC_U], dense[SEC_S], dense[SEC_V], rows, cols, q, nullptr, d_dst, st);
+                return;
+            }
+            auto factor = [&](int i) {
+                if (dense[i]) return FactorSource{dense[i]};
+                const bool dq = H.svd_uv_format == kMethodNF4DQ;
+                return FactorSource{nullptr, P.d_codes[i], dq ? nullptr : P.d_scales_f32[i],
+                                    dq ? P.d_scales_u8[i] : nullptr, P.d_dq_scale[i]};
+            };
+            launch_reconstruct_planes(factor(SEC_U), dense[SEC_S], factor(SEC_V), rows, cols, q, nullptr, d_dst,
+                                      rt.planes, st);
         });
     } else {
         const uint64_t N = static_cast<uint64_t>(rows) * cols;
@@ -1754,7 +1775,7 @@ int bsq_reconstruct_lowrank(const float *d_U, const float *d_S, const float *d_V
                             void *stream) {
     return guarded([&] {
         BSQ_REQUIRE(m > 0 && n > 0 && k > 0, "reconstruct: bad shape");
-        launch_reconstruct(d_U, d_S, d_V, m, n, k, nullptr, d_out, nullptr, static_cast<hipStream_t>(stream));
+        launch_reconstruct(d_U, d_S, d_V, m, n, k, nullptr, d_out, static_cast<hipStream_t>(stream));
     });
 }
 
