@@ -50,39 +50,72 @@ __device__ __forceinline__ uint32_t nf4_code_scan_inline(const float *L, float v
 
 // Nearest NF4 code with the reference's tie rule: for |v| < 2 the scan's
 // answer is the number of exact decision thresholds at or below v, found
-// here with one table lookup and one comparison.  [-1, 1] is
-// cut into 256 bins of width 1/128; bin b holds code_lo = #{T_i <= -1 + b/128}
-// and the threshold lying inside the bin, if any (no bin holds two: the
-// closest thresholds are 0.085 apart).  Every threshold is at least 2.3e-4
-// from a bin edge, while the bin index floor((v + 1) * 128) computed in FP32
-// is off by one only for v within 1.2e-7 of an edge, where the count is the
-// same on both sides; v in [1, 2) and (-2, -1] clamp to the end bins (codes
-// 15 and 0).  |v| >= 2 and non-finite v take the scan.  Exhaustively
-// checked against the scan over all 2^32 floats by the GPU test suite.
+// here with one table lookup and one comparison.  [-1, 2) is cut into 384
+// bins of width 1/128; bin b holds code_lo = #{T_i <= -1 + b/128} and the
+// threshold lying inside the bin, if any (no bin holds two: the closest
+// thresholds are 0.085 apart).  Every threshold is at least 2.3e-4 from a bin
+// edge, while the bin index floor((v + 1) * 128), computed in FP32 with one
+// rounding or two, is off by one only for v within 1.2e-7 of an edge, where
+// the count is the same on both sides; v in (-2, -1] takes bin 0.  |v| >= 2
+// and non-finite v take the scan.  Exhaustively checked against the scan over
+// all 2^32 floats by the GPU test suite.
+constexpr int kNf4Bins = 384;
 struct Nf4Table {
-    uint2 ent[256];  // (bits of the threshold inside bin b, code_lo): one 8-byte read
+    uint2 ent[kNf4Bins];  // (bits of the threshold inside bin b, code_lo): one 8-byte read
 };
 
-__device__ __forceinline__ void nf4_table_build(Nf4Table &t) {
-    constexpr float T[15] = BSQ_NF4_THRESHOLDS;
-    for (int b = threadIdx.x; b < 256; b += blockDim.x) {
-        const float e0 = -1.0f + static_cast<float>(b) / 128.0f, e1 = -1.0f + static_cast<float>(b + 1) / 128.0f;
-        uint32_t lo = 0;
-        float thr = __builtin_inff();
-#pragma unroll
-        for (int i = 0; i < 15; ++i) {
-            lo += (T[i] <= e0) ? 1u : 0u;
-            if (T[i] > e0 && T[i] < e1) thr = T[i];
+// the table's entries, computed by the compiler: copying them costs a
+// workgroup two loads a lane, forming them some 90 instructions
+struct Nf4TableValues {
+    float thr[kNf4Bins];
+    uint32_t lo[kNf4Bins];
+    constexpr Nf4TableValues() : thr(), lo() {
+        constexpr float T[15] = BSQ_NF4_THRESHOLDS;
+        for (int b = 0; b < kNf4Bins; ++b) {
+            const float e0 = -1.0f + static_cast<float>(b) / 128.0f, e1 = -1.0f + static_cast<float>(b + 1) / 128.0f;
+            thr[b] = __builtin_inff();
+            for (int i = 0; i < 15; ++i) {
+                lo[b] += T[i] <= e0 ? 1u : 0u;
+                if (T[i] > e0 && T[i] < e1) thr[b] = T[i];
+            }
         }
-        t.ent[b] = uint2{__float_as_uint(thr), lo};
     }
+};
+__device__ const Nf4TableValues kNf4TableValues{};
+
+__device__ __forceinline__ void nf4_table_build(Nf4Table &t) {
+    for (int b = threadIdx.x; b < kNf4Bins; b += blockDim.x)
+        t.ent[b] = uint2{__float_as_uint(kNf4TableValues.thr[b]), kNf4TableValues.lo[b]};
 }
 
 // the table path alone: |v| < 2
 __device__ __forceinline__ uint32_t nf4_code_small(const Nf4Table &t, float v) {
-    const int b = min(max(static_cast<int>((v + 1.0f) * 128.0f), 0), 255);
+    const int b = min(max(static_cast<int>((v + 1.0f) * 128.0f), 0), kNf4Bins - 1);
     const uint2 e = t.ent[b];
     return e.y + ((v >= __uint_as_float(e.x)) ? 1u : 0u);
+}
+
+// bin of x inv, given inv128 = 128 inv: one FMA and one conversion (which
+// takes negative values to 0).  |x inv128| < 256, so the bin is below 384.
+__device__ __forceinline__ uint32_t nf4_bin(float x, float inv128) {
+    const float t = __builtin_fmaf(x, inv128, 128.0f);
+    uint32_t b;
+    asm("v_cvt_u32_f32 %0, %1" : "=v"(b) : "v"(t));
+    return b;
+}
+
+// Largest magnitude of v[0 .. N), and whether any of them is NaN; infinities
+// give infinity.  (N even: two values an instruction.)
+template <int N>
+__device__ __forceinline__ float magnitude_max(const float (&v)[N], bool &nan) {
+    float m = 0.0f;
+    nan = false;
+#pragma unroll
+    for (int i = 0; i < N; i += 2) {
+        asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(m) : "v"(v[i]), "v"(v[i + 1]));
+        nan = nan || __builtin_isunordered(v[i], v[i + 1]);
+    }
+    return m;
 }
 
 // The same bins with the two candidate levels of each: (bits of the

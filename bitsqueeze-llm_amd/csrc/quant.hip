@@ -76,13 +76,8 @@ __device__ __forceinline__ void store_codes(uint8_t *__restrict__ codes, uint64_
 
 // Encode side: one thread owns chunks of 8 consecutive elements (two 16-byte
 // loads, one 4-byte store of packed nibbles), so a 64-element block is an
-// aligned group of 8 lanes and the per-block scale work is shared by 8 lanes.
-// Each thread takes kUnroll chunks per loop iteration, their loads issued
-// together before any is used (one chunk per iteration left these kernels
-// latency-bound); the encoder also issues the next iteration's loads before
-// encoding the current one (two chunks per iteration measured best with
-// that: four take 144 VGPRs, three waves per SIMD).
-constexpr int kUnroll = 2;
+// aligned group of 8 lanes.
+constexpr int kUnroll = 2;  // chunks per lane and iteration of the global-scale pass
 
 // Pass 1 of NF4_DQ: max over blocks of the block scale (absmax, or 1 for an
 // all-zero block), as float bits (all values >= 0): each workgroup writes
@@ -109,9 +104,13 @@ __global__ __launch_bounds__(kThreads) void dq_gmax_kernel(const float *__restri
 #pragma unroll
         for (int u = 0; u < kUnroll; ++u) {
             const uint64_t chunk = base + u * stride + threadIdx.x;
-            float m = 0.0f;
+            bool nan;
+            float m = magnitude_max(v[u], nan);
+            if (__any(nan || !(m < __builtin_inff()))) {  // uniform
+                m = 0.0f;
 #pragma unroll
-            for (int i = 0; i < 8; ++i) m = fmaxf(m, fabsf(sanitize(v[u][i])));
+                for (int i = 0; i < 8; ++i) m = fmaxf(m, fabsf(sanitize(v[u][i])));
+            }
             m = group8_max(m);
             if (chunk / 8 < nblocks) local = fmaxf(local, m > 0.0f ? m : 1.0f);
         }
@@ -129,6 +128,12 @@ __global__ __launch_bounds__(kThreads) void dq_gmax_kernel(const float *__restri
     }
 }
 
+// Value of lane u of each quad, in all four lanes.
+template <int U>
+__device__ __forceinline__ float quad_get(float v) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), U * 0x55, 0xF, 0xF, false));
+}
+
 // SEL: sel[chunk] flags the chunk's elements that a separation took out
 // (bit i = element 8 chunk + i); they are encoded as 0, as the residual
 // holds them.
@@ -136,28 +141,43 @@ __global__ __launch_bounds__(kThreads) void dq_gmax_kernel(const float *__restri
 // from the largest of row_gmax[0 .. gmax_rows) (a separation's per-row
 // maxima; gmax_rows a multiple of 4 up to kInlineGmaxRows), which every
 // workgroup reduces itself.
-template <bool DQ, bool SEL>
+//
+// A workgroup takes tiles of 256 U chunks, U of them a lane; the loads of a
+// tile go out together and other waves' tiles cover them (few registers, so
+// up to eight waves a SIMD).  In memory terms the pass is 4.5 bytes a value;
+// it was bound by its vector instructions (about 25 a value), so:
+//   - the usual chunk, all finite, takes one instruction for two values to
+//     find the magnitude and one to rule out NaN; chunks with a non-finite
+//     value, at the section's end or scaled past the table take the
+//     element-by-element form;
+//   - a code is a multiplication, one FMA and one conversion to its bin, the
+//     table's read, a comparison and an add, and one instruction to pack it;
+//   - the scale's chain (NF4_DQ: a division, the E4M3 encode and decode, then
+//     1 / scale) is the same in a block's 8 lanes and costs the same for one
+//     lane as for 64, so with U = 4 lane l of a quad runs it for chunk l of
+//     the four and the quad hands the results around.
+template <bool DQ, bool SEL, int U>
 __global__ __launch_bounds__(kThreads) void quant_encode_kernel(
     const float *__restrict__ x, uint64_t n, bool vec_ok, float *__restrict__ scales_f32,
     uint8_t *__restrict__ scales_u8, const uint32_t *__restrict__ gmax, const float *__restrict__ row_gmax,
     uint32_t gmax_rows, float *__restrict__ dq_out, uint8_t *__restrict__ codes,
     uint32_t *__restrict__ flags_reset, const uint8_t *__restrict__ sel) {
+    static_assert(U == 1 || U == 4, "one scale chain a lane");
     __shared__ Nf4Table tab;
     __shared__ float gwmax[kThreads / 64];
     // the pipeline's flags word, cleared here when no earlier kernel of the
     // compress does it (saves a fill launch); nothing reads it before this
     // kernel ends
     if (flags_reset && blockIdx.x == 0 && threadIdx.x == 0) *flags_reset = 0u;
-    const uint64_t nchunks = ceil_div(n, 8);
-    const uint64_t stride = static_cast<uint64_t>(gridDim.x) * kThreads;
+    const uint64_t nchunks = ceil_div(n, 8), ntiles = ceil_div(nchunks, kThreads * U);
+    const uint32_t tid = threadIdx.x;
     float dq = 1.0f;  // NF4_DQ: set below, before the first encode
-    // chunks of one iteration: loaded one iteration ahead (two register
-    // sets), so the loads of iteration i + 1 are in flight while iteration i
-    // is encoded
-    auto load_it = [&](uint64_t base, float (&v)[kUnroll][8], uint32_t (&sb)[kUnroll]) {
+    float v[U][8];
+    uint32_t sb[U] = {};
+    auto load_tile = [&](uint64_t tile) {
 #pragma unroll
-        for (int u = 0; u < kUnroll; ++u) {
-            const uint64_t chunk = base + u * stride + threadIdx.x;
+        for (int u = 0; u < U; ++u) {
+            const uint64_t chunk = tile * (kThreads * U) + u * kThreads + tid;
             if (chunk < nchunks) {
                 load8(x, n, chunk, vec_ok, v[u]);
                 if constexpr (SEL) sb[u] = sel[chunk];
@@ -168,81 +188,24 @@ __global__ __launch_bounds__(kThreads) void quant_encode_kernel(
             }
         }
     };
-    auto encode_it = [&](uint64_t base, float (&v)[kUnroll][8], const uint32_t (&sb)[kUnroll]) {
-#pragma unroll
-        for (int u = 0; u < kUnroll; ++u) {
-            const uint64_t chunk = base + u * stride + threadIdx.x;
-            const bool valid = chunk < nchunks;
-            // sanitised values (a selected entry reads as 0) and this lane's
-            // largest |value|
-            if constexpr (SEL) {
-#pragma unroll
-                for (int i = 0; i < 8; ++i) v[u][i] = ((sb[u] >> i) & 1u) ? 0.0f : v[u][i];
-            }
-            float lm = 0.0f;
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                v[u][i] = sanitize(v[u][i]);
-                lm = fmaxf(lm, fabsf(v[u][i]));
-            }
-            const float m = group8_max(lm);
-            const float absmax = (m > 0.0f) ? m : 1.0f;
-            float scale;
-            uint32_t scode = 0;
-            if constexpr (DQ) {
-                scode = e4m3_encode(absmax / dq);
-                scale = dq * e4m3_decode(scode);
-                if (scale == 0.0f || !__builtin_isfinite(scale)) scale = 1.0f;
-            } else {
-                scale = absmax;
-            }
-            const float inv = 1.0f / scale;
-            if (valid && (threadIdx.x & 7) == 0) {
-                if constexpr (DQ) scales_u8[chunk / 8] = static_cast<uint8_t>(scode);
-                else scales_f32[chunk / 8] = scale;
-            }
-            if (valid) {
-                // |v inv| < 2 (the table) unless a block scale fell far below
-                // the block's absmax (an NF4_DQ scale code of 0 replaced by 1).
-                // Rounding is monotone, so the chunk's largest |v inv| is
-                // exactly fl(lm inv): one test per chunk; the per-element end
-                // test and the scan only for a chunk that needs them.
-                uint32_t c[8];
-                const uint64_t e0 = chunk * 8;
-                if (lm * inv < 2.0f && e0 + 8 <= n) {
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) c[i] = nf4_code_small(tab, v[u][i] * inv);
-                } else {
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) c[i] = (e0 + i < n) ? nf4_code(tab, v[u][i] * inv) : 0u;  // odd tail: low nibble 0
-                }
-                store_codes(codes, n, chunk, vec_ok, c);
-            }
-        }
-    };
-    const uint64_t step = static_cast<uint64_t>(kUnroll) * stride;
-    float va[kUnroll][8], vb[kUnroll][8];
-    uint32_t sa[kUnroll] = {}, sbb[kUnroll] = {};
-    uint64_t base = static_cast<uint64_t>(blockIdx.x) * kThreads;
-    // the first two iterations' loads go out before the code table is built
-    // and the global scale read (neither feeds an address), so the table
-    // work and the barrier overlap the first memory round trip
-    if (base < nchunks) load_it(base, va, sa);
-    if (base + step < nchunks) load_it(base + step, vb, sbb);
+    // the first tile's loads go out before the code table is copied and the
+    // global scale read (neither feeds an address)
+    uint64_t tile = blockIdx.x;
+    if (tile < ntiles) load_tile(tile);
     if constexpr (DQ) {
         if (row_gmax) {  // uniform: wave maxima of the per-row maxima to LDS
             constexpr int kGq = kInlineGmaxRows / (4 * kThreads);
             float gm = 0.0f;
 #pragma unroll
             for (int j = 0; j < kGq; ++j) {
-                const uint32_t i4 = threadIdx.x + kThreads * j;
+                const uint32_t i4 = tid + kThreads * j;
                 if (4 * i4 < gmax_rows) {
                     const f32x4 g = reinterpret_cast<const f32x4 *>(row_gmax)[i4];
                     gm = fmaxf(gm, fmaxf(fmaxf(g.x, g.y), fmaxf(g.z, g.w)));
                 }
             }
             for (int off = 32; off >= 1; off >>= 1) gm = fmaxf(gm, __shfl_xor(gm, off));
-            if ((threadIdx.x & 63) == 0) gwmax[threadIdx.x >> 6] = gm;
+            if ((tid & 63) == 0) gwmax[tid >> 6] = gm;
         }
     }
     nf4_table_build(tab);
@@ -253,14 +216,115 @@ __global__ __launch_bounds__(kThreads) void quant_encode_kernel(
             row_gmax ? __float_as_uint(fmaxf(fmaxf(gwmax[0], gwmax[1]), fmaxf(gwmax[2], gwmax[3]))) : *gmax;
         const float raw = dq_raw_from_gmax(gbits);
         dq = dq_effective(raw);
-        if (blockIdx.x == 0 && threadIdx.x == 0) *dq_out = raw;
+        if (blockIdx.x == 0 && tid == 0) *dq_out = raw;
     }
-    for (bool first = true; base < nchunks; base += 2 * step, first = false) {  // uniform
-        if (!first && base + step < nchunks) load_it(base + step, vb, sbb);
-        encode_it(base, va, sa);
-        if (base + step >= nchunks) break;
-        if (base + 2 * step < nchunks) load_it(base + 2 * step, va, sa);
-        encode_it(base + step, vb, sbb);
+    while (tile < ntiles) {  // uniform
+        const uint64_t chunk0 = tile * (kThreads * U) + tid;
+        float lm[U], bm[U];
+        bool odd = false;  // a chunk of this wave needs the element-by-element form
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if constexpr (SEL) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i)  // bit i set: 0
+                    v[u][i] = __uint_as_float(__float_as_uint(v[u][i]) &
+                                              (static_cast<uint32_t>(static_cast<int32_t>(~sb[u] << (31 - i)) >> 31)));
+            }
+            bool nan;
+            lm[u] = magnitude_max(v[u], nan);
+            if (__any(nan || !(lm[u] < __builtin_inff()))) {  // uniform
+                lm[u] = 0.0f;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    v[u][i] = sanitize(v[u][i]);
+                    lm[u] = fmaxf(lm[u], fabsf(v[u][i]));
+                }
+            }
+            bm[u] = group8_max(lm[u]);
+        }
+        // the scale chain: lane l of a quad for chunk l % U
+        float m = bm[0];
+        if constexpr (U == 4) {
+            const float lo = (tid & 1) ? bm[1] : bm[0], hi = (tid & 1) ? bm[3] : bm[2];
+            m = (tid & 2) ? hi : lo;
+        }
+        const float absmax = (m > 0.0f) ? m : 1.0f;
+        float scale;
+        uint32_t scode = 0;
+        if constexpr (DQ) {
+            scode = e4m3_encode(absmax / dq);
+            scale = dq * e4m3_decode(scode);
+            if (scale == 0.0f || !__builtin_isfinite(scale)) scale = 1.0f;
+        } else {
+            scale = absmax;
+        }
+        const float inv_own = 1.0f / scale;
+        const uint64_t own = chunk0 + (U == 4 ? (tid & 3) * kThreads : 0);
+        if ((tid & 7) < U && (own & ~7ull) < nchunks) {
+            if constexpr (DQ) scales_u8[own / 8] = static_cast<uint8_t>(scode);
+            else scales_f32[own / 8] = scale;
+        }
+        float inv[U];
+        if constexpr (U == 4) {
+            inv[0] = quad_get<0>(inv_own);
+            inv[1] = quad_get<1>(inv_own);
+            inv[2] = quad_get<2>(inv_own);
+            inv[3] = quad_get<3>(inv_own);
+        } else {
+            inv[0] = inv_own;
+        }
+        // |v inv| < 2 (the table) unless a block scale fell far below the
+        // block's absmax (an NF4_DQ scale code of 0 replaced by 1) or 1 / scale
+        // overflows.  Rounding is monotone and 128 a power of two, so the
+        // chunk's largest |v 128 inv| is exactly fl(lm 128 inv).
+#pragma unroll
+        for (int u = 0; u < U; ++u) odd = odd || !(lm[u] * (inv[u] * 128.0f) < 256.0f);
+        odd = __any(odd || 8 * (chunk0 + (U - 1) * kThreads) + 8 > n);  // uniform
+        if (!odd) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const float inv128 = inv[u] * 128.0f;
+                uint32_t word = 0;
+#pragma unroll
+                for (int j = 3; j >= 0; --j)  // byte j = code(2 j) << 4 | code(2 j + 1)
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        const float y = v[u][2 * j + h];
+                        const uint2 e = tab.ent[nf4_bin(y, inv128)];
+                        word = (word << 4) | (e.y + ((y * inv[u] >= __uint_as_float(e.x)) ? 1u : 0u));
+                    }
+                uint8_t *out = codes + 4 * (chunk0 + u * kThreads);
+                if (vec_ok) {  // uniform
+                    *reinterpret_cast<uint32_t *>(out) = word;
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) out[j] = static_cast<uint8_t>(word >> (8 * j));
+                }
+            }
+        } else {
+#pragma unroll 1
+            for (int u = 0; u < U; ++u) {
+                float w[8], iv = inv[0];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) w[i] = v[0][i];
+#pragma unroll
+                for (int t = 1; t < U; ++t)  // (registers are not indexed at run time)
+                    if (u == t) {
+                        iv = inv[t];
+#pragma unroll
+                        for (int i = 0; i < 8; ++i) w[i] = v[t][i];
+                    }
+                const uint64_t chunk = chunk0 + u * kThreads;
+                if (chunk >= nchunks) continue;
+                uint32_t c[8];
+                const uint64_t e0 = chunk * 8;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) c[i] = (e0 + i < n) ? nf4_code(tab, w[i] * iv) : 0u;  // odd tail: low nibble 0
+                store_codes(codes, n, chunk, vec_ok, c);
+            }
+        }
+        tile += gridDim.x;
+        if (tile < ntiles) load_tile(tile);
     }
 }
 
@@ -520,21 +584,16 @@ void launch_rows_gmax(const float *row_gmax, uint32_t rows, uint32_t *gmax, hipS
 }
 
 namespace {
-// one chunk per thread until the grid reaches its cap (small sections keep
-// every CU busy); the unrolled loop then covers the rest.  The cap is the
-// variant's occupancy in workgroups per CU (five or six: 80 to 90
-// registers), so every workgroup is resident from the start: eight per CU
-// ran as a round of five and a round of three (supplement encode 54.5 ->
-// 50.5 us).
-template <bool DQ, bool SEL>
+// Workgroups of the encode: as many as are resident at once, or one a tile.
+template <bool DQ, bool SEL, int U>
 unsigned encode_grid(uint64_t n) {
     static const unsigned per_cu = [] {
         int b = 0;
         BSQ_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &b, reinterpret_cast<const void *>(quant_encode_kernel<DQ, SEL>), kThreads, 0));
+            &b, reinterpret_cast<const void *>(quant_encode_kernel<DQ, SEL, U>), kThreads, 0));
         return static_cast<unsigned>(b > 0 ? b : 1);
     }();
-    return grid_for(ceil_div(n, 8), per_cu);
+    return grid_for(ceil_div(n, 8 * U), per_cu);
 }
 
 template <bool DQ>
@@ -542,19 +601,26 @@ void encode_pass(const float *x, uint64_t n, float *scales_f32, uint8_t *scales_
                  float *dq_out, uint8_t *codes, uint32_t *flags_reset, const uint8_t *sel, hipStream_t stream,
                  const float *row_gmax = nullptr, uint32_t gmax_rows = 0) {
     const bool vec_ok = aligned16(x) && ((reinterpret_cast<uintptr_t>(codes) & 3u) == 0);
-    const unsigned grid = sel ? encode_grid<DQ, true>(n) : encode_grid<DQ, false>(n);
     BSQ_REQUIRE(!sel || n % kQuantBlock == 0, "quant encode: a selection bitmap needs whole blocks");
     BSQ_REQUIRE(!row_gmax || (DQ && gmax_rows > 0 && gmax_rows % 4 == 0 && gmax_rows <= kInlineGmaxRows &&
                               aligned16(row_gmax)),
                 "quant encode: per-row maxima outside the in-kernel reduction's limits");
-    if (sel)
-        quant_encode_kernel<DQ, true><<<grid, kThreads, 0, stream>>>(x, n, vec_ok, scales_f32, scales_u8, gmax,
-                                                                     row_gmax, gmax_rows, dq_out, codes,
-                                                                     flags_reset, sel);
-    else
-        quant_encode_kernel<DQ, false><<<grid, kThreads, 0, stream>>>(x, n, vec_ok, scales_f32, scales_u8, gmax,
-                                                                      row_gmax, gmax_rows, dq_out, codes,
-                                                                      flags_reset, nullptr);
+    auto go = [&](auto kern, unsigned grid) {
+        kern<<<grid, kThreads, 0, stream>>>(x, n, vec_ok, scales_f32, scales_u8, gmax, row_gmax, gmax_rows, dq_out,
+                                            codes, flags_reset, sel);
+    };
+    // one chunk a lane keeps the most workgroups and loads in flight (2048 x
+    // 4096 NF4 8.6 us, with four chunks 9.9; 1000 x 5003 6.4 and 9.3); four
+    // share the scale chain and win once every resident workgroup has several
+    // tiles (4096 x 11008 NF4 43 and 41, NF4_DQ's two passes 78 and 76; 4096 x
+    // 4096 even)
+    if (n >= 1ull << 25) {
+        if (sel) go(quant_encode_kernel<DQ, true, 4>, encode_grid<DQ, true, 4>(n));
+        else go(quant_encode_kernel<DQ, false, 4>, encode_grid<DQ, false, 4>(n));
+    } else {
+        if (sel) go(quant_encode_kernel<DQ, true, 1>, encode_grid<DQ, true, 1>(n));
+        else go(quant_encode_kernel<DQ, false, 1>, encode_grid<DQ, false, 1>(n));
+    }
     BSQ_HIP(hipGetLastError());
 }
 }  // namespace
