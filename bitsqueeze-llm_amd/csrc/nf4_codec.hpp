@@ -50,29 +50,30 @@ __device__ __forceinline__ uint32_t nf4_code_scan_inline(const float *L, float v
 
 // Nearest NF4 code with the reference's tie rule: for |v| < 2 the scan's
 // answer is the number of exact decision thresholds at or below v, found
-// here with one table lookup and one comparison.  [-1, 2) is cut into 384
-// bins of width 1/128; bin b holds code_lo = #{T_i <= -1 + b/128} and the
+// here with one table lookup and one comparison.  [-1, 2) is cut into 48
+// bins of width 1/16; bin b holds code_lo = #{T_i <= -1 + b/16} and the
 // threshold lying inside the bin, if any (no bin holds two: the closest
-// thresholds are 0.085 apart).  Every threshold is at least 2.3e-4 from a bin
-// edge, while the bin index floor((v + 1) * 128), computed in FP32 with one
+// thresholds are 0.081 apart).  Every threshold is at least 1.6e-3 from a bin
+// edge, while the bin index floor((v + 1) * 16), computed in FP32 with one
 // rounding or two, is off by one only for v within 1.2e-7 of an edge, where
 // the count is the same on both sides; v in (-2, -1] takes bin 0.  |v| >= 2
 // and non-finite v take the scan.  Exhaustively checked against the scan over
-// all 2^32 floats by the GPU test suite.
-constexpr int kNf4Bins = 384;
+// all 2^32 floats by the GPU test suite.  So few bins span one and a half
+// rounds of the LDS banks: 384 bins of 1/128 took 93 us against 85 in the
+// fused encode and top-k pass of 4096 x 11008 (with its other changes).
+constexpr int kNf4PerUnit = 16, kNf4Bins = 3 * kNf4PerUnit;
 struct Nf4Table {
     uint2 ent[kNf4Bins];  // (bits of the threshold inside bin b, code_lo): one 8-byte read
 };
 
-// the table's entries, computed by the compiler: copying them costs a
-// workgroup two loads a lane, forming them some 90 instructions
+// the table's entries, computed by the compiler
 struct Nf4TableValues {
     float thr[kNf4Bins];
     uint32_t lo[kNf4Bins];
     constexpr Nf4TableValues() : thr(), lo() {
         constexpr float T[15] = BSQ_NF4_THRESHOLDS;
         for (int b = 0; b < kNf4Bins; ++b) {
-            const float e0 = -1.0f + static_cast<float>(b) / 128.0f, e1 = -1.0f + static_cast<float>(b + 1) / 128.0f;
+            const float e0 = -1.0f + static_cast<float>(b) / kNf4PerUnit, e1 = -1.0f + static_cast<float>(b + 1) / kNf4PerUnit;
             thr[b] = __builtin_inff();
             for (int i = 0; i < 15; ++i) {
                 lo[b] += T[i] <= e0 ? 1u : 0u;
@@ -90,15 +91,16 @@ __device__ __forceinline__ void nf4_table_build(Nf4Table &t) {
 
 // the table path alone: |v| < 2
 __device__ __forceinline__ uint32_t nf4_code_small(const Nf4Table &t, float v) {
-    const int b = min(max(static_cast<int>((v + 1.0f) * 128.0f), 0), kNf4Bins - 1);
+    const int b = min(max(static_cast<int>((v + 1.0f) * static_cast<float>(kNf4PerUnit)), 0), kNf4Bins - 1);
     const uint2 e = t.ent[b];
     return e.y + ((v >= __uint_as_float(e.x)) ? 1u : 0u);
 }
 
-// bin of x inv, given inv128 = 128 inv: one FMA and one conversion (which
-// takes negative values to 0).  |x inv128| < 256, so the bin is below 384.
-__device__ __forceinline__ uint32_t nf4_bin(float x, float inv128) {
-    const float t = __builtin_fmaf(x, inv128, 128.0f);
+// bin of x inv, given inv_bins = kNf4PerUnit inv: one FMA and one conversion
+// (which takes negative values and NaN to 0).  |x inv| < 2, so the bin is
+// below kNf4Bins.
+__device__ __forceinline__ uint32_t nf4_bin(float x, float inv_bins) {
+    const float t = __builtin_fmaf(x, inv_bins, static_cast<float>(kNf4PerUnit));
     uint32_t b;
     asm("v_cvt_u32_f32 %0, %1" : "=v"(b) : "v"(t));
     return b;
@@ -116,41 +118,6 @@ __device__ __forceinline__ float magnitude_max(const float (&v)[N], bool &nan) {
         nan = nan || __builtin_isunordered(v[i], v[i + 1]);
     }
     return m;
-}
-
-// The same bins with the two candidate levels of each: (bits of the
-// threshold, code_lo, L[code_lo], L[code_lo + 1]) in one 16-byte entry, so an
-// encoder that also needs the level of the code (the fused encode + error
-// pass) reads both with one lookup.
-struct Nf4LevelTable {
-    uint4 ent[256];
-};
-
-__device__ __forceinline__ void nf4_level_table_build(Nf4LevelTable &t) {
-    constexpr float T[15] = BSQ_NF4_THRESHOLDS;
-    constexpr float L[16] = BSQ_NF4_LEVELS;
-    for (int b = threadIdx.x; b < 256; b += blockDim.x) {
-        const float e0 = -1.0f + static_cast<float>(b) / 128.0f, e1 = -1.0f + static_cast<float>(b + 1) / 128.0f;
-        uint32_t lo = 0;
-        float thr = __builtin_inff();
-#pragma unroll
-        for (int i = 0; i < 15; ++i) {
-            lo += (T[i] <= e0) ? 1u : 0u;
-            if (T[i] > e0 && T[i] < e1) thr = T[i];
-        }
-        // a bin whose code_lo is 15 holds no threshold (thr = inf): its upper
-        // level is never taken
-        t.ent[b] = uint4{__float_as_uint(thr), lo, __float_as_uint(L[lo]), __float_as_uint(L[lo < 15 ? lo + 1 : 15])};
-    }
-}
-
-// code of v (|v| < 2, as nf4_code_small) and its level L[code]
-__device__ __forceinline__ uint32_t nf4_code_level_small(const Nf4LevelTable &t, float v, float &level) {
-    const int b = min(max(static_cast<int>((v + 1.0f) * 128.0f), 0), 255);
-    const uint4 e = t.ent[b];
-    const bool up = v >= __uint_as_float(e.x);
-    level = __uint_as_float(up ? e.w : e.z);
-    return e.y + (up ? 1u : 0u);
 }
 
 __device__ __forceinline__ uint32_t nf4_code(const Nf4Table &t, float v) {

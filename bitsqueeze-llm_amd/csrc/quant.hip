@@ -275,22 +275,22 @@ __global__ __launch_bounds__(kThreads) void quant_encode_kernel(
         }
         // |v inv| < 2 (the table) unless a block scale fell far below the
         // block's absmax (an NF4_DQ scale code of 0 replaced by 1) or 1 / scale
-        // overflows.  Rounding is monotone and 128 a power of two, so the
-        // chunk's largest |v 128 inv| is exactly fl(lm 128 inv).
+        // overflows.  Rounding is monotone and the bins' number a power of
+        // two, so the chunk's largest |v inv_bins| is exactly fl(lm inv_bins).
 #pragma unroll
-        for (int u = 0; u < U; ++u) odd = odd || !(lm[u] * (inv[u] * 128.0f) < 256.0f);
+        for (int u = 0; u < U; ++u) odd = odd || !(lm[u] * (inv[u] * kNf4PerUnit) < 2.0f * kNf4PerUnit);
         odd = __any(odd || 8 * (chunk0 + (U - 1) * kThreads) + 8 > n);  // uniform
         if (!odd) {
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                const float inv128 = inv[u] * 128.0f;
+                const float inv_bins = inv[u] * kNf4PerUnit;
                 uint32_t word = 0;
 #pragma unroll
                 for (int j = 3; j >= 0; --j)  // byte j = code(2 j) << 4 | code(2 j + 1)
 #pragma unroll
                     for (int h = 0; h < 2; ++h) {
                         const float y = v[u][2 * j + h];
-                        const uint2 e = tab.ent[nf4_bin(y, inv128)];
+                        const uint2 e = tab.ent[nf4_bin(y, inv_bins)];
                         word = (word << 4) | (e.y + ((y * inv[u] >= __uint_as_float(e.x)) ? 1u : 0u));
                     }
                 uint8_t *out = codes + 4 * (chunk0 + u * kThreads);
@@ -612,9 +612,9 @@ void encode_pass(const float *x, uint64_t n, float *scales_f32, uint8_t *scales_
     // one chunk a lane keeps the most workgroups and loads in flight (2048 x
     // 4096 NF4 8.6 us, with four chunks 9.9; 1000 x 5003 6.4 and 9.3); four
     // share the scale chain and win once every resident workgroup has several
-    // tiles (4096 x 11008 NF4 43 and 41, NF4_DQ's two passes 78 and 76; 4096 x
-    // 4096 even)
-    if (n >= 1ull << 25) {
+    // tiles (4096 x 11008 NF4 43 and 41), with NF4_DQ's longer chain earlier
+    // (4096 x 4096 after a separation 19.1 and 17.5)
+    if (n >= (DQ ? 1ull << 24 : 1ull << 25)) {
         if (sel) go(quant_encode_kernel<DQ, true, 4>, encode_grid<DQ, true, 4>(n));
         else go(quant_encode_kernel<DQ, false, 4>, encode_grid<DQ, false, 4>(n));
     } else {

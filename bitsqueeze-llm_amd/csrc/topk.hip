@@ -519,7 +519,7 @@ template <TopkSource SRC, int NV4>
 __global__ __launch_bounds__(kThreads) void topk_reg_kernel(TopkArgs a) {
     constexpr bool ENC = SRC == TopkSource::EncodeNF4 || SRC == TopkSource::EncodeNF4DQ;
     __shared__ Shared sh;
-    __shared__ Nf4LevelTable etab;  // encode sources: the NF4 code and level table (unused, and dropped, otherwise)
+    __shared__ Nf4Table etab;  // encode sources: the NF4 code table (unused, and dropped, otherwise)
     __shared__ __attribute__((aligned(16))) unsigned long long bk[kFastCap];
     __shared__ float bv[kFastCap];
     // the row's selected columns, one bit each (separation: residual, bitmap)
@@ -550,7 +550,7 @@ __global__ __launch_bounds__(kThreads) void topk_reg_kernel(TopkArgs a) {
         if (dq == 0.0f || !__builtin_isfinite(dq)) dq = 1.0f;
     }
     if constexpr (ENC) {
-        nf4_level_table_build(etab);
+        nf4_table_build(etab);
         if constexpr (SRC == TopkSource::EncodeNF4DQ) {
             if (!a.enc_row_gmax) {  // uniform
                 const float raw = dq_raw_from_gmax(*a.enc_gmax);
@@ -652,11 +652,17 @@ __global__ __launch_bounds__(kThreads) void topk_reg_kernel(TopkArgs a) {
         // DPP row), one lane per block runs the chain once for all of them,
         // and the quads read their block's scale back.
         const int g = static_cast<int>((tid >> 4) & 3u), wv = static_cast<int>(tid >> 6), wl = static_cast<int>(tid & 63u);
+        bool clean = true;  // every value of the wave's row part is finite (padding aside)
 #pragma unroll
         for (int m = 0; m < NV4; ++m) {
-            float lm = 0.0f;
+            bool nan;
+            float lm = magnitude_max(v[m], nan);  // padding: 0
+            if (__any((nan && tid + kThreads * m < q4) || !(lm < __builtin_inff()))) {  // uniform
+                clean = false;
+                lm = 0.0f;
 #pragma unroll
-            for (int u = 0; u < 4; ++u) lm = fmaxf(lm, fabsf(sanitize(v[m][u])));
+                for (int u = 0; u < 4; ++u) lm = fmaxf(lm, fabsf(sanitize(v[m][u])));
+            }
             const float bm = row16_max(lm);
             if ((tid & 15u) == 0) enc_bmax[wv][4 * m + g] = bm;
         }
@@ -675,10 +681,11 @@ __global__ __launch_bounds__(kThreads) void topk_reg_kernel(TopkArgs a) {
             }
             const float inv = 1.0f / scale;
             // |w| < 2 in the whole block unless its scale fell far below its
-            // absmax (an NF4_DQ scale code of 0 replaced by 1); rounding is
-            // monotone, so the block's largest |w| is exactly fl(bm * inv).
-            // The flag rides in the sign of inv (> 0).
-            enc_scl[wv][wl] = float2{scale, (bm * inv < 2.0f) ? inv : -inv};
+            // absmax (an NF4_DQ scale code of 0 replaced by 1) or 1 / scale
+            // overflows; rounding is monotone, so the block's largest
+            // |w| kNf4PerUnit is exactly the product tested.  The flag rides
+            // in the sign of inv (> 0).
+            enc_scl[wv][wl] = float2{scale, (bm * (inv * kNf4PerUnit) < 2.0f * kNf4PerUnit) ? inv : -inv};
             const uint32_t c4b = static_cast<uint32_t>(64 * wv + 16 * (wl & 3) + kThreads * (wl >> 2));
             if (c4b < q4) {
                 const uint64_t blk = (row0 + 4ull * c4b) >> 6;
@@ -694,25 +701,31 @@ __global__ __launch_bounds__(kThreads) void topk_reg_kernel(TopkArgs a) {
             const float2 sc = enc_scl[wv][4 * m + g];
             const float scale = sc.x, inv = fabsf(sc.y);
             const bool small = sc.y > 0.0f;  // the table for the whole block
-            uint32_t packed = 0;
+            uint32_t packed = 0;             // element 2j in the high nibble: bytes (c0 c1) (c2 c3)
+            if (clean && __all(small)) {     // uniform; padding stays NaN by itself
+                const float inv_bins = inv * kNf4PerUnit;
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const float w = sanitize(v[m][u]) * inv;
-                float lv;
-                uint32_t c;
-                if (small) {
-                    c = nf4_code_level_small(etab, w, lv);
-                } else {
-                    c = (fabsf(w) < 2.0f) ? nf4_code_level_small(etab, w, lv) : nf4_code_scan_inline(sh.L, w);
-                    lv = sh.L[c];
+                for (int h = 0; h < 4; ++h) {
+                    const int u = h ^ 2;
+                    const uint2 e = etab.ent[nf4_bin(v[m][u], inv_bins)];
+                    const uint32_t c = e.y + ((v[m][u] * inv >= __uint_as_float(e.x)) ? 1u : 0u);
+                    packed = (packed << 4) | c;
+                    v[m][u] = v[m][u] - scale * sh.L[c];
+                    // the error is formed here: left to the compiler, the
+                    // subtraction sinks to the first later use and the levels
+                    // and scales of every quad stay live until then
+                    asm volatile("" : "+v"(v[m][u]));
                 }
-                // element 2j in the high nibble: bytes (c0 c1) (c2 c3)
-                packed |= c << (8 * (u >> 1) + 4 * (1 - (u & 1)));
-                v[m][u] = inside ? v[m][u] - scale * lv : __builtin_nanf("");
-                // the error is formed here: left to the compiler, the
-                // subtraction sinks to the first later use and the levels
-                // and scales of every quad stay live until then
-                asm volatile("" : "+v"(v[m][u]));
+            } else {
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const float w = sanitize(v[m][u]) * inv;
+                    const uint32_t c =
+                        (small || fabsf(w) < 2.0f) ? nf4_code_small(etab, w) : nf4_code_scan_inline(sh.L, w);
+                    packed |= c << (8 * (u >> 1) + 4 * (1 - (u & 1)));
+                    v[m][u] = inside ? v[m][u] - scale * sh.L[c] : __builtin_nanf("");
+                    asm volatile("" : "+v"(v[m][u]));
+                }
             }
             if (inside) {
                 const uint64_t e = row0 + 4ull * c4;
@@ -737,16 +750,17 @@ __global__ __launch_bounds__(kThreads) void topk_reg_kernel(TopkArgs a) {
             for (int u = 0; u < 4; ++u) asm volatile("" : "+v"(v[m][u]));
         return t;
     };
-    // the lane's largest |v| (a compare-select skips NaN, which ranks lowest;
-    // all-NaN lanes keep -1), i.e. its largest 32-bit order key
+    // the lane's largest |v| (NaN, which ranks lowest, is skipped; all-NaN
+    // lanes keep -1), i.e. its largest 32-bit order key.  (A signalling NaN in
+    // the input may hide the lane's other values: its filter threshold is then
+    // lower than it could be, which the exact ranking does not mind.)
     float mx = -1.0f;
 #pragma unroll
     for (int m = 0; m < NV4; ++m)
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const float f = fabsf(v[m][u]);
-            mx = f > mx ? f : mx;
-        }
+        for (int u = 0; u < 4; u += 2)
+            asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(mx) : "v"(v[m][u]), "v"(v[m][u + 1]));
+    mx = mx >= 0.0f ? mx : -1.0f;
     const uint32_t key32 = mx >= 0.0f ? __float_as_uint(mx) + 1u : 0u;
     const bool nonzero = mx > FLT_EPSILON;  // false for NaN-only and padding lanes
     if (a.flags && __syncthreads_or(nonzero ? 1 : 0)) {
