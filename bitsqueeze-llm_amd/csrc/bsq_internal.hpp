@@ -272,12 +272,28 @@ struct H2Scales {
 bool h2_supported(int K);
 uint64_t h2_workspace_bytes(int M, int N, int K);
 uint64_t h2_plane_units(int K, int N);
-void launch_h2_scales(const float *A, int m, int n, const H2Scales &s, hipStream_t stream);
+// The split operand B of a product: two planes [k / 8][np][8] of f16 pieces,
+// `rows` (K rounded up to 64) of k, zero past K.  In the group of eight that K
+// ends in, entry k is at place (k + rot) % 8: the product with A reads the
+// last eight values of A's rows there.  With `exponent`, row k also carries 2^(exponent[k] - *emax).
+// Columns past B's may hold anything: they only reach results not stored.
+struct H2Planes {
+    uint16_t *hi = nullptr, *lo = nullptr;
+    const int *exponent = nullptr, *emax = nullptr;
+    int np = 0, K = 0, rows = 0, rot = 0;
+};
+H2Planes h2_planes(bool ta, int K, int q, const H2Scales &s, uint16_t *planes);
+// The scales of A's rows; in the same launch `fill` N(0, 1) draws into R.
+void launch_h2_scales(const float *A, int m, int n, const H2Scales &s, float *R, uint64_t fill, uint64_t seed,
+                      hipStream_t stream);
+// B's planes; with new_rows > 0 (the rows of A), first s.emax and s.common from
+// the exponents that launch_h2_scales wrote.
+void launch_h2_split(const float *B, int q, const H2Planes &b, const H2Scales &s, int new_rows, hipStream_t stream);
 // C = A B (ta false: m x n times n x q) or A^T B (n x m times m x q), A
-// row-major m x n, B and C row-major with q columns; B's entries below 32 in
-// magnitude.
-void launch_h2_gemm(bool ta, int m, int n, int q, const float *A, const H2Scales &s, const float *B, uint16_t *planes,
-                    float *C, float *workspace, uint64_t workspace_bytes, hipStream_t stream);
+// row-major m x n, C row-major with q columns, `b` the planes of B, whose
+// entries are below 32 in magnitude.
+void launch_h2_gemm(bool ta, int m, int n, int q, const float *A, const H2Scales &s, const H2Planes &b, float *C,
+                    float *workspace, uint64_t workspace_bytes, hipStream_t stream);
 
 // N(0, 1) draws: Philox4x32-10 counter-based generator + Box-Muller.
 void launch_gaussian_fill(float *out, uint64_t n, uint64_t seed, hipStream_t stream);

@@ -27,6 +27,7 @@
 // modules/svd_lowrank_cuda/src/svd_lowrank_cuda.cu:250-282); any basis of the
 // same column space serves the range finder.
 #include "bsq_internal.hpp"
+#include "h2_split.hpp"
 
 #include <algorithm>
 #include <type_traits>
@@ -697,6 +698,9 @@ __global__ __launch_bounds__(kTrinvThreads) void trinv_kernel(const double *__re
 // operand), and even and odd steps accumulate in two chains.  Replaces the
 // triangular inverse and the X * L^{-T} product (two launches, one of them
 // latency-bound on k / 16 CUs).
+// With planes.rows > 0, Q goes out as the f16 pieces that the next product
+// with the big matrix takes (zero from row M to planes.rows): a lane holds
+// four consecutive rows of a column, half of a 16-byte unit of eight.
 // pv[i] = src[8 i] for i < 2 J (J <= 7): constant slot indices on every path,
 // so that the slots stay in registers.
 template <int PV>
@@ -724,7 +728,8 @@ constexpr int kSolveRows = 32;
 template <int NB>
 __global__ __launch_bounds__(256, 2) void chol_solve_kernel(const float *__restrict__ X, int M, int k,
                                                             const double *__restrict__ Lin,
-                                                            const double *__restrict__ LIin, float *__restrict__ Q) {
+                                                            const double *__restrict__ LIin, float *__restrict__ Q,
+                                                            H2Planes planes) {
     typedef float f32x4v __attribute__((ext_vector_type(4)));
     constexpr int KP = NB * 32, QP = KP + 4, LP = (NB > 1 ? (NB - 1) * 32 : 32) + 4, TP = 36;
     constexpr int PV = NB > 1 ? 2 * (NB - 1) : 1;  // 16-byte panel loads per thread, widest panel
@@ -754,6 +759,15 @@ __global__ __launch_bounds__(256, 2) void chol_solve_kernel(const float *__restr
     } while (0)
     for (int i = 0; i < PV; ++i) pv[i] = make_double2(0.0, 0.0);
     BSQ_SOLVE_FETCH(0);
+    const int row0 = r0 + 4 * kk;
+    const bool split = row0 < planes.rows;
+    float f[4] = {};
+    if (split) {
+        const int em = planes.exponent ? *planes.emax : 0;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) f[u] = b_scale(planes.exponent, em, min(row0 + u, M - 1));
+    }
+    const uint64_t unit0 = 2 * static_cast<uint64_t>(row0 / 8) * planes.np + (kk & 1);  // 8-byte units
     // unrolled: every trip count and LDS offset below is a constant
 #pragma unroll
     for (int J = 0; J < NB; ++J) {
@@ -808,23 +822,43 @@ __global__ __launch_bounds__(256, 2) void chol_solve_kernel(const float *__restr
         }
         q += q1;
         // -Q_J -> LDS (operand of the later block columns), Q_J to the output
+        const int col = 32 * J + 16 * h + cc;
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-            const int rl = 4 * kk + u, col = 32 * J + 16 * h + cc, row = r0 + rl;
-            Qs[g][rl][col] = -q[u];
-            if (row < M && col < k) Q[static_cast<uint64_t>(row) * k + col] = q[u];
+            Qs[g][4 * kk + u][col] = -q[u];
+            if (planes.rows == 0 && row0 + u < M && col < k) Q[static_cast<uint64_t>(row0 + u) * k + col] = q[u];
+        }
+        if (split && col < k) {
+            uint32_t h01, l01, h23, l23;
+            split2(q[0], q[1], f[0], f[1], h01, l01);
+            split2(q[2], q[3], f[2], f[3], h23, l23);
+            const uint64_t at = unit0 + 2 * col;
+            if (row0 / 8 != M / 8 || planes.rot == 0) {
+                reinterpret_cast<uint2 *>(planes.hi)[at] = uint2{h01, h23};
+                reinterpret_cast<uint2 *>(planes.lo)[at] = uint2{l01, l23};
+            } else {
+                const uint64_t unit = 4 * (at & ~uint64_t{1});
+                const uint32_t h[4] = {h01, h01 >> 16, h23, h23 >> 16}, l[4] = {l01, l01 >> 16, l23, l23 >> 16};
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const uint64_t t = unit + ((row0 + u + planes.rot) & 7);
+                    planes.hi[t] = static_cast<uint16_t>(h[u]);
+                    planes.lo[t] = static_cast<uint16_t>(l[u]);
+                }
+            }
         }
     }
 }
 
 template <int NB>
 void chol_solve(const double *G, int k, double *Lbuf, const float *X, int M, float *Q, int *status,
-                hipStream_t stream) {
+                const H2Planes &planes, hipStream_t stream) {
     constexpr uint64_t KP = NB * 32;
     double *L = Lbuf, *LI = Lbuf + KP * KP;
     chol_blocked_kernel<NB><<<1, kCholThreads, 0, stream>>>(G, k, L, LI, status, nullptr);
     BSQ_HIP(hipGetLastError());
-    chol_solve_kernel<NB><<<static_cast<unsigned>(ceil_div(M, kSolveRows)), 256, 0, stream>>>(X, M, k, L, LI, Q);
+    chol_solve_kernel<NB><<<static_cast<unsigned>(ceil_div(std::max(M, planes.rows), kSolveRows)), 256, 0, stream>>>(
+        X, M, k, L, LI, Q, planes);
     BSQ_HIP(hipGetLastError());
 }
 
@@ -1024,18 +1058,21 @@ void launch_chol_blocked(const double *G, int k, double *Lbuf, float *B, int *st
 
 // G = L L^T (with shifted restarts on breakdown) and Q = X L^{-T} for the
 // M x k FP32 matrix X (row-major, leading dimension k) whose Gram G is.
+// With planes (h2_planes), Q goes there alone.
 void launch_chol_solve(const double *G, int k, double *Lbuf, const float *X, int M, float *Q, int *status,
-                       hipStream_t stream) {
+                       const H2Planes &planes, hipStream_t stream) {
     BSQ_REQUIRE(chol_blocked_supported(k) && M > 0 && X && Q && X != Q, "chol solve: bad arguments");
+    BSQ_REQUIRE(planes.rows == 0 || (planes.rows % 8 == 0 && planes.rows >= M && planes.K == M && planes.hi && planes.np >= k),
+                "chol solve: bad planes");
     switch (ceil_div(k, 32)) {
-        case 1: chol_solve<1>(G, k, Lbuf, X, M, Q, status, stream); break;
-        case 2: chol_solve<2>(G, k, Lbuf, X, M, Q, status, stream); break;
-        case 3: chol_solve<3>(G, k, Lbuf, X, M, Q, status, stream); break;
-        case 4: chol_solve<4>(G, k, Lbuf, X, M, Q, status, stream); break;
-        case 5: chol_solve<5>(G, k, Lbuf, X, M, Q, status, stream); break;
-        case 6: chol_solve<6>(G, k, Lbuf, X, M, Q, status, stream); break;
-        case 7: chol_solve<7>(G, k, Lbuf, X, M, Q, status, stream); break;
-        default: chol_solve<8>(G, k, Lbuf, X, M, Q, status, stream); break;
+        case 1: chol_solve<1>(G, k, Lbuf, X, M, Q, status, planes, stream); break;
+        case 2: chol_solve<2>(G, k, Lbuf, X, M, Q, status, planes, stream); break;
+        case 3: chol_solve<3>(G, k, Lbuf, X, M, Q, status, planes, stream); break;
+        case 4: chol_solve<4>(G, k, Lbuf, X, M, Q, status, planes, stream); break;
+        case 5: chol_solve<5>(G, k, Lbuf, X, M, Q, status, planes, stream); break;
+        case 6: chol_solve<6>(G, k, Lbuf, X, M, Q, status, planes, stream); break;
+        case 7: chol_solve<7>(G, k, Lbuf, X, M, Q, status, planes, stream); break;
+        default: chol_solve<8>(G, k, Lbuf, X, M, Q, status, planes, stream); break;
     }
 }
 

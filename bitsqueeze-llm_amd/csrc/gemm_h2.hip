@@ -19,11 +19,20 @@
 // true the rows run along K: B's row i takes the inverse power times
 // 2^(E_max) (E_max the exponent of the largest entry of A), so the product
 // needs one common factor.  B (an orthonormal basis or the sketch, entries
-// below 32) is scaled by 2^11 and split ahead (split_b_kernel) into planes
-// [k / 8][column][8] whose 16-byte units go to LDS as they lie; A is split as
-// it is staged.  All scalings are exact.  Rows holding infinities or NaN give
-// NaN results, as sums over them do.
+// below 32) is scaled by 2^11 and split ahead into planes [k / 8][column][8]
+// whose 16-byte units go to LDS as they lie: by the orthonormalisation that
+// makes it (chol_solve_kernel, k <= 256) or by split_b_kernel.  A is split as
+// it is staged.  K is padded to pairs of slices: B's planes hold zeros there
+// and A's loads repeat values of the same row or column.  (The reduction added
+// the last K % 64 products in FP32, one by one: 1000 x 1003, rank 8, a whole
+// round trip 408 us, padded 318.)  A small matrix's factorisation is bound by
+// its launches: planes written by the orthonormalisation, the sketch drawn in
+// row_scale_kernel's launch and the scales' maximum taken in split_b_kernel's
+// replace 2 niter + 2 of them (4096 x 4096, rank 8, niter 2, a round trip 505
+// -> 476 us, rank 256 1946 -> 1933).  All scalings are exact.  Rows holding
+// infinities or NaN give NaN results, as sums over them do.
 #include "bsq_internal.hpp"
+#include "gaussian.hpp"
 #include "h2_split.hpp"
 #include "tile_map.hpp"
 
@@ -39,7 +48,6 @@ constexpr int kThreads = 256;
 constexpr int T = 128;        // output tile
 constexpr int BK = 32;        // K slice
 constexpr int KG = BK / 8;    // groups of eight k per slice
-constexpr int kScaleB = 11;   // B's scale, a power of two
 
 __device__ __forceinline__ void dma16(const u32x4 *g, const u32x4 *l) {
     __builtin_amdgcn_global_load_lds((glb_void_t *)(g), (lds_void_t *)(reinterpret_cast<size_t>(l)), 16, 0, 0);
@@ -59,11 +67,19 @@ __device__ __forceinline__ void stage_barrier() {
 // Row exponents and scales of a row-major matrix: rs[i] = 2^(14 - E_i) scales
 // row i into f16's range, ri[i] = 2^(E_i - 14 - kScaleB) undoes it together
 // with B's scale.  One workgroup per row: the matrix is read once, at the
-// rate of a copy's reads.
-__global__ __launch_bounds__(kThreads) void row_scale_kernel(const float *__restrict__ A, int cols, int *__restrict__ E,
-                                                             float *__restrict__ rs, float *__restrict__ ri) {
+// rate of a copy's reads.  Workgroups past the last row draw the sketch (fill
+// values into R), which needs nothing of A.
+__global__ __launch_bounds__(kThreads) void row_scale_kernel(const float *__restrict__ A, int rows, int cols,
+                                                             int *__restrict__ E, float *__restrict__ rs,
+                                                             float *__restrict__ ri, float *__restrict__ R,
+                                                             uint64_t fill, uint64_t seed) {
     __shared__ uint32_t wmax[kThreads / 64];
     const int r = blockIdx.x, tid = threadIdx.x;
+    if (r >= rows) {  // uniform
+        gaussian_fill(R, fill, seed, static_cast<uint64_t>(r - rows) * kThreads + tid,
+                      static_cast<uint64_t>(gridDim.x - rows) * kThreads);
+        return;
+    }
     const float *row = A + static_cast<uint64_t>(r) * cols;
     uint32_t m = 0;  // bit patterns of magnitudes order as the magnitudes do, NaN above infinity
     const int head = min(cols, static_cast<int>((16 - (reinterpret_cast<uintptr_t>(row) & 15u)) & 15u) / 4);
@@ -90,46 +106,47 @@ __global__ __launch_bounds__(kThreads) void row_scale_kernel(const float *__rest
     }
 }
 
-// emax[0] = max_i E[i], and pow2(emax - 14 - kScaleB) beside it (one workgroup)
-__global__ __launch_bounds__(1024) void scale_max_kernel(const int *__restrict__ E, int rows, int *__restrict__ emax,
-                                                         float *__restrict__ common) {
-    __shared__ int wmax[16];
-    int m = -112;
-    for (int i = threadIdx.x; i < rows; i += 1024) m = max(m, E[i]);
-    for (int off = 32; off >= 1; off >>= 1) m = max(m, __shfl_xor(m, off));
-    if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = m;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int w = 1; w < 16; ++w) m = max(m, wmax[w]);
-        *emax = m;
-        *common = pow2(m - 14 - kScaleB);
-    }
-}
-
-// The first 8 kgroups rows of B (N columns, row-major) into its two planes,
-// [k / 8][np][8] f16 each, zero beyond column N: entry (k, n) times 2^kScaleB, and with E given also times
-// 2^(E[k] - *emax).  One lane per column and group of eight k.
-__global__ __launch_bounds__(kThreads) void split_b_kernel(const float *__restrict__ B, int N, int np, int kgroups,
-                                                           const int *__restrict__ E, const int *__restrict__ emax,
+// B (K x N, row-major) into its two planes, [k / 8][np][8] f16 each, kgroups
+// groups of k, zero beyond row K and column N: entry (k, n) times b_scale, at
+// place (k + rot) % 8 of its group if that is the partial one.
+// One lane per column and group of eight k.  With rows > 0 the maximum of E's
+// first `rows` entries is not yet known: the workgroups that need it find it
+// (E, at most a few tens of KB, comes from L2), and the first leaves it and
+// pow2(max - 14 - kScaleB) in emax and common.
+__global__ __launch_bounds__(kThreads) void split_b_kernel(const float *__restrict__ B, int K, int N, int np, int kgroups,
+                                                           int rot,
+                                                           const int *__restrict__ E, int rows, bool scaled,
+                                                           int *__restrict__ emax, float *__restrict__ common,
                                                            u32x4 *__restrict__ hi, u32x4 *__restrict__ lo) {
+    __shared__ int wmax[kThreads / 64];
+    int em = 0;
+    if (rows > 0 && (scaled || blockIdx.x == 0)) {  // uniform
+        em = -112;
+#pragma unroll 8
+        for (int i = threadIdx.x; i < rows; i += kThreads) em = max(em, E[i]);
+        for (int off = 32; off >= 1; off >>= 1) em = max(em, __shfl_xor(em, off));
+        if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = em;
+        __syncthreads();
+        em = max(max(wmax[0], wmax[1]), max(wmax[2], wmax[3]));
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            *emax = em;
+            *common = pow2(em - 14 - kScaleB);
+        }
+    } else if (scaled) {
+        em = *emax;
+    }
     const int t = blockIdx.x * kThreads + threadIdx.x;
     const int kg = t / np, n = t - kg * np;
     if (kg >= kgroups) return;
     float y[8];
+    const int turn = kg == K / 8 ? rot : 0;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-        y[i] = n < N ? B[static_cast<uint64_t>(8 * kg + i) * N + n] : 0.0f;
-    }
-    float f[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) f[i] = static_cast<float>(1 << kScaleB);
-    if (E) {
-        const int em = *emax;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) f[i] = pow2(max(E[8 * kg + i] - em, -138) + kScaleB);
+        const int k = 8 * kg + ((i - turn) & 7);
+        y[i] = n < N && k < K ? B[static_cast<uint64_t>(k) * N + n] : 0.0f;
     }
     u32x4 h, l;
-    split8(y, [&](int i) { return f[i]; }, h, l);
+    split8(y, [&](int i) { return b_scale(scaled ? E : nullptr, em, min(8 * kg + i, K - 1)); }, h, l);
     hi[t] = h;
     lo[t] = l;
 }
@@ -139,7 +156,7 @@ struct H2Args {
     const u32x4 *bh, *bl;  // B's planes
     const float *rs;       // scales of A's rows
     float *ws;             // partial tiles [tile row][tile column][part][tile]
-    int M, K, lda;
+    int M, N, K, lda;
     int np;                // columns of the planes (a multiple of 64)
     int tiles_n;           // output tiles per row of tiles
     int pairs;             // pairs of K slices per tile
@@ -212,11 +229,13 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         const int m0 = ca.tm * T, k0 = ca.ks * BK;
         asm volatile("" ::: "memory");  // stays behind the DMA before it
         if constexpr (!TA) {
-            const int k = k0 + 8 * (tid & 3);
+            const int k = min(k0 + 8 * (tid & 3), g.K - 8);
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 const int r = min(m0 + 64 * h + (tid >> 2), g.M - 1);
                 vs[h] = g.rs[r];
+                // past K: the row's last eight values, which meet a partial
+                // group of B turned to fit them (H2Planes), or zeros
                 // rows may start at any multiple of four bytes
                 __builtin_memcpy(&va[h][0], __builtin_assume_aligned(g.A + static_cast<uint64_t>(r) * g.lda + k, 4), 32);
             }
@@ -226,13 +245,16 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
             for (int h = 0; h < 2; ++h) c[h] = 4u * static_cast<uint32_t>(min(m0 + 64 * h + lane, g.M - 1));
 #pragma unroll
-            for (int i = 0; i < 8; ++i) vs[i] = g.rs[k0 + 8 * wave + i];
-            const char *p = reinterpret_cast<const char *>(g.A) +
-                            4u * static_cast<uint64_t>(k0 + 8 * __builtin_amdgcn_readfirstlane(wave)) * g.lda;
+            for (int i = 0; i < 8; ++i) vs[i] = g.rs[min(k0 + 8 * wave + i, g.K - 1)];
+            const int k = k0 + 8 * __builtin_amdgcn_readfirstlane(wave);
+            const char *p = reinterpret_cast<const char *>(g.A) + 4u * static_cast<uint64_t>(min(k, g.K - 1)) * g.lda;
 #pragma unroll
-            for (int i = 0; i < 8; ++i, p += 4u * static_cast<uint64_t>(g.lda))
+            for (int i = 0; i < 8; ++i) {
 #pragma unroll
                 for (int h = 0; h < 2; ++h) va[h][i] = *reinterpret_cast<const float *>(p + c[h]);
+                // past K: the last row again, against zeros of B
+                p += k + i + 1 < g.K ? 4u * static_cast<uint64_t>(g.lda) : 0u;
+            }
         }
         ca.next(nk);
     };
@@ -288,8 +310,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
                    ((static_cast<uint64_t>(t) * g.tiles_n + tn) * g.maxparts + (range - first)) * (T * T / 4) + unit;
 #pragma unroll
         for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int jj = 0; jj < 2; ++jj)
+            for (int jj = 0; jj < 2; ++jj) {
+                if (tn * T + wn0 + 32 * jj >= g.N) continue;  // uniform: columns past C's
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
                     f32x4 v;
@@ -298,6 +320,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
                         v[e] = acc.hi[i][jj][4 * q + e] + acc.lo[i][jj][4 * q + e] * kLoInv;
                     W[((2 * i + jj) * 4 + q) * 64] = v;
                 }
+            }
     };
 
     // a slice: its A and B are in the current stage once every wave has
@@ -339,13 +362,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 }
 
 // C = the sum of each tile's parts in order, times the row's (ri) or the
-// common factor, plus the k past the last whole pair of slices (fewer than 64,
-// summed in FP32 from A and B themselves).  A lane takes one 16-byte unit of
-// the parts: four consecutive rows of a column, 32 lanes 32 columns.
+// common factor.  A lane takes one 16-byte unit of the parts: four consecutive
+// rows of a column, 32 lanes 32 columns.
 template <bool TA>
-__global__ __launch_bounds__(256) void h2_reduce_kernel(H2Args g, int N, const float *__restrict__ B,
-                                                        const float *__restrict__ ri, const float *__restrict__ common,
-                                                        float *__restrict__ C) {
+__global__ __launch_bounds__(256) void h2_reduce_kernel(H2Args g, const float *__restrict__ ri,
+                                                        const float *__restrict__ common, float *__restrict__ C) {
     constexpr int kUnits = T * T / 4;
     const int tile = static_cast<int>(blockIdx.x) / (kUnits / 256);
     const int unit = (static_cast<int>(blockIdx.x) % (kUnits / 256)) * 256 + threadIdx.x;
@@ -356,19 +377,14 @@ __global__ __launch_bounds__(256) void h2_reduce_kernel(H2Args g, int N, const f
     const int lane = unit & 63, q = (unit >> 6) & 3, jj = (unit >> 8) & 1, i = (unit >> 9) & 1, wave = unit >> 10;
     const int gi = tm * T + (wave >> 1) * 64 + 32 * i + 8 * q + 4 * (lane >> 5);
     const int gj = tn * T + (wave & 1) * 64 + 32 * jj + (lane & 31);
-    if (gi >= g.M || gj >= N) return;
+    if (gi >= g.M || gj >= g.N) return;
     f32x4 s = W[0];
 #pragma unroll 4
     for (int p = 1; p < parts; ++p) s += W[static_cast<uint64_t>(p) * kUnits];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-        const int r = min(gi + e, g.M - 1);
-        float v = s[e] * (TA ? *common : ri[r]);
-        for (int k = g.pairs * 2 * BK; k < g.K; ++k) {
-            const float a = TA ? g.A[static_cast<uint64_t>(k) * g.lda + r] : g.A[static_cast<uint64_t>(r) * g.lda + k];
-            v = fmaf(a, B[static_cast<uint64_t>(k) * N + gj], v);
-        }
-        if (gi + e < g.M) C[static_cast<uint64_t>(r) * N + gj] = v;
+        const int r = gi + e;
+        if (r < g.M) C[static_cast<uint64_t>(r) * g.N + gj] = s[e] * (TA ? *common : ri[r]);
     }
 }
 
@@ -385,7 +401,7 @@ H2Plan h2_plan(int M, int N, int K) {
     H2Plan p{};
     p.tiles_m = static_cast<int>(ceil_div(M, T));
     p.tiles_n = static_cast<int>(ceil_div(N, T));
-    p.pairs = K / (2 * BK);  // the rest of K goes with the reduction
+    p.pairs = static_cast<int>(ceil_div(K, 2 * BK));
     p.units = p.tiles_m * p.pairs;
     const int most = std::max(1, 2 * cu_count() / p.tiles_n);
     p.ranges = std::max(1, std::min({most, std::max(p.tiles_m, p.units / 2), p.units}));
@@ -407,52 +423,73 @@ int pad64(int n) { return static_cast<int>(ceil_div(n, 64) * 64); }
 uint64_t h2_workspace_bytes(int M, int N, int K) { return h2_plan(M, N, K).bytes; }
 
 // f16 values of the two planes of a K x N operand B.
-uint64_t h2_plane_units(int K, int N) { return static_cast<uint64_t>(K / (2 * BK)) * 2 * BK * pad64(N) * 2; }
+uint64_t h2_plane_units(int K, int N) { return 2 * static_cast<uint64_t>(pad64(K)) * pad64(N); }
 
 bool h2_supported(int K) { return K >= 2 * BK; }
 
-void launch_h2_scales(const float *A, int m, int n, const H2Scales &s, hipStream_t stream) {
-    BSQ_REQUIRE(A && m > 0 && n > 0 && s.exponent && s.scale && s.inverse && s.emax && s.common, "h2 scales: bad arguments");
-    row_scale_kernel<<<static_cast<unsigned>(m), kThreads, 0, stream>>>(A, n, s.exponent, s.scale, s.inverse);
-    BSQ_HIP(hipGetLastError());
-    scale_max_kernel<<<1, 1024, 0, stream>>>(s.exponent, m, s.emax, s.common);
+void launch_h2_scales(const float *A, int m, int n, const H2Scales &s, float *R, uint64_t fill, uint64_t seed,
+                      hipStream_t stream) {
+    BSQ_REQUIRE(A && m > 0 && n > 0 && s.exponent && s.scale && s.inverse && (R || fill == 0),
+                "h2 scales: bad arguments");
+    const uint64_t draws = std::min<uint64_t>(ceil_div(fill, 4 * kThreads), static_cast<uint64_t>(cu_count()) * 8);
+    row_scale_kernel<<<static_cast<unsigned>(m + draws), kThreads, 0, stream>>>(A, m, n, s.exponent, s.scale,
+                                                                               s.inverse, R, fill, seed);
     BSQ_HIP(hipGetLastError());
 }
 
-void launch_h2_gemm(bool ta, int m, int n, int q, const float *A, const H2Scales &s, const float *B, uint16_t *planes,
-                    float *C, float *workspace, uint64_t workspace_bytes, hipStream_t stream) {
+H2Planes h2_planes(bool ta, int K, int q, const H2Scales &s, uint16_t *planes) {
+    H2Planes b;
+    b.K = K;
+    b.rows = pad64(K);
+    b.rot = ta ? 0 : -K & 7;
+    b.np = pad64(q);
+    b.hi = planes;
+    b.lo = planes + static_cast<uint64_t>(b.rows) * b.np;
+    b.exponent = ta ? s.exponent : nullptr;
+    b.emax = s.emax;
+    return b;
+}
+
+void launch_h2_split(const float *B, int q, const H2Planes &b, const H2Scales &s, int new_rows, hipStream_t stream) {
+    BSQ_REQUIRE(q > 0 && (B || b.rows == 0) && s.emax && s.common, "h2 split: bad arguments");
+    const uint64_t units = static_cast<uint64_t>(b.rows / 8) * b.np;
+    if (units == 0 && new_rows == 0) return;
+    split_b_kernel<<<static_cast<unsigned>(std::max<uint64_t>(1, ceil_div(units, kThreads))), kThreads, 0, stream>>>(
+        B, b.K, q, b.np, b.rows / 8, b.rot, s.exponent, new_rows, b.exponent != nullptr, s.emax, s.common,
+        reinterpret_cast<u32x4 *>(b.hi), reinterpret_cast<u32x4 *>(b.lo));
+    BSQ_HIP(hipGetLastError());
+}
+
+void launch_h2_gemm(bool ta, int m, int n, int q, const float *A, const H2Scales &s, const H2Planes &b, float *C,
+                    float *workspace, uint64_t workspace_bytes, hipStream_t stream) {
     const int M = ta ? n : m, K = ta ? m : n;
-    BSQ_REQUIRE(M > 0 && q > 0 && h2_supported(K) && A && B && C && planes && workspace, "h2 gemm: bad arguments");
+    BSQ_REQUIRE(M > 0 && q > 0 && h2_supported(K) && A && C && b.hi && workspace, "h2 gemm: bad arguments");
     const H2Plan p = h2_plan(M, q, K);
     BSQ_REQUIRE(p.bytes <= workspace_bytes, "h2 gemm: workspace too small");
     H2Args g{};
-    const int np = pad64(q), kgroups = p.pairs * 2 * KG;
+    BSQ_REQUIRE(b.K == K && b.np == pad64(q), "h2 gemm: planes of another operand");
     g.A = A;
-    auto *bh = reinterpret_cast<u32x4 *>(planes);
-    auto *bl = bh + static_cast<uint64_t>(kgroups) * np;
-    g.bh = bh;
-    g.bl = bl;
+    g.bh = reinterpret_cast<const u32x4 *>(b.hi);
+    g.bl = reinterpret_cast<const u32x4 *>(b.lo);
     g.rs = s.scale;
     g.ws = workspace;
     g.M = M;
+    g.N = q;
     g.K = K;
     g.lda = n;
-    g.np = np;
+    g.np = b.np;
     g.tiles_n = p.tiles_n;
     g.pairs = p.pairs;
     g.units = p.units;
     g.ranges = p.ranges;
     g.maxparts = p.maxparts;
-    split_b_kernel<<<static_cast<unsigned>(ceil_div(static_cast<uint64_t>(kgroups) * np, kThreads)), kThreads, 0, stream>>>(
-        B, q, np, kgroups, ta ? s.exponent : nullptr, s.emax, bh, bl);
-    BSQ_HIP(hipGetLastError());
     const dim3 grid(static_cast<unsigned>(p.ranges * p.tiles_n)),
         rgrid(static_cast<unsigned>(p.tiles_m * p.tiles_n * (T * T / 4 / 256)));
     if (ta) gemm_h2_kernel<true><<<grid, kThreads, 0, stream>>>(g);
     else gemm_h2_kernel<false><<<grid, kThreads, 0, stream>>>(g);
     BSQ_HIP(hipGetLastError());
-    if (ta) h2_reduce_kernel<true><<<rgrid, 256, 0, stream>>>(g, q, B, nullptr, s.common, C);
-    else h2_reduce_kernel<false><<<rgrid, 256, 0, stream>>>(g, q, B, s.inverse, nullptr, C);
+    if (ta) h2_reduce_kernel<true><<<rgrid, 256, 0, stream>>>(g, nullptr, s.common, C);
+    else h2_reduce_kernel<false><<<rgrid, 256, 0, stream>>>(g, s.inverse, nullptr, C);
     BSQ_HIP(hipGetLastError());
 }
 

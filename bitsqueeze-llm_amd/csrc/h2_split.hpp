@@ -40,28 +40,41 @@ __device__ __forceinline__ int row_exponent(uint32_t bits) {
 // 2^e, e in [-149, 127]
 __device__ __forceinline__ float pow2(int e) { return __builtin_ldexpf(1.0f, e); }
 
-// eight values x, scaled by f, to their pieces.  Three mixed-precision FMAs a
-// value write the pieces into their halves (h = f16(f x), f x - h exactly,
-// l = f16 of 2^11 times that); left to the compiler it is five instructions,
-// with the products and the packing of their own.
+// two values x, scaled by f, to their pieces, packed.  Three mixed-precision
+// FMAs a value write the pieces into their halves (h = f16(f x), f x - h
+// exactly, l = f16 of 2^11 times that); left to the compiler it is five
+// instructions, with the products and the packing of their own.
+__device__ __forceinline__ void split2(float x0, float x1, float f0, float f1, uint32_t &h, uint32_t &l) {
+    uint32_t hp, lp;
+    float r0, r1;
+    asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "=v"(hp) : "v"(x0), "v"(f0));
+    asm("v_fma_mixhi_f16 %0, %1, %2, 0" : "+v"(hp) : "v"(x1), "v"(f1));
+    asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel_hi:[0,0,1]" : "=v"(r0) : "v"(x0), "v"(f0), "v"(hp));
+    asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "=v"(r1) : "v"(x1), "v"(f1), "v"(hp));
+    asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "=v"(lp) : "v"(r0), "s"(kLo));
+    asm("v_fma_mixhi_f16 %0, %1, %2, 0" : "+v"(lp) : "v"(r1), "s"(kLo));
+    h = hp;
+    l = lp;
+}
+
+// eight values x, scaled by f, to their pieces
 template <class F>
 __device__ __forceinline__ void split8(const float (&x)[8], F &&f, u32x4 &h, u32x4 &l) {
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
-        const float x0 = x[2 * p], x1 = x[2 * p + 1], f0 = f(2 * p), f1 = f(2 * p + 1);
         uint32_t hp, lp;
-        float r0, r1;
-        asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "=v"(hp) : "v"(x0), "v"(f0));
-        asm("v_fma_mixhi_f16 %0, %1, %2, 0" : "+v"(hp) : "v"(x1), "v"(f1));
-        asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel_hi:[0,0,1]" : "=v"(r0) : "v"(x0), "v"(f0), "v"(hp));
-        asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel:[0,0,1] op_sel_hi:[0,0,1]"
-            : "=v"(r1)
-            : "v"(x1), "v"(f1), "v"(hp));
-        asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "=v"(lp) : "v"(r0), "s"(kLo));
-        asm("v_fma_mixhi_f16 %0, %1, %2, 0" : "+v"(lp) : "v"(r1), "s"(kLo));
+        split2(x[2 * p], x[2 * p + 1], f(2 * p), f(2 * p + 1), hp, lp);
         h[p] = hp;
         l[p] = lp;
     }
+}
+
+// The range finder's small operand B (an orthonormal basis or the sketch):
+// scaled by 2^kScaleB, and in products with A^T its row k also by
+// 2^(E[k] - emax) (E, emax: the row exponents of A and their maximum).
+constexpr int kScaleB = 11;
+__device__ __forceinline__ float b_scale(const int *__restrict__ E, int emax, int k) {
+    return E ? pow2(max(E[k] - emax, -138) + kScaleB) : static_cast<float>(1 << kScaleB);
 }
 
 // The matrix instructions of one 16-deep step of a wave's 64 x 64 block, from

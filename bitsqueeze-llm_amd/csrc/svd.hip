@@ -17,6 +17,7 @@
 // V_hat = Y U_hat / S by one more GEMM.  Signs are normalised so that the
 // largest-magnitude entry of every column of U is positive.
 #include "bsq_internal.hpp"
+#include "gaussian.hpp"
 
 #include <algorithm>
 #include <mutex>
@@ -43,48 +44,15 @@ void launch_chol_blocked(const double *G, int k, double *Lbuf, float *B, int *st
 void launch_orth_refine(const double *G, const double *rowsq, int k, double *Lbuf, float *B, int *status, int *run,
                         hipStream_t stream);
 void launch_chol_solve(const double *G, int k, double *Lbuf, const float *X, int M, float *Q, int *status,
-                       hipStream_t stream);
+                       const H2Planes &planes, hipStream_t stream);
 void launch_syev(const double *G, int k, double *W, double *Z, double *small, double *scratch, int *iscratch,
                  double *lambda, float *Uh, hipStream_t stream);
 
 namespace {
 
-// Philox4x32-10 (Salmon, Moraes, Dror, Shaw, "Parallel random numbers: as
-// easy as 1, 2, 3", SC'11): counter = element group index, key = seed.
-__device__ __forceinline__ uint4 philox4x32_10(uint4 c, uint2 k) {
-    constexpr uint32_t M0 = 0xD2511F53u, M1 = 0xCD9E8D57u, W0 = 0x9E3779B9u, W1 = 0xBB67AE85u;
-#pragma unroll
-    for (int r = 0; r < 10; ++r) {
-        const uint32_t hi0 = __umulhi(M0, c.x), lo0 = M0 * c.x;
-        const uint32_t hi1 = __umulhi(M1, c.z), lo1 = M1 * c.z;
-        c = make_uint4(hi1 ^ c.y ^ k.x, lo1, hi0 ^ c.w ^ k.y, lo0);
-        k.x += W0;
-        k.y += W1;
-    }
-    return c;
-}
-
 __global__ void gaussian_fill_kernel(float *__restrict__ out, uint64_t n, uint64_t seed) {
-    const uint64_t groups = (n + 3) / 4;
-    for (uint64_t g = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; g < groups;
-         g += static_cast<uint64_t>(gridDim.x) * blockDim.x) {
-        const uint4 r = philox4x32_10(make_uint4(static_cast<uint32_t>(g), static_cast<uint32_t>(g >> 32), 0u, 0u),
-                                      make_uint2(static_cast<uint32_t>(seed), static_cast<uint32_t>(seed >> 32)));
-        // Box-Muller on (r.x, r.y) and (r.z, r.w); u1 in (0, 1]
-        constexpr float kInv32 = 2.3283064365386963e-10f;
-        constexpr float kTwoPi = 6.283185307179586f;
-        const float u1 = (static_cast<float>(r.x) + 1.0f) * kInv32, u2 = static_cast<float>(r.y) * kInv32;
-        const float u3 = (static_cast<float>(r.z) + 1.0f) * kInv32, u4 = static_cast<float>(r.w) * kInv32;
-        const float ra = sqrtf(-2.0f * logf(fminf(u1, 1.0f))), rb = sqrtf(-2.0f * logf(fminf(u3, 1.0f)));
-        float s1, c1, s2, c2;
-        sincosf(kTwoPi * u2, &s1, &c1);
-        sincosf(kTwoPi * u4, &s2, &c2);
-        const float v[4] = {ra * c1, ra * s1, rb * c2, rb * s2};
-        const uint64_t e0 = g * 4;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            if (e0 + i < n) out[e0 + i] = v[i];
-    }
+    gaussian_fill(out, n, seed, static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x,
+                  static_cast<uint64_t>(gridDim.x) * blockDim.x);
 }
 
 // S[t] = sqrt(max(lambda[t], 0))
@@ -388,29 +356,41 @@ void svd_run(SvdPlan *p, const float *A, const float *sketch, uint64_t seed, flo
     BSQ_REQUIRE(p && A && U && S && V, "svd: null argument");
     const int m = p->m, n = p->n, k = p->k, Mw = p->Mw, Nw = p->Nw;
     const float *R = sketch;
-    if (!R) {
-        launch_gaussian_fill(p->R, static_cast<uint64_t>(Nw) * k, seed, st);
-        R = p->R;
-    }
-    if (p->h2) launch_h2_scales(A, m, n, p->h2s, st);
-    // out = A B (n x k, ta false) or A^T B (m x k)
-    auto times = [&](bool ta, const float *Bm, float *out) {
+    if (!R) R = p->R;
+    const uint64_t draws = sketch ? 0 : static_cast<uint64_t>(Nw) * k;
+    if (p->h2) launch_h2_scales(A, m, n, p->h2s, p->R, draws, seed, st);
+    else if (draws) launch_gaussian_fill(p->R, draws, seed, st);
+    // the planes of the operand of A B (ta false) or A^T B
+    auto planes = [&](bool ta) { return h2_planes(ta, ta ? m : n, k, p->h2s, p->planes); };
+    if (p->h2 && sketch) launch_h2_split(nullptr, k, H2Planes{}, p->h2s, m, st);  // the scales' maximum alone
+    // out = A B (n x k, ta false) or A^T B (m x k); in_planes: B's planes are written
+    auto times = [&](bool ta, const float *Bm, float *out, bool in_planes) {
         timed_launch(kTimeRangeFinder, st, [&] {
             // a caller's sketch may hold anything: it takes the FP32 product
-            if (p->h2 && Bm != sketch)
-                launch_h2_gemm(ta, m, n, k, A, p->h2s, Bm, p->planes, out, p->gemm_ws, p->gemm_ws_bytes, st);
-            else
+            if (p->h2 && Bm != sketch) {
+                const H2Planes b = planes(ta);
+                if (!in_planes) launch_h2_split(Bm, k, b, p->h2s, Bm == R ? m : 0, st);
+                launch_h2_gemm(ta, m, n, k, A, p->h2s, b, out, p->gemm_ws, p->gemm_ws_bytes, st);
+            } else {
                 launch_gemm(ta, false, ta ? n : m, k, ta ? m : n, A, n, Bm, k, out, k, p->gemm_ws,
                             p->gemm_ws_bytes, st);
+            }
         });
     };
-    auto aw_times = [&](const float *Bm, float *out) { times(p->transposed, Bm, out); };    // X (Mw x k) = A_w B
-    auto awt_times = [&](const float *Bm, float *out) { times(!p->transposed, Bm, out); };  // Y (Nw x k) = A_w^T B
-    // one CholeskyQR pass: out = in * L^{-T}, G = in^T in = L L^T
-    auto orth = [&](const float *in, float *out, int rows) {
+    const bool fused = p->h2 && p->Lbuf;  // orth writes its result's planes
+    auto aw_times = [&](const float *Bm, float *out, bool in_planes) {  // X (Mw x k) = A_w B
+        times(p->transposed, Bm, out, in_planes);
+    };
+    auto awt_times = [&](const float *Bm, float *out, bool in_planes) {  // Y (Nw x k) = A_w^T B
+        times(!p->transposed, Bm, out, in_planes);
+    };
+    // one CholeskyQR pass: out = in * L^{-T}, G = in^T in = L L^T.  `only`: the
+    // result is the operand of a product with A alone, `ta` its form, and goes
+    // to its planes in place of out.
+    auto orth = [&](const float *in, float *out, int rows, bool only, bool ta) {
         launch_gram(in, rows, k, k, p->G, p->gram_ws, st);
         if (p->Lbuf) {  // out L^T = in, by blocked forward substitution
-            launch_chol_solve(p->G, k, p->Lbuf, in, rows, out, p->status, st);
+            launch_chol_solve(p->G, k, p->Lbuf, in, rows, out, p->status, only && p->h2 ? planes(ta) : H2Planes{}, st);
             return;
         }
         if (chol_inv_2x2_supported(k))  // Linv holds L^{-1}
@@ -421,15 +401,15 @@ void svd_run(SvdPlan *p, const float *A, const float *sketch, uint64_t seed, flo
                     p->gemm_ws_bytes, st);
     };
     float *Xa = p->X, *Xb = p->X2, *Ya = p->Y, *Yb = p->Y2;
-    aw_times(R, Xa);
-    orth(Xa, Xb, Mw);
+    aw_times(R, Xa, false);
+    orth(Xa, Xb, Mw, p->niter > 0, !p->transposed);
     std::swap(Xa, Xb);
     for (int it = 0; it < p->niter; ++it) {
-        awt_times(Xa, Ya);
-        orth(Ya, Yb, Nw);
+        awt_times(Xa, Ya, fused);
+        orth(Ya, Yb, Nw, true, p->transposed);
         std::swap(Ya, Yb);
-        aw_times(Ya, Xa);
-        orth(Xa, Xb, Mw);
+        aw_times(Ya, Xa, fused);
+        orth(Xa, Xb, Mw, it + 1 < p->niter, !p->transposed);
         std::swap(Xa, Xb);
     }
     // second pass on the final basis: CholeskyQR2, or, when the first pass
@@ -440,11 +420,11 @@ void svd_run(SvdPlan *p, const float *A, const float *sketch, uint64_t seed, flo
         launch_gemm(false, false, Mw, k, k, Xa, k, p->Linv, k, Xb, k, p->gemm_ws,
                     p->gemm_ws_bytes, st);
     } else {
-        orth(Xa, Xb, Mw);
+        orth(Xa, Xb, Mw, false, false);
     }
     std::swap(Xa, Xb);
     // Y = A_w^T Q = B^T;  B B^T = Y^T Y = U_hat diag(S^2) U_hat^T
-    awt_times(Xa, Ya);
+    awt_times(Xa, Ya, false);
     launch_gram(Ya, Nw, k, k, p->G, p->gram_ws, st);
     launch_syev(p->G, k, p->W, p->Z, p->small, p->scratch, p->iscratch, p->lambda, p->Uh, st);
     sqrt_eig_kernel<<<static_cast<unsigned>(ceil_div(k, 256)), 256, 0, st>>>(p->lambda, k, S);

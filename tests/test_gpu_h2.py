@@ -3,8 +3,9 @@ bsq_svd_lowrank with the built-in sketch (a caller's sketch takes the FP32
 product), against the FP64 oracle given the same sketch.
 
 Sizes sit at the edges of the kernel's 128 x 128 tiles, its pairs of 32-deep
-slices and its 64-column operand planes (remainders of K go with the
-reduction), both orientations, rows of a length that is no multiple of four
+slices and its 64-column operand planes (K padded with zeros; a last group of
+fewer than eight k lies turned in the planes of products with A), both
+orientations, rows of a length that is no multiple of four
 (unaligned row starts), and matrices whose rows differ in scale by 2^28, with
 zero rows among them.
 
@@ -44,6 +45,20 @@ def svd_and_oracle(A, q, it):
 def test_products_at_tile_edges(m, n, q, it):
     A = low_rank(m, n, min(m, n, 96), np.random.default_rng(m * 7 + n))
     got, ref = svd_and_oracle(A, q, it)
+    assert np.linalg.norm(got - ref) <= TOL * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("sketch", [False, True])
+@pytest.mark.parametrize("q", [33, 257])  # planes from the orthonormalisation, and split from FP32 bases
+@pytest.mark.parametrize("m,n", [(513, 522), (523, 516), (517, 518), (519, 576), (584, 520)])
+def test_last_group_of_k(m, n, q, sketch):
+    """Every remainder of K by eight, in both products."""
+    A = low_rank(m, n, 96, np.random.default_rng(m + 3 * n))
+    if not sketch:
+        got, ref = svd_and_oracle(A, q, 1)
+    else:
+        R = np.random.default_rng(q).standard_normal((min(m, n), q)).astype(np.float32)
+        got, ref = O.reconstruct(*B.svd_lowrank(A, q, 1, R)), O.reconstruct(*O.svd_lowrank(A, q, 1, R))
     assert np.linalg.norm(got - ref) <= TOL * np.linalg.norm(ref)
 
 
