@@ -439,78 +439,19 @@ __global__ __launch_bounds__(kBig) void sytrd_kernel(double *__restrict__ W, int
 // ---------------------------------------------------------------------------
 // Householder tridiagonalisation for 256 < k <= 512, the same reduction
 // (LAPACK dsytd2 order: reflector j from column j, p = A v, w = tau p -
-// (tau^2 / 2)(p.v) v, A -= v w^T + w v^T) spread over two kernels per column
-// on a global-memory working copy A (full symmetric storage):
+// (tau^2 / 2)(p.v) v, A -= v w^T + w v^T) on a global-memory working copy A
+// (full symmetric storage), for its first k - 256 columns:
 //   trd_step_kernel (one launch per column, many CUs): every workgroup
 //     forms w_{j-1} from p_{j-1}, row j of A with update j-1 applied (its
 //     column by symmetry) and reflector j; workgroup 0 writes d[j], e[j],
 //     tau[j] and row j of H (zero up to column j); then one wave per row of
 //     the trailing block applies update j-1 and forms p_j = A v_j in the
 //     same pass;
-//   trd_col_kernel (one workgroup) finishes the last column: w_{k-3},
-//     d[k-2], e[k-2] and d[k-1].
+// The last 256 columns go to the register kernel (sytrd.hip).
 // Every column thus costs one launch and one read and write of the
 // trailing block on all CUs, instead of two reads and a write on one CU.
 // ---------------------------------------------------------------------------
-constexpr int kTrdColThreads = 512;  // one index per lane (k <= 512)
-
-__global__ __launch_bounds__(kTrdColThreads) void trd_col_kernel(
-    const double *__restrict__ A, int k, int j, const double *__restrict__ vprev, const double *__restrict__ p,
-    double *__restrict__ w, double *__restrict__ vcur, double *__restrict__ d, double *__restrict__ e,
-    double *__restrict__ tau, double *__restrict__ H) {
-    __shared__ double red[kTrdColThreads / 64];
-    __shared__ double s_wj, s_alpha;
-    const int i = threadIdx.x;
-    const bool in = i < k;
-    // w_{j-1} on indices >= j (zero below): p_{j-1} = A_{j-1} v_{j-1}
-    double wi = 0.0, vpi = 0.0;
-    if (j > 0) {
-        const double tp = tau[j - 1];
-        const double pi = (in && i >= j) ? p[i] : 0.0;
-        vpi = (in && i >= j) ? vprev[i] : 0.0;
-        const double pv = block_sum(pi * vpi, red);
-        wi = tp * pi - (0.5 * tp * tp * pv) * vpi;
-        if (in) w[i] = wi;
-        if (i == j) s_wj = wi;
-        __syncthreads();
-    }
-    // row j with update j-1 applied (v_{j-1}[j] = 1), as trd_step_kernel
-    // forms it
-    double x = 0.0;
-    if (in && i >= j) {
-        x = A[static_cast<uint64_t>(j) * k + i];
-        if (j > 0) x -= (vprev[j] * wi + s_wj * vpi);
-    }
-    if (i == j) d[j] = x;
-    if (i == j + 1) s_alpha = x;
-    const double sig = block_sum((in && i >= j + 2) ? x * x : 0.0, red);
-    const double alpha = s_alpha;  // written before block_sum's barriers
-    double t = 0.0, beta = alpha, scal = 0.0;
-    if (sig > 0.0) {
-        const double nrm = sqrt(fma(alpha, alpha, sig));
-        beta = (alpha >= 0.0) ? -nrm : nrm;
-        t = (beta - alpha) / beta;
-        scal = 1.0 / (alpha - beta);
-    }
-    if (in) {
-        const double v = (i == j + 1) ? 1.0 : ((i > j + 1) ? x * scal : 0.0);
-        vcur[i] = v;
-        H[static_cast<uint64_t>(j) * k + i] = v;
-    }
-    if (i == 0) {
-        e[j] = beta;
-        tau[j] = t;
-    }
-    if (j == k - 2) {  // the last call: d[k-1] with update k-3, H's last row zero
-        if (i == k - 1) {
-            d[k - 1] = A[static_cast<uint64_t>(k - 1) * k + (k - 1)] - (vpi * wi + wi * vpi);
-            tau[k - 1] = 0.0;
-        }
-        if (in) H[static_cast<uint64_t>(k - 1) * k + i] = 0.0;
-    }
-}
-
-// One column step j = 0 .. k-3 in one launch: every workgroup forms w_{j-1}
+// One column step j in one launch: every workgroup forms w_{j-1}
 // and reflector j itself from the same data in the same order (so they all
 // hold the same bits; workgroup 0 writes d[j], e[j], tau[j] and row j of H),
 // then its waves take one trailing row each: update j-1 applied, p_j = A v_j.
@@ -1184,7 +1125,7 @@ __global__ __launch_bounds__(256) void backtransform_rows_kernel(const double *_
         for (int q = 0; q < NQ; ++q) {
             const int lin = threadIdx.x + 256 * q, rr = lin / (KPL * 64), i = lin % (KPL * 64);
             const int j = j0 - rr;
-            pre[q] = (j >= jl && i < k) ? H[static_cast<uint64_t>(j) * k + i] : 0.0;
+            pre[q] = (j >= jl && i > j && i < k) ? H[static_cast<uint64_t>(j) * k + i] : 0.0;
         }
         pt = (threadIdx.x < RB && j0 - static_cast<int>(threadIdx.x) >= jl) ? tau[j0 - threadIdx.x] : 0.0;
     };
@@ -1251,6 +1192,8 @@ __global__ __launch_bounds__(256) void backtransform_rows_kernel(const double *_
 
 bool sytrd_blocked_supported(int k);
 void launch_sytrd_blocked(const double *G, int k, double *d, double *e, double *tau, double *H, hipStream_t stream);
+void launch_sytrd_tail(const double *A, int k, const double *p, double *d, double *e, double *tau, double *H,
+                       hipStream_t stream);
 
 // ---------------------------------------------------------------------------
 // launchers
@@ -1321,20 +1264,21 @@ void launch_syev(const double *G, int k, double *W, double *Z, double *small, do
     bool reg = true;
     if (sytrd_blocked_supported(k)) {
         launch_sytrd_blocked(G, k, d, e, tau, W, stream);
-    } else if (k > 256 && k <= kTrdColThreads) {
+    } else if (k > 256 && k <= kTrdStepThreads) {
         // working copy and vectors in the scratch, which the eigenvector
         // kernels below only use afterwards
-        double *A = scratch, *p0 = scratch + static_cast<size_t>(k) * k, *p1 = p0 + k, *w = p1 + k, *vl = w + k;
+        double *A = scratch, *p0 = scratch + static_cast<size_t>(k) * k, *p1 = p0 + k;
         BSQ_HIP(hipMemcpyAsync(A, G, static_cast<size_t>(k) * k * sizeof(double), hipMemcpyDeviceToDevice, stream));
-        // one launch per reflector j = 0 .. k-3, then the last column
-        for (int j = 0; j + 3 <= k; ++j) {
+        // one launch per reflector j = 0 .. k-257
+        const int j0 = k - 256;
+        for (int j = 0; j < j0; ++j) {
             const unsigned rows = static_cast<unsigned>(k - j - 1);
             trd_step_kernel<<<static_cast<unsigned>(ceil_div(rows, kTrdStepThreads / 64)), kTrdStepThreads, 0,
                               stream>>>(A, k, j, (j & 1) ? p0 : p1, (j & 1) ? p1 : p0, d, e, tau, W);
         }
-        const int jl = k - 2;  // p_{k-3} was written by step k-3 into ((k-3) & 1) ? p1 : p0
-        trd_col_kernel<<<1, kTrdColThreads, 0, stream>>>(A, k, jl, W + static_cast<size_t>(jl - 1) * k,
-                                                         ((jl - 1) & 1) ? p1 : p0, w, vl, d, e, tau, W);
+        BSQ_HIP(hipGetLastError());
+        // p_{j0-1} was written by step j0-1 into ((j0-1) & 1) ? p1 : p0
+        launch_sytrd_tail(A, k, ((j0 - 1) & 1) ? p1 : p0, d, e, tau, W, stream);
     } else {
         reg = false;
         BSQ_HIP(hipMemcpyAsync(W, G, static_cast<size_t>(k) * k * sizeof(double), hipMemcpyDeviceToDevice, stream));

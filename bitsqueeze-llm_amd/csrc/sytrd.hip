@@ -12,7 +12,16 @@
 //   4. w = tau p - (tau^2 / 2) (v^T A v) v, then A -= v w^T + w v^T.
 // Four workgroup barriers per step; blocks left of column j are skipped
 // (v vanishes there).  Output: d, e, tau and the reflectors row-wise,
-// H[j][i] = v_j[i] (zero for i <= j, one at i = j + 1).
+// H[j][i] = v_j[i] (one at i = j + 1; entries i <= j are not read).
+//
+// For 256 < k <= 512 it reduces the trailing 256 columns of a matrix whose
+// first k - 256 columns went one launch each (trd_step_kernel), applying that
+// kernel's last, pending update as it loads: a column costs 2.7 us here and
+// 5.5 us and a launch gap there (rank 512 of 1500 x 1500, a whole round trip
+// 5245 -> 4680 us, rank 300 of 700 x 800 3440 -> 2850 with the shorter
+// products).  At NB = 8 the loop over block columns stays rolled and the
+// tiles lie in the L1 / L2 caches: unrolled they fit the registers but for
+// five, and a 256-column reduction took 780 us against 690.
 #include "bsq_internal.hpp"
 #include "wave_ops.hpp"
 
@@ -28,8 +37,12 @@ __device__ __forceinline__ int opaque(int v) {
     return v;
 }
 
-template <int NB>
-__global__ __launch_bounds__(kTrdThreads) void sytrd_blocked_kernel(const double *__restrict__ G, int k,
+// PENDING: G and H have leading dimension `pitch` (k otherwise), the row of H before its first
+// and tau[-1] hold a reflector whose p (its matrix times v) is given, with the
+// update A -= v w^T + w v^T still to be applied to G.
+template <int NB, bool PENDING>
+__global__ __launch_bounds__(kTrdThreads) void sytrd_blocked_kernel(const double *__restrict__ G, int pitch, int k,
+                                                                     const double *__restrict__ p,
                                                                      double *__restrict__ d, double *__restrict__ e,
                                                                      double *__restrict__ tau,
                                                                      double *__restrict__ H) {
@@ -42,6 +55,7 @@ __global__ __launch_bounds__(kTrdThreads) void sytrd_blocked_kernel(const double
     __shared__ double red[kTrdThreads / 64];
     __shared__ double s_tau;
 
+    const int ld = PENDING ? pitch : k;
     double r[NE];
     {
         const int tid = threadIdx.x, tx = tid & 31, ty = tid >> 5;
@@ -52,9 +66,31 @@ __global__ __launch_bounds__(kTrdThreads) void sytrd_blocked_kernel(const double
                 // branch-free: G inside (both triangles of the diagonal blocks), 0 in the padding
                 const int i = a * 32 + ty, c = b * 32 + tx;
                 const bool inside = (i < k) && (c < k);
-                const double g = G[inside ? static_cast<uint64_t>(i) * k + c : 0];
+                const double g = G[inside ? static_cast<uint64_t>(i) * ld + c : 0];
                 r[tri(a, b)] = inside ? g : 0.0;
             }
+        if constexpr (PENDING) {
+            // w = tau p - (tau^2 / 2) (p.v) v
+            const double *vp = H - ld;
+            const double tp = tau[-1];
+            const double vi = tid < k ? vp[tid] : 0.0, pi = tid < k ? p[tid] : 0.0;
+            const double part = wave_sum_dpp(vi * pi);
+            if ((tid & 63) == 0) red[tid >> 6] = part;
+            __syncthreads();
+            double pv = 0.0;
+#pragma unroll
+            for (int m = 0; m < (KP + 63) / 64; ++m) pv += red[m];
+            if (tid < KP) {
+                vs[tid] = vi;
+                ws[tid] = tp * pi - (0.5 * tp * tp * pv) * vi;
+            }
+            __syncthreads();
+#pragma unroll
+            for (int a = 0; a < NB; ++a)
+#pragma unroll
+                for (int b = 0; b <= a; ++b)
+                    r[tri(a, b)] -= vs[a * 32 + ty] * ws[b * 32 + tx] + ws[a * 32 + ty] * vs[b * 32 + tx];
+        }
     }
     const int steps = k - 2;  // reflectors j = 0 .. k-3
 #pragma unroll
@@ -96,7 +132,7 @@ __global__ __launch_bounds__(kTrdThreads) void sytrd_blocked_kernel(const double
                     if (i < KP) {
                         const double v = (i == j + 1) ? 1.0 : ((i > j + 1 && i < k) ? xs[i] * scal : 0.0);
                         vs[i] = v;
-                        if (i < k) H[static_cast<uint64_t>(j) * k + i] = v;
+                        if (i < k) H[static_cast<uint64_t>(j) * ld + i] = v;
                     }
                 }
                 if (lane == 0) {
@@ -198,7 +234,7 @@ __global__ __launch_bounds__(kTrdThreads) void sytrd_blocked_kernel(const double
 
 template <int NB>
 void sytrd_blocked(const double *G, int k, double *d, double *e, double *tau, double *H, hipStream_t stream) {
-    sytrd_blocked_kernel<NB><<<1, kTrdThreads, 0, stream>>>(G, k, d, e, tau, H);
+    sytrd_blocked_kernel<NB, false><<<1, kTrdThreads, 0, stream>>>(G, k, k, nullptr, d, e, tau, H);
     BSQ_HIP(hipGetLastError());
 }
 
@@ -219,6 +255,19 @@ void launch_sytrd_blocked(const double *G, int k, double *d, double *e, double *
         case 7: sytrd_blocked<7>(G, k, d, e, tau, H, stream); break;
         default: sytrd_blocked<8>(G, k, d, e, tau, H, stream); break;
     }
+}
+
+// The rest of a reduction whose first j0 = k - 256 reflectors are done, the last
+// one's update pending: A (k x k) holds the trailing block with the updates
+// before it, p that reflector's product (indexed as A's rows).
+void launch_sytrd_tail(const double *A, int k, const double *p, double *d, double *e, double *tau, double *H,
+                       hipStream_t stream) {
+    BSQ_REQUIRE(k > 256 && A && p && H, "sytrd tail: bad arguments");
+    const int j0 = k - 256;
+    const size_t at = static_cast<size_t>(j0) * k + j0;
+    sytrd_blocked_kernel<8, true><<<1, kTrdThreads, 0, stream>>>(A + at, k, 256, p + j0, d + j0, e + j0, tau + j0,
+                                                                 H + at);
+    BSQ_HIP(hipGetLastError());
 }
 
 }  // namespace bsq

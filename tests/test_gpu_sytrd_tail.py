@@ -1,0 +1,30 @@
+"""The tridiagonalisation's hand-over above rank 256: the first k - 256 columns
+by one launch each, the last 256 in the register kernel (sytrd.hip), through
+bsq_svd_lowrank against the FP64 oracle with the same sketch.
+
+Sizes: the smallest hand-over (one and two columns, either parity of the
+double-buffered product), one in the middle, and the largest.  Tolerance as
+for the range finder's products: 2 niter + 2 FP32-accurate products of up to
+700 terms (2^-24 sqrt(700) = 1.6e-6 each) with the orthonormalisations
+between, 2e-5."""
+import numpy as np
+import pytest
+
+import bitsqz_amd as B
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("rank", [96, 600])  # a singular Gram matrix, and a regular one
+@pytest.mark.parametrize("q", [257, 258, 385, 511, 512])
+def test_hand_over(q, rank):
+    rng = np.random.default_rng(q + rank)
+    a = rng.standard_normal((700, rank)) * np.arange(1, rank + 1) ** -0.7
+    A = (a @ rng.standard_normal((rank, 600))).astype(np.float32)
+    U, S, V = B.svd_lowrank(A, q, 1)
+    R = B.gaussian(600 * q, 1241).reshape(600, q)
+    Uo, So, Vo = O.svd_lowrank(A, q, 1, R)
+    got, ref = O.reconstruct(U, S, V), O.reconstruct(Uo, So, Vo)
+    assert np.linalg.norm(got - ref) <= 2e-5 * np.linalg.norm(ref)
+    assert np.linalg.norm(S - So) <= 2e-5 * np.linalg.norm(So)
