@@ -15,40 +15,35 @@
 
 namespace bsq {
 
-// FP8 E4M3 encode exactly as quantization_cuda.cu:64-109 writes it.
-__device__ __forceinline__ uint32_t e4m3_encode(float value) {
-    if (!__builtin_isfinite(value)) value = (value < 0.0f) ? -kE4M3Max : kE4M3Max;
-    const uint32_t sign = __builtin_signbit(value) ? 1u : 0u;
-    float a = fabsf(value);
-    if (a == 0.0f) return sign << 7;
-    if (a > kE4M3Max) a = kE4M3Max;
-    int e2 = 0;
-    const float mant = frexpf(a, &e2);
-    int ef = e2 - 1 + 7;
-    if (ef <= 0) {
-        int mf = static_cast<int>(rintf(a * 512.0f));
-        if (mf > 7) mf = 7;
-        return (sign << 7) | static_cast<uint32_t>(mf & 7);
-    }
-    int mf = static_cast<int>(rintf(((mant * 2.0f) - 1.0f) * 8.0f));
-    if (mf > 7) {
-        mf = 0;
-        ef += 1;
-    }
-    if (ef >= 16) {
-        ef = 15;
-        mf = 7;
-    }
-    return (sign << 7) | (static_cast<uint32_t>(ef & 15) << 3) | static_cast<uint32_t>(mf & 7);
+// The value whose conversion to E4M3 (round to nearest even) is the code of
+// quantization_cuda.cu:64-109: +-448 at most (NaN and infinities included, NaN
+// positive), and below the normal range (2^-6) at most the largest subnormal
+// 7 / 512, as the code's mantissa is clamped at 7 there.
+__device__ __forceinline__ float e4m3_operand(float value) {
+    const float w = fmaxf(fminf(value, kE4M3Max), -kE4M3Max);  // fminf takes NaN to 448
+    constexpr float kMinNormal = 0.015625f, kMaxSub = 0.013671875f;
+    return fabsf(w) < kMinNormal ? __builtin_amdgcn_fmed3f(w, -kMaxSub, kMaxSub) : w;
 }
 
-// FP8 E4M3 decode (quantization_cuda.cu:111-128); 0x7F decodes to 480.
+// FP8 E4M3 encode exactly as quantization_cuda.cu:64-109 writes it, on the
+// converter (v_cvt_pk_fp8_f32); 25 instructions a value with frexp and rint,
+// six here.
+__device__ __forceinline__ uint32_t e4m3_encode(float value) {
+    const float w = e4m3_operand(value);
+    return static_cast<uint32_t>(__builtin_amdgcn_cvt_pk_fp8_f32(w, w, 0, false)) & 0xFFu;
+}
+
+// four codes, the first in the low byte
+__device__ __forceinline__ uint32_t e4m3_encode4(float a, float b, float c, float d) {
+    const int lo = __builtin_amdgcn_cvt_pk_fp8_f32(e4m3_operand(a), e4m3_operand(b), 0, false);
+    return static_cast<uint32_t>(__builtin_amdgcn_cvt_pk_fp8_f32(e4m3_operand(c), e4m3_operand(d), lo, true));
+}
+
+// FP8 E4M3 decode (quantization_cuda.cu:111-128); 0x7F decodes to 480.  The
+// code's exponent and mantissa read as FP32's are 2^-120 of the value, with
+// subnormals for subnormals.
 __device__ __forceinline__ float e4m3_decode(uint32_t v) {
-    const uint32_t ef = (v >> 3) & 15u, mf = v & 7u;
-    float r;
-    if (ef == 0) r = (static_cast<float>(mf) / 8.0f) * 0.015625f;  // 2^(1-7)
-    else r = (1.0f + static_cast<float>(mf) / 8.0f) * __builtin_ldexpf(1.0f, static_cast<int>(ef) - 7);
-    return (v & 0x80u) ? -r : r;
+    return __uint_as_float(static_cast<uint32_t>(static_cast<int32_t>(v << 24) >> 4) & 0x87F00000u) * 0x1.0p120f;
 }
 
 }  // namespace bsq
