@@ -16,9 +16,10 @@ figure of the dominant kernel and the reference's CPU codec timed on this
 host.  For the HOST-input workload (c5) the lanes' figure is device-resident
 like the others, and `host_input_step` adds the H2D to a single-lane step.
 
-Dominant kernel: on the SVD workloads, the FP32-MFMA GEMMs that touch the
+Dominant kernel: on the SVD workloads, the matrix-core GEMMs that touch the
 full matrix (the range finder's 2 + 2 it products and the low-rank
-reconstructions, 2 * rows * cols * rank flops each); on the direct
+reconstructions, 2 * rows * cols * rank flops each, every FP32 product as
+three f16 ones, so the peak is a third of the dense f16 rate); on the direct
 workloads, the HBM-bound stage with the largest time per step (outlier
 separation, direct encode, error top-k or direct decode), at its
 algorithmic bytes.  Every one of them is bracketed with HIP events on the
@@ -53,7 +54,8 @@ import bitsqz_amd as B  # noqa: E402
 
 METRIC = "compress+decompress GB/s (FP32 in) at 4096×11008; % HBM/MFMA roofline"
 HBM_PEAK_GBS = 8000.0
-FP32_MFMA_PEAK_TFLOPS = 157.3
+F16_MFMA_PEAK_TFLOPS = 2500.0
+SPLIT_PEAK_TFLOPS = round(F16_MFMA_PEAK_TFLOPS / 3, 1)  # FP32 products as three f16 products
 
 # name -> (rows, cols, outlier ratio, error ratio, svd_ranks, svd_niters, uv, s, direct, generator, input)
 # generator: "normal", "outlier_cols", or ("lowrank", rank, decay, noise std, outlier columns, their scale)
@@ -176,13 +178,15 @@ def committed_traffic(workload: str, cls: str):
 
 
 def roofline_time_ms(rows, cols, svd, nit, q, err_on, payload_bytes):
-    """T_roof of the whole step: MFMA time of the GEMMs over the m x n matrix
-    (2 N q (2 + 2 it) + 2 N q (1 + [error top-k])) for the SVD path, HBM time
-    of 8N + 2P bytes for the direct path."""
+    """T_roof of the whole step: for the SVD path the matrix-core time of the
+    GEMMs over the m x n matrix (2 + 2 it products and 1 + [error top-k]
+    reconstructions of 2 N q flops each, three f16 products an FP32 one) or the
+    HBM time of the matrix in each of them where that is longer; HBM time of
+    8N + 2P bytes for the direct path."""
     n = rows * cols
     if svd >= 1:
-        flops = 2.0 * n * q * (2 + 2 * nit) + 2.0 * n * q * (1 + (1 if err_on else 0))
-        return flops / (FP32_MFMA_PEAK_TFLOPS * 1e12) * 1e3
+        gemm, matrix = 2.0 * n * q / (SPLIT_PEAK_TFLOPS * 1e12), 4.0 * n / (HBM_PEAK_GBS * 1e9)
+        return ((2 + 2 * nit + 1) * max(gemm, matrix) + (max(gemm, 2 * matrix) if err_on else 0.0)) * 1e3
     return (8.0 * n + 2.0 * payload_bytes) / (HBM_PEAK_GBS * 1e9) * 1e3
 
 
@@ -521,7 +525,7 @@ def main():
             e.update({"alg_bytes": alg[name], "gbs": round(gbs, 1), "frac_hbm": round(gbs / HBM_PEAK_GBS, 4)})
         else:
             tf = 2.0 * n * q / (avg * 1e-3) / 1e12
-            e.update({"alg_flops": 2.0 * n * q, "tflops": round(tf, 2), "frac_mfma": round(tf / FP32_MFMA_PEAK_TFLOPS, 4)})
+            e.update({"alg_flops": 2.0 * n * q, "tflops": round(tf, 2), "frac_mfma": round(tf / SPLIT_PEAK_TFLOPS, 4)})
         by_class[name] = e
 
     if svd >= 1:
@@ -534,13 +538,12 @@ def main():
         kflops = 2.0 * rows * cols * q
         achieved = kflops / (kms * 1e-3) / 1e12
         traffic, tsrc = committed_traffic(args.workload, "gemm_mxn")
-        roofline = {"bound": "mfma", "achieved": round(achieved, 2), "peak": FP32_MFMA_PEAK_TFLOPS,
-                    "unit": "TFLOP/s", "frac": round(achieved / FP32_MFMA_PEAK_TFLOPS, 4),
+        roofline = {"bound": "mfma", "achieved": round(achieved, 2), "peak": SPLIT_PEAK_TFLOPS,
+                    "unit": "TFLOP/s", "frac": round(achieved / SPLIT_PEAK_TFLOPS, 4),
                     "traffic": traffic, "traffic_source": tsrc,
-                    "kernel": "the FP32-MFMA GEMMs over the m x n matrix: range finder A_w B (gemm_dma_kernel, "
-                              "split-K + splitk_reduce_kernel) and A_w^T B (gemm_streamk_kernel + "
-                              "streamk_reduce_kernel), reconstructions U diag(S) V^T (gemm_dma_kernel RECON on "
-                              "the compress side, recon_q_kernel from the packed factors on the decompress side)",
+                    "kernel": "the GEMMs over the m x n matrix, FP32 values as two f16 pieces: range finder A_w B and "
+                              "A_w^T B (gemm_h2_kernel + h2_reduce_kernel, split_b_kernel), reconstructions "
+                              "U diag(S) V^T (factor_planes_kernel + recon_planes_kernel)",
                     "avg_ms": round(kms, 5), "launches": launches, "alg_flops": kflops, "by_class": by_class}
     else:
         hbm = {k: v for k, v in by_class.items() if k in alg}
