@@ -206,6 +206,7 @@ __global__ __launch_bounds__(kThreads) void topk_select_kernel(TopkArgs a) {
         sh.kt = 0;
         sh.kth = 0;
     }
+    if (a.flags_reset && r == 0 && threadIdx.x == 0) *a.flags_reset = 0u;
     float dq = 1.0f;
     if constexpr (SRC == TopkSource::DenseMinusNF4DQ) {
         dq = *a.dq;
@@ -1237,7 +1238,9 @@ bool launch_topk_select(const TopkArgs &args, hipStream_t stream) {
     BSQ_REQUIRE(a.k >= 1 && a.k <= a.cols, "top-k: k must be in [1, cols]");
     BSQ_REQUIRE(a.a && a.indices && a.values, "top-k: null pointer");
     BSQ_REQUIRE(!(a.flags_reset && a.flags), "top-k: a pass that sets the flags word cannot also clear it");
-    if (a.flags_reset && !reg) {
+    // the row kernels clear the word themselves (a fill launch took 3.7 us of a
+    // 49 us round trip of 1000 x 5003); the bands beyond kTopkMaxK do not
+    if (a.flags_reset && a.k > kTopkMaxK) {
         BSQ_HIP(hipMemsetAsync(a.flags_reset, 0, sizeof(uint32_t), stream));
         a.flags_reset = nullptr;
     }
