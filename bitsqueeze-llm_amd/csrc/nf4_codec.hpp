@@ -56,12 +56,14 @@ __device__ __forceinline__ uint32_t nf4_code_scan_inline(const float *L, float v
 // thresholds are 0.081 apart).  Every threshold is at least 1.6e-3 from a bin
 // edge, while the bin index floor((v + 1) * 16), computed in FP32 with one
 // rounding or two, is off by one only for v within 1.2e-7 of an edge, where
-// the count is the same on both sides; v in (-2, -1] takes bin 0.  |v| >= 2
-// and non-finite v take the scan.  Exhaustively checked against the scan over
-// all 2^32 floats by the GPU test suite.  So few bins span one and a half
+// the count is the same on both sides; v in (-2, -1] takes bin 0, and the
+// largest v below 2 rounds up to bin 48, which holds code 15 as the bins
+// before it do.  |v| >= 2 and non-finite v take the scan.  Both forms of the
+// bin are checked exhaustively against the scan over all 2^32 floats by the
+// GPU test suite.  So few bins span one and a half
 // rounds of the LDS banks: 384 bins of 1/128 took 93 us against 85 in the
 // fused encode and top-k pass of 4096 x 11008 (with its other changes).
-constexpr int kNf4PerUnit = 16, kNf4Bins = 3 * kNf4PerUnit;
+constexpr int kNf4PerUnit = 16, kNf4Bins = 3 * kNf4PerUnit + 1;
 struct Nf4Table {
     uint2 ent[kNf4Bins];  // (bits of the threshold inside bin b, code_lo): one 8-byte read
 };
@@ -96,14 +98,20 @@ __device__ __forceinline__ uint32_t nf4_code_small(const Nf4Table &t, float v) {
     return e.y + ((v >= __uint_as_float(e.x)) ? 1u : 0u);
 }
 
-// bin of x inv, given inv_bins = kNf4PerUnit inv: one FMA and one conversion
-// (which takes negative values and NaN to 0).  |x inv| < 2, so the bin is
-// below kNf4Bins.
+// bin of x inv, |x inv| < 2, given inv_bins = kNf4PerUnit inv: one FMA and one
+// conversion (which takes negative values and NaN to 0).  The sum rounds to
+// 3 kNf4PerUnit at most, the table's last entry.
 __device__ __forceinline__ uint32_t nf4_bin(float x, float inv_bins) {
     const float t = __builtin_fmaf(x, inv_bins, static_cast<float>(kNf4PerUnit));
     uint32_t b;
     asm("v_cvt_u32_f32 %0, %1" : "=v"(b) : "v"(t));
     return b;
+}
+
+// code of x inv, |x inv| < 2 (NaN: 0)
+__device__ __forceinline__ uint32_t nf4_code_binned(const Nf4Table &t, float x, float inv, float inv_bins) {
+    const uint2 e = t.ent[nf4_bin(x, inv_bins)];
+    return e.y + ((x * inv >= __uint_as_float(e.x)) ? 1u : 0u);
 }
 
 // Largest magnitude of v[0 .. N), and whether any of them is NaN; infinities

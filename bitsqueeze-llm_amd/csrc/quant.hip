@@ -288,11 +288,8 @@ __global__ __launch_bounds__(kThreads) void quant_encode_kernel(
 #pragma unroll
                 for (int j = 3; j >= 0; --j)  // byte j = code(2 j) << 4 | code(2 j + 1)
 #pragma unroll
-                    for (int h = 0; h < 2; ++h) {
-                        const float y = v[u][2 * j + h];
-                        const uint2 e = tab.ent[nf4_bin(y, inv_bins)];
-                        word = (word << 4) | (e.y + ((y * inv[u] >= __uint_as_float(e.x)) ? 1u : 0u));
-                    }
+                    for (int h = 0; h < 2; ++h)
+                        word = (word << 4) | nf4_code_binned(tab, v[u][2 * j + h], inv[u], inv_bins);
                 uint8_t *out = codes + 4 * (chunk0 + u * kThreads);
                 if (vec_ok) {  // uniform
                     *reinterpret_cast<uint32_t *>(out) = word;
@@ -521,10 +518,13 @@ __global__ __launch_bounds__(kThreads) void nf4_code_sweep_kernel(uint64_t lo, u
     for (uint64_t p = lo + static_cast<uint64_t>(blockIdx.x) * kThreads + threadIdx.x; p < hi;
          p += static_cast<uint64_t>(gridDim.x) * kThreads) {
         const uint32_t bits = static_cast<uint32_t>(p);
-        const uint32_t c = nf4_code(tab, __uint_as_float(bits));
+        const float v = __uint_as_float(bits);
+        const uint32_t c = nf4_code(tab, v);
 #pragma unroll
         for (int i = 0; i < 16; ++i) hl[i] += (c == static_cast<uint32_t>(i)) ? 1u : 0u;
-        cs += static_cast<unsigned long long>(c) * (bits % 65521u);
+        // the histogram is nf4_code's, the checksum the encoders' form where they use it
+        const uint32_t cb = fabsf(v) < 2.0f ? nf4_code_binned(tab, v, 1.0f, static_cast<float>(kNf4PerUnit)) : c;
+        cs += static_cast<unsigned long long>(cb) * (bits % 65521u);
     }
 #pragma unroll
     for (int i = 0; i < 16; ++i) atomicAdd(&h[i], hl[i]);

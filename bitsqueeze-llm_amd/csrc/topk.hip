@@ -708,8 +708,7 @@ __global__ __launch_bounds__(kThreads) void topk_reg_kernel(TopkArgs a) {
 #pragma unroll
                 for (int h = 0; h < 4; ++h) {
                     const int u = h ^ 2;
-                    const uint2 e = etab.ent[nf4_bin(v[m][u], inv_bins)];
-                    const uint32_t c = e.y + ((v[m][u] * inv >= __uint_as_float(e.x)) ? 1u : 0u);
+                    const uint32_t c = nf4_code_binned(etab, v[m][u], inv, inv_bins);
                     packed = (packed << 4) | c;
                     v[m][u] = v[m][u] - scale * sh.L[c];
                     // the error is formed here: left to the compiler, the

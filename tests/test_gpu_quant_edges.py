@@ -72,3 +72,40 @@ def test_encode_unaligned_input(method):
     B.check(B.lib().bsq_stream_synchronize(None), "sync")
     scales = sf.download(np.float32, nb) if method == B.NF4 else su.download(np.uint8, nb)
     check(x, method, (scales, c.download(np.uint8, (n + 1) // 2), float(dq.download(np.float32, 1)[0])))
+
+
+def below_two(rows, cols):
+    """Rows whose blocks of 64 hold values up to the float below 2 at an NF4_DQ
+    block scale of 1 (a scale code of 0 under the large value of row 0): the
+    largest the code table takes, whose sum with the bin offset rounds up to
+    the table's end.  Every third block also reaches 2, which the scan takes."""
+    top = np.nextafter(np.float32(2.0), np.float32(0.0))
+    v = np.array([top, -top, np.nextafter(top, np.float32(0.0)), 1.9375, 1.0, 0.5, -1.0, 0.0], np.float32)
+    x = np.tile(v, rows * cols // 8).reshape(rows, cols)
+    x[:, 64 * 2 + 5::192] = 2.0
+    x[0, 0] = 4e6
+    return x
+
+
+@pytest.mark.parametrize("rows", [1, 33, 1 << 15])  # one chunk a lane, a tile's remainder, four chunks a lane
+def test_encode_largest_table_value(rows):
+    x = below_two(rows, 512).ravel()
+    check(x, B.NF4_DQ, B.quant_compress(x, B.NF4_DQ))
+
+
+@pytest.mark.parametrize("outlier", [0.0, 0.004])  # with the separation: its bitmap and row maxima
+@pytest.mark.parametrize("cols", [512, 4096])
+def test_fused_encode_largest_table_value(cols, outlier):
+    rows = 36
+    x = below_two(rows, cols)
+    if outlier:
+        x[:, : B.topk_num_columns(cols, outlier) + 1] = 5e6  # one a row stays and sets the global scale
+    B.compress_release()
+    B.check(B.compress_initialize(rows, cols, outlier, 0.01, -1, 1, B.QUANT_NONE, B.QUANT_NONE, B.NF4_DQ,
+                                  B.INPUT_HOST), "init")
+    try:
+        data = B.compress(x)
+    finally:
+        B.compress_release()
+    cfg = O.Config(rows, cols, outlier, 0.01, -1, 1, O.QUANT_NONE, O.QUANT_NONE, O.NF4_DQ)
+    assert O.mask_pointer(data) == O.mask_pointer(O.compress(x, cfg).to_bytes())
