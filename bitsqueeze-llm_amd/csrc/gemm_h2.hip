@@ -135,6 +135,7 @@ __global__ __launch_bounds__(kThreads) void split_b_kernel(const float *__restri
     } else if (scaled) {
         em = *emax;
     }
+    if (kgroups == 0) return;  // the maximum alone (a caller's sketch): no planes, np is 0
     const int t = blockIdx.x * kThreads + threadIdx.x;
     const int kg = t / np, n = t - kg * np;
     if (kg >= kgroups) return;
