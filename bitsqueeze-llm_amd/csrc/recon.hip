@@ -263,7 +263,9 @@ __global__ __launch_bounds__(kThreads) void factor_planes_kernel(PlaneSource u, 
         dq = *p.dq;
         if (dq == 0.0f || !__builtin_isfinite(dq)) dq = 1.0f;
     }
-    const bool quick = k % 8 == 0;  // a group of eight in one 64-element block, its codes in one aligned word
+    // a group of eight in one 64-element block, its codes in one aligned word
+    // (a caller's code arrays may start at any byte)
+    const bool quick = k % 8 == 0 && (reinterpret_cast<uintptr_t>(p.codes) & 3u) == 0;
     auto values = [&](int kg, float (&x)[8]) {
         const int k0 = 8 * kg;
         const uint64_t e0 = base + k0;
