@@ -300,6 +300,9 @@ struct Runtime {
     Meta *meta = nullptr;
     SvdPlan *svd = nullptr;
     uint8_t *planes = nullptr;      // the factors' pieces (launch_reconstruct_planes)
+    // decompress: the stream whose work last used the planes and the decoded
+    // factors, or null (see order_factor_buffers)
+    hipStream_t factor_stream = nullptr;
     const float *sketch = nullptr;  // injected Gaussian sketch (test hook)
     // decompress-side staging for quantised sections (shared, like the reference's buffers)
     float *q_scales_f32 = nullptr;
@@ -917,6 +920,22 @@ void decompress_device(Runtime &rt, const bsq_device_packed_t &P, const bool has
                         true, st, err_gate);
 }
 
+// The decompress runtime has one set of decoded factors and planes and two
+// streams that use them: a device-resident decode runs on the compress
+// runtime's stream while one exists, a host object's on its own.  Work on `st`
+// that writes them waits for what another stream has in flight.  The event is
+// recorded here, when the other stream is known to have been used, so decodes
+// that stay on one stream record none.
+void order_factor_buffers(Runtime &rt, hipStream_t st) {
+    const hipStream_t other = rt.factor_stream;
+    rt.factor_stream = st;
+    if (!other || other == st) return;
+    // a compress stream that is gone was drained before it was destroyed
+    if (other != rt.stream && !(g_comp.initialized && g_comp.stream == other)) return;
+    BSQ_HIP(hipEventRecord(rt.cev[0], other));
+    BSQ_HIP(hipStreamWaitEvent(st, rt.cev[0], 0));
+}
+
 // True when some index of the host top-k blob at `p` (num_topk_columns per
 // row) is >= cols.  Such an index addresses a later row in the reference's
 // scatter (topk_cuda_utils.cuh:132-149), which the row-local fused scatter
@@ -1280,6 +1299,7 @@ void decompress_host(Runtime &rt, const bitsqz_llm_array_t *c, float *d_dst) {
         P.d_dense[i] = dense_dst;
     };
     if (c->flags & kFlagSvd) {
+        order_factor_buffers(rt, st);
         const uint16_t q = static_cast<uint16_t>(c->effective_rank);
         stage_section(SEC_U, c->section_u, c->svd_uv_format, static_cast<uint64_t>(rows) * q, rt.sec[SEC_U].dense);
         stage_section(SEC_S, c->section_s, c->svd_s_format, q, rt.sec[SEC_S].dense);
@@ -1581,6 +1601,7 @@ int bsq_device_decompress(const bsq_device_packed_t *packed, float *d_dst, uint3
                         "rank mismatch with the decompress runtime");
         }
         const hipStream_t st = g_comp.initialized ? g_comp.stream : g_decomp.stream;
+        if (H.flags & kFlagSvd) order_factor_buffers(g_decomp, st);
         // the error section is present iff the device flags word says so: the
         // scatter reads it on the device, so pass the full k and let the
         // kernel gate on the flag (no host synchronisation)
