@@ -196,7 +196,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     constexpr int kPitchA = T + 2;  // 16-byte units per k group of a staged A plane: +2 spreads the writes' banks
     __shared__ u32x4 a0[2 * KG * kPitchA], a1[2 * KG * kPitchA];  // h plane, l plane
     __shared__ __attribute__((aligned(1024))) u32x4 b0[2 * KG * T], b1[2 * KG * T];
-    constexpr int kLoadsA = TA ? 18 : 6;  // vector loads of one A slice and its scales, at least
+    // vector loads of one A slice's values, at least: 16 bytes are the widest
+    // (64 bytes a lane of each of two rows), and 16 rows of A^T are a runtime
+    // stride apart.  Their addresses differ by lane, so none is a scalar load.
+    constexpr int kLoadsA = TA ? 16 : 4;
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm0 = (wave >> 1) * 64, wn0 = (wave & 1) * 64;
@@ -226,7 +229,17 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 
     float va[2][8];  // A values in flight
     float vs[TA ? 8 : 2];
-    auto load_a = [&]() __attribute__((always_inline)) {
+    // the scales of the next A slice: where the wait has no loads to spare
+    // they go out before the B transfers (with A^T their registers are not to
+    // be had that early: it spilled)
+    auto load_scales = [&]() __attribute__((always_inline)) {
+        asm volatile("" ::: "memory");
+        if constexpr (!TA) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) vs[h] = g.rs[min(ca.tm * T + 64 * h + (tid >> 2), g.M - 1)];
+        }
+    };
+    auto load_values = [&]() __attribute__((always_inline)) {
         const int m0 = ca.tm * T, k0 = ca.ks * BK;
         asm volatile("" ::: "memory");  // stays behind the DMA before it
         if constexpr (!TA) {
@@ -234,7 +247,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 const int r = min(m0 + 64 * h + (tid >> 2), g.M - 1);
-                vs[h] = g.rs[r];
                 // past K: the row's last eight values, which meet a partial
                 // group of B turned to fit them (H2Planes), or zeros
                 // rows may start at any multiple of four bytes
@@ -336,17 +348,20 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         Frags f0, f1;
         fetch(f0, ac, bc, 0);
         stage_a(an);
+        load_scales();
         dma_b(bn);
-        load_a();
+        load_values();
         fetch(f1, ac, bc, 1);
         acc.multiply(f0);
         acc.multiply(f1);
     };
     if (n <= 0 || range >= g.ranges) return;  // uniform (ranges <= units and grid = ranges x tiles_n: does not occur)
-    load_a();
+    load_scales();
+    load_values();
     dma_b(b0);
     stage_a(a0);
-    load_a();
+    load_scales();
+    load_values();
     int left = n, c_pr = p0 - tile0 * g.pairs;
     for (int t = tile0; left > 0; ++t, c_pr = 0) {  // the range's tile rows
         const int here = min(g.pairs - c_pr, left);
