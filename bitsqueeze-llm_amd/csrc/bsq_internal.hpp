@@ -244,9 +244,9 @@ void svd_run(SvdPlan *plan, const float *A, const float *sketch, uint64_t seed, 
 // `minuend` is not null (recon.hip).
 void launch_reconstruct(const float *U, const float *S, const float *V, int m, int n, int k,
                         const float *minuend, float *out, hipStream_t stream);
-// The same bits with scratch of factor_plane_bytes (16-byte aligned) and each
-// factor in FP32 (dense) or as NF4 / NF4_DQ codes with their block scales (and
-// NF4_DQ's global scale); ranks from 32.
+// The same bits with scratch of factor_plane_bytes (16-byte aligned; none for
+// small matrices of low rank) and each factor in FP32 (dense) or as NF4 / NF4_DQ codes with their
+// block scales (and NF4_DQ's global scale).
 struct FactorSource {
     const float *dense = nullptr;
     const uint8_t *codes = nullptr;
@@ -254,7 +254,6 @@ struct FactorSource {
     const uint8_t *scales_u8 = nullptr;
     const float *dq = nullptr;
 };
-bool reconstruct_planes_supported(int k);
 uint64_t factor_plane_bytes(int m, int n, int k);
 void launch_reconstruct_planes(const FactorSource &U, const float *S, const FactorSource &V, int m, int n, int k,
                                const float *minuend, float *out, void *planes, hipStream_t stream);

@@ -3,11 +3,13 @@
 // (reference modules/reconstruct_lowrank_cuda/src/reconstruct_lowrank_cuda.cu:
 // 21-62, 120-171; the subtraction of src/bitsqz_llm.cu:1141-1163).
 //
-// Each 128 x 128 tile of the output is one workgroup.  The rows of U diag(S)
-// and of V are scaled by powers of two that bring their largest magnitude into
-// [2^14, 2^15), and the tile leaves scaled back, straight from the
-// accumulators: 32 lanes write 128 contiguous bytes of a row.  Two forms, with
-// the same pieces summed in the same order, so with the same results:
+// At low ranks recon_low_rank_kernel sums in FP32 (low_rank_form, with the
+// rule's reason).  Else each 128 x 128 tile of the output is one workgroup.  The
+// rows of U diag(S) and of V are scaled by powers of two that bring their
+// largest magnitude into [2^14, 2^15), and the tile leaves scaled back, straight
+// from the accumulators: 32 lanes write 128 contiguous bytes of a row.  Two
+// forms, with the same pieces summed in the same order, so with the same
+// results:
 //   recon_planes_kernel  where the caller has room for the pieces
 //                        (FactorPlanes): factor_planes_kernel splits each
 //                        factor once, from FP32 or straight from its NF4 /
@@ -27,6 +29,8 @@
 #include "h2_split.hpp"
 #include "scalar_codecs.hpp"
 #include "tile_map.hpp"
+
+#include <type_traits>
 
 namespace bsq {
 namespace {
@@ -49,8 +53,26 @@ __device__ __forceinline__ int factor_exponent(uint32_t bits) {
 // scale of a row: its largest magnitude to [2^14, 2^15)
 __device__ __forceinline__ float factor_scale(int e) { return pow2(14 - min(e, 127)); }
 
-// eight values of a row from k on (rows may start at any multiple of four
-// bytes), zero past the row's end
+// Values k .. k + 3 of a row of K >= 4 (which may start at any multiple of four
+// bytes), zero past its end, in two steps: the load, at the last four values
+// where those lie past the end, and (once loads of other rows are out too) the
+// turn to their places.  Guarded loads wait one for another: a ragged last
+// slice by them took 4 us more at any size.
+__device__ __forceinline__ void load_row4(const float *row, int k, int K, float (&v)[4]) {
+    __builtin_memcpy(&v[0], __builtin_assume_aligned(row + min(k, K - 4), 4), 16);
+}
+__device__ __forceinline__ void turn_row4(int k, int K, float (&v)[4]) {
+    const int past = max(k - (K - 4), 0);
+    if (past & 1) {
+        v[0] = v[1], v[1] = v[2], v[2] = v[3], v[3] = 0.0f;
+    }
+    if (past & 2) {
+        v[0] = v[2], v[1] = v[3], v[2] = v[3] = 0.0f;
+    }
+    if (past >= 4) v[0] = v[1] = v[2] = v[3] = 0.0f;
+}
+
+// eight values of a row from k on, zero past the row's end
 __device__ __forceinline__ void load_row8(const float *row, int k, int K, float (&v)[8]) {
     if (k + 8 <= K) {
         __builtin_memcpy(&v[0], __builtin_assume_aligned(row + k, 4), 32);
@@ -133,10 +155,38 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
             for (int h = 0; h < 4; ++h) __builtin_memcpy(&v[h][0], __builtin_assume_aligned(rows[h] + k, 4), 32);
             __builtin_memcpy(&s8[0], __builtin_assume_aligned(g.S + k, 4), 32);
+        } else if (g.k % 4 == 0) {  // uniform
+            // clamped quads and selected zeros (guarded loads wait one for
+            // another: 4 us more at any size)
+#pragma unroll
+            for (int c = 0; c < 8; c += 4) {
+                const int kc = min(k + c, g.k - 4);
+#pragma unroll
+                for (int h = 0; h < 4; ++h) __builtin_memcpy(&v[h][c], __builtin_assume_aligned(rows[h] + kc, 4), 16);
+                __builtin_memcpy(&s8[c], __builtin_assume_aligned(g.S + kc, 4), 16);
+            }
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const bool past = k + (i & 4) >= g.k;
+#pragma unroll
+                for (int h = 0; h < 4; ++h) v[h][i] = past ? 0.0f : v[h][i];
+                s8[i] = past ? 0.0f : s8[i];
+            }
         } else {
 #pragma unroll
-            for (int h = 0; h < 4; ++h) load_row8(rows[h], k, g.k, v[h]);
-            load_row8(g.S, k, g.k, s8);
+            for (int i = 0; i < 8; ++i) {
+                const int kc = min(k + i, g.k - 1);
+#pragma unroll
+                for (int h = 0; h < 4; ++h) v[h][i] = rows[h][kc];
+                s8[i] = g.S[kc];
+            }
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const bool past = k + i >= g.k;
+#pragma unroll
+                for (int h = 0; h < 4; ++h) v[h][i] = past ? 0.0f : v[h][i];
+                s8[i] = past ? 0.0f : s8[i];
+            }
         }
     };
     uint32_t bits[4] = {0, 0, 0, 0};
@@ -434,62 +484,214 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         [&](int row, int t) { return factor_value(pl.v, row, t, g.k); });
 }
 
-// Ranks below 32: FP32 sums over k.  There the two pieces' own rounding (7e-8
-// of the result) is no smaller than an FP32 chain's, and a full slice would be
-// mostly padding.  64 x 64 tiles, 4 x 4 outputs a lane, the factors in LDS.
-__global__ __launch_bounds__(kThreads) void recon_low_rank_kernel(ReconArgs g) {
-    constexpr int TS = 64;
-    __shared__ float us[BK][TS + 4], vs[BK][TS + 4];
+// Low ranks on the FP32 matrix instructions: the whole of k is in LDS after one
+// round trip to memory, with packed factors decoded on the way, and a 64 x 64
+// tile goes out as 16-byte stores (V's rows are the instruction's rows, so a
+// lane holds four consecutive columns).  Small matrices are bound by that round
+// trip, large ones by the output's writes to about rank 32 and by the matrix
+// instructions above.  4-byte loads and guarded tails cost more than either:
+// every load and store of a tile inside the matrix is one of 16 bytes without a
+// branch of its own (8192 x 8192, rank 32 86 -> 60 us, rank 48 143 -> 81).
+// The order of the sums is that of gemm.hip's kernels: lane group kk takes
+// k = 16 s + 4 kk + t at step t of slice s.
+// QUADS: every quad of k is one load (ranks from four; of packed factors,
+// multiples of four, whose quads lie in one 64-element block), else by element.
+template <int KS, bool PACKED, bool SUB, bool QUADS>
+__global__ __launch_bounds__(kThreads) void recon_low_rank_kernel(ReconArgs g, PlaneSource u, PlaneSource v) {
+    constexpr int TS = 64, G = 4 * KS;  // quads of k per row
+    constexpr int KP = 16 * KS + 4, Q = TS * G / kThreads, F = TS / 32;
+    constexpr float Lc[16] = BSQ_NF4_LEVELS;
+    __shared__ __attribute__((aligned(16))) float us[TS][KP], vs[TS][KP];
+    __shared__ float levels[16];
     int tile_m, tile_n, z;
     xcd_tile(static_cast<int>(ceil_div(g.m, TS)), static_cast<int>(ceil_div(g.n, TS)), 1, tile_m, tile_n, z);
-    const int m0 = tile_m * TS, n0 = tile_n * TS, tid = threadIdx.x;
-    for (int e = tid; e < TS * g.k; e += kThreads) {
-        const int r = e / g.k, t = e - r * g.k;
-        us[t][r] = g.U[static_cast<uint64_t>(min(m0 + r, g.m - 1)) * g.k + t] * g.S[t];
-        vs[t][r] = g.V[static_cast<uint64_t>(min(n0 + r, g.n - 1)) * g.k + t];
+    const int m0 = tile_m * TS, n0 = tile_n * TS, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, K = g.k;
+    if constexpr (PACKED) {
+        if (tid < 16) levels[tid] = Lc[tid];
+        __syncthreads();
+    }
+    // the quads of a factor's rows from row r0 on; rows past the factor repeat
+    // its last one.  Quads that reach past k are loaded where they end at it
+    // and turned to their places by stage().
+    auto load = [&](const PlaneSource &p, int r0, float (&x)[Q][4]) __attribute__((always_inline)) {
+        const bool packed = PACKED && !p.dense;
+        float dq = 1.0f;
+        if (packed && p.scales_u8) {
+            dq = *p.dq;
+            if (dq == 0.0f || !__builtin_isfinite(dq)) dq = 1.0f;
+        }
+        const bool words = (reinterpret_cast<uintptr_t>(p.codes) & 1u) == 0;
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const int lin = tid + kThreads * q, k0 = 4 * (lin % G);
+            const uint64_t base = static_cast<uint64_t>(min(r0 + lin / G, p.rows - 1)) * K;
+            if (!packed && QUADS) {
+                load_row4(p.dense + base, k0, K, x[q]);
+            } else if (QUADS) {
+                const uint64_t e = base + min(k0, K - 4);
+                const uint8_t *c = p.codes + e / 2;
+                const uint32_t w = words ? *reinterpret_cast<const uint16_t *>(c) : c[0] | (c[1] << 8);
+                const float s = block_scale(p, e / kQuantBlock, dq);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) x[q][i] = s * levels[(w >> (8 * (i / 2) + (i % 2 ? 0 : 4))) & 15u];
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const uint64_t e = base + min(k0 + i, K - 1);
+                    if (!packed) {
+                        x[q][i] = p.dense[e];
+                    } else {
+                        const uint32_t byte = p.codes[e >> 1];
+                        x[q][i] = block_scale(p, e / kQuantBlock, dq) * levels[(e & 1) ? (byte & 15u) : (byte >> 4)];
+                    }
+                }
+            }
+        }
+    };
+    auto stage = [&](float (&x)[Q][4], float (*dst)[KP]) __attribute__((always_inline)) {
+        if (QUADS && K % 4 != 0) {  // uniform
+#pragma unroll
+            for (int q = 0; q < Q; ++q) turn_row4(4 * ((tid + kThreads * q) % G), K, x[q]);
+        }
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const int lin = tid + kThreads * q, k0 = 4 * (lin % G);
+            f32x4 y;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) y[i] = k0 + i < K ? x[q][i] : 0.0f;
+            *reinterpret_cast<f32x4 *>(&dst[lin / G][k0]) = y;
+        }
+    };
+    {
+        float xu[Q][4], xv[Q][4], xs[Q][4];
+        load(u, m0, xu);
+        load(v, n0, xv);
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const int k0 = 4 * ((tid + kThreads * q) % G);
+            if (QUADS) {
+                load_row4(g.S, k0, K, xs[q]);
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) xs[q][i] = g.S[min(k0 + i, K - 1)];
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < Q; ++q)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) xu[q][i] *= xs[q][i];
+        stage(xu, us);
+        stage(xv, vs);
     }
     __syncthreads();
-    const int r0 = 4 * (tid >> 4), c0 = 4 * (tid & 15);
-    float acc[4][4] = {};
-    for (int t = 0; t < g.k; ++t) {
-        const float4 u = *reinterpret_cast<const float4 *>(&us[t][r0]), w = *reinterpret_cast<const float4 *>(&vs[t][c0]);
-        const float uu[4] = {u.x, u.y, u.z, u.w}, ww[4] = {w.x, w.y, w.z, w.w};
+    const int row0 = (wave >> 1) * 32 + (lane & 15), col0 = (wave & 1) * 32, kk = lane >> 4;
+    const bool inside = m0 + TS <= g.m && n0 + TS <= g.n;  // uniform
+    auto at = [&](int i, int j) {  // column block i, row block j
+        return static_cast<uint64_t>(m0 + row0 + 16 * j) * g.n + (n0 + col0 + 16 * i + 4 * kk);
+    };
+    // (rows of out and minuend may start at any multiple of four bytes)
+    f32x4 acc[F][F], mv[F][F];
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+    for (int j = 0; j < F; ++j)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(uu[i], ww[j], acc[i][j]);
-    }
-    const bool vec = g.n % 4 == 0 && (reinterpret_cast<uintptr_t>(g.out) & 15u) == 0 &&
-                     (reinterpret_cast<uintptr_t>(g.minuend) & 15u) == 0;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int row = m0 + r0 + i, col = n0 + c0;
-        if (row >= g.m || col >= g.n) continue;
-        const uint64_t e = static_cast<uint64_t>(row) * g.n + col;
-        if (vec) {  // whole quads: n % 4 == 0
-            float4 x{acc[i][0], acc[i][1], acc[i][2], acc[i][3]};
-            if (g.minuend) {
-                const float4 mv = *reinterpret_cast<const float4 *>(g.minuend + e);
-                x = float4{mv.x - x.x, mv.y - x.y, mv.z - x.z, mv.w - x.w};
-            }
-            *reinterpret_cast<float4 *>(g.out + e) = x;
-        } else {
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                if (col + j < g.n) g.out[e + j] = g.minuend ? g.minuend[e + j] - acc[i][j] : acc[i][j];
+        for (int i = 0; i < F; ++i) {
+            acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if (SUB && inside) __builtin_memcpy(&mv[i][j], __builtin_assume_aligned(g.minuend + at(i, j), 4), 16);
         }
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+        f32x4 a[F], b[F];
+#pragma unroll
+        for (int i = 0; i < F; ++i) {
+            a[i] = *reinterpret_cast<const f32x4 *>(&vs[col0 + 16 * i + (lane & 15)][16 * s + 4 * kk]);
+            b[i] = *reinterpret_cast<const f32x4 *>(&us[row0 + 16 * i][16 * s + 4 * kk]);
+        }
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int i = 0; i < F; ++i)
+#pragma unroll
+                for (int j = 0; j < F; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][t], b[j][t], acc[i][j], 0, 0, 0);
+    }
+    if (inside) {
+#pragma unroll
+        for (int j = 0; j < F; ++j)
+#pragma unroll
+            for (int i = 0; i < F; ++i) {
+                const f32x4 x = SUB ? mv[i][j] - acc[i][j] : acc[i][j];
+                __builtin_memcpy(__builtin_assume_aligned(g.out + at(i, j), 4), &x, 16);
+            }
+        return;
+    }
+#pragma unroll
+    for (int j = 0; j < F; ++j)
+#pragma unroll
+        for (int i = 0; i < F; ++i) {
+            const int row = m0 + row0 + 16 * j, col = n0 + col0 + 16 * i + 4 * kk;
+            if (row >= g.m) continue;
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+                if (col + t < g.n) g.out[at(i, j) + t] = SUB ? g.minuend[at(i, j) + t] - acc[i][j][t] : acc[i][j][t];
+        }
+}
+
+template <bool PACKED, bool SUB>
+void low_rank(const ReconArgs &g, const PlaneSource &u, const PlaneSource &v, hipStream_t stream) {
+    const dim3 grid(static_cast<unsigned>(ceil_div(g.m, 64) * ceil_div(g.n, 64)));
+    auto go = [&](auto kern) { kern<<<grid, kThreads, 0, stream>>>(g, u, v); };
+    auto depth = [&](auto quads) {
+        constexpr bool Q = decltype(quads)::value;
+        if (g.k <= 16) go(recon_low_rank_kernel<1, PACKED, SUB, Q>);
+        else if constexpr (PACKED || Q) {
+            if (g.k <= 32) go(recon_low_rank_kernel<2, PACKED, SUB, Q>);
+            else if (g.k <= 48) go(recon_low_rank_kernel<3, PACKED, SUB, Q>);
+            else if (g.k <= 64) go(recon_low_rank_kernel<4, PACKED, SUB, Q>);
+            else if (g.k <= 96) go(recon_low_rank_kernel<6, PACKED, SUB, Q>);
+            else go(recon_low_rank_kernel<8, PACKED, SUB, Q>);
+        }
+    };
+    if (PACKED ? g.k % 4 == 0 : g.k >= 4) depth(std::true_type{});
+    else depth(std::false_type{});
+    BSQ_HIP(hipGetLastError());
+}
+
+void launch_low_rank(const ReconArgs &g, const PlaneSource &u, const PlaneSource &v, hipStream_t stream) {
+    const bool dense = u.dense && v.dense;
+    if (g.minuend) {
+        if (dense) low_rank<false, true>(g, u, v, stream);
+        else low_rank<true, true>(g, u, v, stream);
+    } else {
+        if (dense) low_rank<false, false>(g, u, v, stream);
+        else low_rank<true, false>(g, u, v, stream);
     }
 }
 
 }  // namespace
 
 namespace {
+// Which form a shape takes, with scratch or without, so that both give the same
+// bits.  FP32 sums to rank 64 at any size (8192 x 8192, rank 48 81 us against
+// 102 from two slices of pieces, rank 64 96 and 98; 512 x 1024, rank 64 4.4 and
+// 11.2), and to rank 128 while the 128 x 128 tiles of the other form would leave
+// CUs idle (2048 x 2048, 256 tiles, rank 128 14.7 and 16.5 us, rank 80 12.8 and
+// 16.2; 2048 x 4096, rank 80 21.8 and 19.5).
+bool low_rank_form(int m, int n, int k) {
+    return k <= 64 || (k <= 128 && ceil_div(m, T) * ceil_div(n, T) <= static_cast<uint64_t>(cu_count()));
+}
+// Whether packed factors are decoded ahead of the low-rank kernel (two launches,
+// 5 us) and not in each tile, which costs 0.012 us per rank and tile a CU:
+// 4096 x 4096, rank 64 39 us against 46, rank 8 27 against 25.
+bool decodes_first(int m, int n, int k) {
+    return ceil_div(m, 64) * ceil_div(n, 64) * k > 400ull * cu_count();
+}
+uint64_t dense_bytes(int rows, int k) { return ceil_div(static_cast<uint64_t>(rows) * k, 4) * 16; }
 int padded_rows(int rows) { return static_cast<int>(ceil_div(rows, 64) * 64); }
 int plane_groups(int k) { return static_cast<int>(ceil_div(k, BK) * KG); }
 }  // namespace
 
 uint64_t factor_plane_bytes(int m, int n, int k) {
-    if (k < BK) return 0;
+    if (low_rank_form(m, n, k)) return decodes_first(m, n, k) ? dense_bytes(m, k) + dense_bytes(n, k) : 0;
     return 2ull * 16 * plane_groups(k) * (static_cast<uint64_t>(padded_rows(m)) + padded_rows(n)) +
            sizeof(int) * (static_cast<uint64_t>(m) + n);
 }
@@ -498,20 +700,38 @@ void launch_reconstruct(const float *U, const float *S, const float *V, int m, i
                         float *out, hipStream_t stream) {
     BSQ_REQUIRE(m > 0 && n > 0 && k > 0 && U && S && V && out, "reconstruct: bad arguments");
     const ReconArgs g{U, S, V, minuend, out, m, n, k};
-    if (k < BK)
-        recon_low_rank_kernel<<<static_cast<unsigned>(ceil_div(m, 64) * ceil_div(n, 64)), kThreads, 0, stream>>>(g);
-    else
-        recon_kernel<<<static_cast<unsigned>(ceil_div(m, T) * ceil_div(n, T)), kThreads, 0, stream>>>(g);
+    if (low_rank_form(m, n, k)) {
+        launch_low_rank(g, PlaneSource{U, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, m, 0},
+                        PlaneSource{V, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, n, 0},
+                        stream);
+        return;
+    }
+    recon_kernel<<<static_cast<unsigned>(ceil_div(m, T) * ceil_div(n, T)), kThreads, 0, stream>>>(g);
     BSQ_HIP(hipGetLastError());
 }
 
-bool reconstruct_planes_supported(int k) { return k >= BK; }
-
 void launch_reconstruct_planes(const FactorSource &U, const float *S, const FactorSource &V, int m, int n, int k,
                                const float *minuend, float *out, void *planes, hipStream_t stream) {
-    BSQ_REQUIRE(m > 0 && n > 0 && reconstruct_planes_supported(k) && S && out && planes, "reconstruct: bad arguments");
+    BSQ_REQUIRE(m > 0 && n > 0 && k > 0 && S && out && (planes || factor_plane_bytes(m, n, k) == 0),
+                "reconstruct: bad arguments");
     for (const FactorSource *f : {&U, &V})
         BSQ_REQUIRE(f->dense || (f->codes && (f->scales_f32 || (f->scales_u8 && f->dq))), "reconstruct: missing factor");
+    if (low_rank_form(m, n, k)) {
+        auto source = [&](const FactorSource &f, int rows, uint64_t at) {
+            const float *dense = f.dense;
+            if (!dense && decodes_first(m, n, k)) {
+                auto *to = reinterpret_cast<float *>(static_cast<uint8_t *>(planes) + at);
+                launch_quant_decode(static_cast<uint64_t>(rows) * k, f.scales_u8 ? kMethodNF4DQ : kMethodNF4,
+                                    f.scales_f32, f.scales_u8, f.dq, f.codes, to, stream);
+                dense = to;
+            }
+            return PlaneSource{dense, f.codes, f.scales_f32, f.scales_u8, f.dq, nullptr, nullptr, nullptr, nullptr,
+                               rows, 0};
+        };
+        const PlaneSource u = source(U, m, 0), v = source(V, n, dense_bytes(m, k));
+        launch_low_rank(ReconArgs{nullptr, S, nullptr, minuend, out, m, n, k}, u, v, stream);
+        return;
+    }
     const int kgroups = plane_groups(k), up = padded_rows(m), vp = padded_rows(n);
     auto *uh = static_cast<u32x4 *>(planes);
     u32x4 *ul = uh + static_cast<uint64_t>(kgroups) * up, *vh = ul + static_cast<uint64_t>(kgroups) * up,

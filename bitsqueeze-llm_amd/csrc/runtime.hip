@@ -677,15 +677,10 @@ void compress_device(Runtime &rt, const float *d_in, bsq_device_packed_t *out, c
                                 sc.codes, &rt.meta->gmax, st);
         }
         mark(3);
-        // the reconstruction decodes U and V as it splits them; S, and all
-        // three at ranks outside that form, are decoded in place
-        const bool planes = reconstruct_planes_supported(rt.q);
-        for (int i = 0; i < 3; ++i) {
-            Section &sc = rt.sec[i];
-            if (sc.method == kMethodNone || te.capacity == 0 || (planes && i != SEC_S)) continue;
-            launch_quant_decode(sc.count, sc.method, sc.scales_f32, sc.scales_u8, &rt.meta->dq[i], sc.codes,
-                                sc.dense, st);
-        }
+        // the reconstruction decodes U and V itself; S is decoded in place
+        if (S.method != kMethodNone && te.capacity > 0)
+            launch_quant_decode(S.count, S.method, S.scales_f32, S.scales_u8, &rt.meta->dq[SEC_S], S.codes, S.dense,
+                                st);
         mark(4);
         if (te.capacity > 0) {
             // reconstruct + subtract fused (src/bitsqz_llm.cu:1141-1163)
@@ -695,11 +690,8 @@ void compress_device(Runtime &rt, const float *d_in, bsq_device_packed_t *out, c
                     if (sc.method == kMethodNone) return FactorSource{sc.dense};
                     return FactorSource{nullptr, sc.codes, sc.scales_f32, sc.scales_u8, &rt.meta->dq[i]};
                 };
-                if (planes)
-                    launch_reconstruct_planes(factor(SEC_U), S.dense, factor(SEC_V), rows, cols, rt.q, residual,
-                                              rt.d_err, rt.planes, st);
-                else
-                    launch_reconstruct(U.dense, S.dense, V.dense, rows, cols, rt.q, residual, rt.d_err, st);
+                launch_reconstruct_planes(factor(SEC_U), S.dense, factor(SEC_V), rows, cols, rt.q, residual,
+                                          rt.d_err, rt.planes, st);
             });
             mark(5);
             TopkArgs a;
@@ -869,30 +861,21 @@ void decompress_device(Runtime &rt, const bsq_device_packed_t &P, const bool has
     const uint32_t ke = has_error ? P.topk_k[1] : 0, ko = has_outlier ? P.topk_k[0] : 0;
     if (H.flags & kFlagSvd) {
         const int q = static_cast<uint16_t>(H.effective_rank);
-        const bool planes = reconstruct_planes_supported(q);  // U and V are decoded as they are split
-        const float *dense[3];
-        for (int i = 0; i < 3; ++i) {
-            dense[i] = P.d_dense[i];
-            if (dense[i] || (planes && i != SEC_S)) continue;
-            Section &sc = rt.sec[i];  // decompress runtime's dense U / S / V
-            const int method = (i == SEC_S) ? H.svd_s_format : H.svd_uv_format;
-            launch_quant_decode(P.count[i], method, P.d_scales_f32[i], P.d_scales_u8[i], P.d_dq_scale[i],
-                                P.d_codes[i], sc.dense, st);
-            dense[i] = sc.dense;
+        const float *s_dense = P.d_dense[SEC_S];  // the reconstruction decodes U and V itself
+        if (!s_dense) {
+            launch_quant_decode(P.count[SEC_S], H.svd_s_format, P.d_scales_f32[SEC_S], P.d_scales_u8[SEC_S],
+                                P.d_dq_scale[SEC_S], P.d_codes[SEC_S], rt.sec[SEC_S].dense, st);
+            s_dense = rt.sec[SEC_S].dense;
         }
         timed_launch(kTimeReconstruct, st, [&] {
-            if (!planes) {
-                launch_reconstruct(dense[SEC_U], dense[SEC_S], dense[SEC_V], rows, cols, q, nullptr, d_dst, st);
-                return;
-            }
             auto factor = [&](int i) {
-                if (dense[i]) return FactorSource{dense[i]};
+                if (P.d_dense[i]) return FactorSource{P.d_dense[i]};
                 const bool dq = H.svd_uv_format == kMethodNF4DQ;
                 return FactorSource{nullptr, P.d_codes[i], dq ? nullptr : P.d_scales_f32[i],
                                     dq ? P.d_scales_u8[i] : nullptr, P.d_dq_scale[i]};
             };
-            launch_reconstruct_planes(factor(SEC_U), dense[SEC_S], factor(SEC_V), rows, cols, q, nullptr, d_dst,
-                                      rt.planes, st);
+            launch_reconstruct_planes(factor(SEC_U), s_dense, factor(SEC_V), rows, cols, q, nullptr, d_dst, rt.planes,
+                                      st);
         });
     } else {
         const uint64_t N = static_cast<uint64_t>(rows) * cols;
