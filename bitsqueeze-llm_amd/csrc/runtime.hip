@@ -1250,8 +1250,20 @@ void decompress_host(Runtime &rt, const bitsqz_llm_array_t *c, float *d_dst) {
         P.topk_k[t] = h.num_topk_columns;
     }
 
-    // Every section is decoded as soon as it arrives (the staging of packed
-    // sections is shared).
+    // Packed U and V of the SVD path stay packed for the reconstruction, which
+    // decodes them itself, when both and a packed S fit the shared staging side
+    // by side; otherwise every section is decoded as soon as it arrives and the
+    // next one takes its place.  (Decoded here by launches of their own, they
+    // took 72 us of a 512 x 1024 rank 64 decode in place of 64.)
+    const uint64_t q_of = (c->flags & kFlagSvd) ? static_cast<uint16_t>(c->effective_rank) : 0;
+    const uint64_t uq = rows * q_of, vq = cols * q_of;
+    const uint64_t v_code_off = ceil_div(uq / 2 + 1, 256) * 256, v_scale_off = ceil_div(ceil_div(uq, kQuantBlock), 64) * 64;
+    const uint64_t s_code_off = v_code_off + ceil_div(vq / 2 + 1, 256) * 256,
+                   s_scale_off = v_scale_off + ceil_div(ceil_div(vq, kQuantBlock), 64) * 64;
+    const bool keep_packed = q_of > 0 && rt.quant_initialized && c->section_u.storage == BITSQZ_SECTION_QUANT &&
+                             c->section_v.storage == BITSQZ_SECTION_QUANT &&
+                             s_code_off + (q_of + 1) / 2 <= (N + 1) / 2 &&
+                             s_scale_off + ceil_div(q_of, kQuantBlock) <= ceil_div(N, kQuantBlock);
     auto stage_section = [&](int i, const bitsqz_section_t &s, int method, uint64_t count, float *dense_dst) {
         if (s.storage == BITSQZ_SECTION_FP32) {
             BSQ_REQUIRE(s.size == count * 4, "FP32 section size mismatch");
@@ -1269,14 +1281,25 @@ void decompress_host(Runtime &rt, const bitsqz_llm_array_t *c, float *d_dst) {
         // the header and block scales staged at once, the codes piecewise
         const bitsqz_section_t head{s.offset, 48 + ssz, s.storage};
         const uint8_t *pl = staged(head);
-        float *sc_f32 = rt.q_scales_f32;
-        uint8_t *sc_u8 = rt.q_scales_u8, *codes = rt.q_codes;
+        const bool packed = keep_packed && (i == SEC_U || i == SEC_V);
+        const uint64_t coff = !keep_packed ? 0 : (i == SEC_V ? v_code_off : (i == SEC_S ? s_code_off : 0));
+        const uint64_t soff = !keep_packed ? 0 : (i == SEC_V ? v_scale_off : (i == SEC_S ? s_scale_off : 0));
+        float *sc_f32 = rt.q_scales_f32 + soff;
+        uint8_t *sc_u8 = rt.q_scales_u8 + soff, *codes = rt.q_codes + coff;
         void *sdst = method == kMethodNF4 ? static_cast<void *>(sc_f32) : static_cast<void *>(sc_u8);
         BSQ_HIP(hipMemcpyAsync(sdst, pl + s.offset + 48, ssz, hipMemcpyHostToDevice, st));
         h2d_pieces(codes, s.offset + 48 + ssz, (count + 1) / 2, st);
         if (method == kMethodNF4DQ)
             BSQ_HIP(hipMemcpyAsync(&rt.meta->dq[i], pl + s.offset + 40, 4, hipMemcpyHostToDevice, st));
         P.count[i] = count;
+        if (packed) {
+            const bool dq = method == kMethodNF4DQ;
+            P.d_codes[i] = codes;
+            P.d_scales_f32[i] = dq ? nullptr : sc_f32;
+            P.d_scales_u8[i] = dq ? sc_u8 : nullptr;
+            P.d_dq_scale[i] = dq ? &rt.meta->dq[i] : nullptr;
+            return;
+        }
         // decode now (the staging buffers are shared between sections)
         launch_quant_decode(count, method, sc_f32, sc_u8, &rt.meta->dq[i], codes, dense_dst, st);
         P.d_dense[i] = dense_dst;

@@ -1,11 +1,11 @@
-"""The reconstruction from packed NF4 / NF4_DQ factors decoded inline
-(recon.hip) on the GPU.
+"""The reconstruction from packed NF4 / NF4_DQ factors (recon.hip) on the GPU.
 
   * Through the ABI, every section and the decode are checked bit for bit
-    against the oracle by `check_sections`: the decompress side decodes U and
-    V inside the reconstruction, and the result must equal the FP32
-    reconstruction of the decoded factors plus the error set, then the
-    outlier set (src/bitsqz_llm.cu:1341-1387).
+    against the oracle by `check_sections`: the decompress side hands U and V
+    to the reconstruction packed, which decodes them as it splits them (or, at
+    rank 64 of small matrices, as it stages them), and the result must equal
+    the reconstruction of the decoded FP32 factors plus the error set, then
+    the outlier set (src/bitsqz_llm.cu:1341-1387).
   * The device-resident decompress (packed U and V taken straight from the
     compress runtime) must give the same bytes.
 

@@ -42,6 +42,8 @@ def test_hand_over_by_size(k):
 
 @pytest.mark.parametrize("rows,cols,q,uv,s,ro,re", [
     (70, 131, 1, B.NF4, B.QUANT_NONE, 0.0, 0.05),
+    (40, 44, 40, B.NF4, B.NF4_DQ, 0.0, 0.05),            # the packed sections outgrow the host decode's staging
+    (66, 66, 24, B.NF4_DQ, B.NF4_DQ, 0.0, 0.05),         # and fit it but for their alignment
     (131, 70, 3, B.NF4_DQ, B.NF4, 0.02, 0.05),
     (129, 257, 8, B.NF4, B.NF4, 0.02, 0.03),
     (200, 300, 30, B.NF4_DQ, B.QUANT_NONE, 0.01, 0.03),
