@@ -303,8 +303,15 @@ uint64_t plan_bytes(int m, int n, int q, int niter, bool h2) {
 // scratch array of the no-allocation entry point holds every plan that it
 // held without the operand planes: one that would outgrow it only through
 // them keeps the FP32 products, in both entry points, so their results agree.
+// Small matrices keep them too, where every operand fits the FP32 kernels'
+// 16-byte transfers: there the two-piece form's launches (row scales, split,
+// reductions) cost more than its products save (64 x 64, rank 8 187 us a
+// factorisation against 216, 256 x 256 231 and 245, 384 x 384 253 and 253,
+// 512 x 512 296 and 255; rank 1, whose products go another way, 203 and 195).
 bool plan_uses_h2(int m, int n, int q, int niter) {
     if (!h2_supported(std::min(m, n))) return false;
+    const int k = std::max(1, std::min({q, m, n}));
+    if (std::max(m, n) < 384 && m % 16 == 0 && n % 16 == 0 && k % 4 == 0) return false;
     return plan_bytes(m, n, q, niter, true) <= kNoAllocScratchBytes ||
            plan_bytes(m, n, q, niter, false) > kNoAllocScratchBytes;
 }

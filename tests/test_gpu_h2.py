@@ -37,7 +37,9 @@ def svd_and_oracle(A, q, it):
 
 
 @pytest.mark.parametrize("m,n,q,it", [
-    (64, 64, 8, 1),      # one pair of slices, a single partial tile
+    (64, 64, 8, 1),      # (the FP32 products, which matrices as small as this keep)
+    (368, 240, 32, 1), (240, 384, 32, 1), (240, 256, 33, 2),  # either side of their limits
+    (64, 64, 7, 1),      # one pair of slices, a single partial tile
     (127, 65, 1, 2),     # K remainder 1 and 63, one column
     (129, 190, 63, 1), (190, 129, 64, 1), (257, 1283, 65, 2), (1283, 257, 129, 1),
     (1024, 320, 128, 0), (320, 1024, 256, 2), (700, 703, 300, 1),
