@@ -609,18 +609,16 @@ void encode_pass(const float *x, uint64_t n, float *scales_f32, uint8_t *scales_
         kern<<<grid, kThreads, 0, stream>>>(x, n, vec_ok, scales_f32, scales_u8, gmax, row_gmax, gmax_rows, dq_out,
                                             codes, flags_reset, sel);
     };
-    // one chunk a lane keeps the most workgroups and loads in flight (2048 x
-    // 4096 NF4 8.6 us, with four chunks 9.9; 1000 x 5003 6.4 and 9.3); four
+    // one chunk a lane keeps the most workgroups and loads in flight; four
     // share the scale chain and win once every resident workgroup has several
-    // tiles (4096 x 11008 NF4 43 and 41), with NF4_DQ's longer chain earlier
-    // (4096 x 4096 after a separation 19.1 and 17.5)
-    if (n >= (DQ ? 1ull << 24 : 1ull << 25)) {
-        if (sel) go(quant_encode_kernel<DQ, true, 4>, encode_grid<DQ, true, 4>(n));
-        else go(quant_encode_kernel<DQ, false, 4>, encode_grid<DQ, false, 4>(n));
-    } else {
-        if (sel) go(quant_encode_kernel<DQ, true, 1>, encode_grid<DQ, true, 1>(n));
-        else go(quant_encode_kernel<DQ, false, 1>, encode_grid<DQ, false, 1>(n));
-    }
+    // tiles.  One and four at 2^23, 2^24, 2^24.6 and 2^25 values (whole
+    // compress, inputs not in the caches): NF4 9.1 and 9.8, 16.1 and 16.1, 24.6
+    // and 23.2, 31.9 and 30.1 us; NF4_DQ 19.1 and 20.6, 32.3 and 32.8, 45.0 and
+    // 44.9, 58.7 and 57.8.  Behind a separation's bitmap they never win (2^24
+    // 37.6 and 37.8, 2^25 71.2 and 71.5).
+    if (sel) go(quant_encode_kernel<DQ, true, 1>, encode_grid<DQ, true, 1>(n));
+    else if (n >= 1ull << 25) go(quant_encode_kernel<DQ, false, 4>, encode_grid<DQ, false, 4>(n));
+    else go(quant_encode_kernel<DQ, false, 1>, encode_grid<DQ, false, 1>(n));
     BSQ_HIP(hipGetLastError());
 }
 }  // namespace

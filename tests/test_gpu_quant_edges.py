@@ -87,7 +87,7 @@ def below_two(rows, cols):
     return x
 
 
-@pytest.mark.parametrize("rows", [1, 33, 1 << 15])  # one chunk a lane, a tile's remainder, four chunks a lane
+@pytest.mark.parametrize("rows", [1, 33, 1 << 16])  # one chunk a lane, a tile's remainder, four chunks a lane
 def test_encode_largest_table_value(rows):
     x = below_two(rows, 512).ravel()
     check(x, B.NF4_DQ, B.quant_compress(x, B.NF4_DQ))
