@@ -11,7 +11,9 @@
 // reductions: 4096 x 11008 with q = 128 101 -> 47 us (A^T B) and 98 -> 47 us
 // (A B); 16384 x 14336 with q = 512 1986 -> 838 and 1590 -> 825 us, 0.86
 // PFLOP/s of f16 products (a large library bf16 product reaches 1.2 on this
-// card; the clock falls to 1.9 GHz under the matrix cores' power).
+// card).  There the clock falls to 1.9 GHz (2.3 to 2.5 in the memory-bound and
+// one-workgroup kernels beside them) and the matrix cores are busy in 0.43 to
+// 0.48 of the cycles.
 //
 // Scales.  Row i of A is scaled so that its largest magnitude falls in
 // [2^14, 2^15) (row_scale_kernel, once per matrix).  With TA = false that is
@@ -173,20 +175,18 @@ __host__ __device__ __forceinline__ int h2_owner(int64_t u, int64_t units, int r
 
 // Stream-K: the K slices of all tile rows, in pairs, are cut into equal
 // contiguous ranges; the tiles_n workgroups of a range run the same slices of
-// A against their own columns of B, side by side on one XCD, so A comes from
-// HBM once (with ranges cut over the tiles themselves the workgroups of a tile
-// row drift apart: 6.9 GB instead of 2.2 GB through the L2s' misses at
-// 14336 x 16384 x 512).  Each workgroup writes its partial sum of every tile
-// it touches and h2_reduce_kernel adds a tile's parts in order.
+// A against their own columns of B, side by side on one XCD, so they share A
+// in its L2 (16384 x 14336 with q = 512: 1.4 GB come from HBM for A B, of which
+// A is 0.94, and 4.5 GB for A^T B).  Each workgroup writes its partial sum of
+// every tile it touches and h2_reduce_kernel adds a tile's parts in order.
 //
 // 128 x 128 tiles, four waves of 64 x 64 in 32 x 32 blocks with both sums in
 // accumulator registers (128 of 256 a lane), so two workgroups share a CU and
 // one's staging and barriers run under the other's matrix instructions.
 // 128 x 256 and 256 x 128 tiles (one workgroup a CU, three quarters of the
 // operand bytes per product) measured the same within 3 %, as one 128 x 128
-// workgroup a CU does: the matrix cores' power, not the operands' way, sets
-// the rate.  Slices of 32 k: B's pieces go global -> LDS directly one slice
-// ahead; A's values are fetched into registers two slices ahead (row-major: a
+// workgroup a CU does.  Slices of 32 k: B's pieces go global -> LDS directly one
+// slice ahead; A's values are fetched into registers two slices ahead (row-major: a
 // lane takes eight consecutive k of two rows; A^T: eight k-rows of two
 // columns, so the transposition is only a choice of registers), then split and
 // written to LDS in the same [k group][row] units of 16 bytes that the
@@ -197,8 +197,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     __shared__ u32x4 a0[2 * KG * kPitchA], a1[2 * KG * kPitchA];  // h plane, l plane
     __shared__ __attribute__((aligned(1024))) u32x4 b0[2 * KG * T], b1[2 * KG * T];
     // vector loads of one A slice's values, at least: 16 bytes are the widest
-    // (64 bytes a lane of each of two rows), and 16 rows of A^T are a runtime
-    // stride apart.  Their addresses differ by lane, so none is a scalar load.
+    // (32 bytes a lane of each of two rows), and A^T's are one row apart, a
+    // runtime stride.  Their addresses differ by lane, so none is a scalar load.
     constexpr int kLoadsA = TA ? 16 : 4;
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;

@@ -16,12 +16,14 @@
 //
 // For 256 < k <= 512 it reduces the trailing 256 columns of a matrix whose
 // first k - 256 columns went one launch each (trd_step_kernel), applying that
-// kernel's last, pending update as it loads: a column costs 2.7 us here and
+// kernel's last, pending update as it loads: a column costs 3.0 us here and
 // 5.5 us and a launch gap there (rank 512 of 1500 x 1500, a whole round trip
 // 5245 -> 4680 us, rank 300 of 700 x 800 3440 -> 2850 with the shorter
-// products).  At NB = 8 the loop over block columns stays rolled and the
-// tiles lie in the L1 / L2 caches: unrolled they fit the registers but for
-// five, and a 256-column reduction took 780 us against 690.
+// products).  At NB = 8 the loop over block columns is unrolled as at the other
+// sizes (the build raises the unroller's limit for this file), the 36 elements
+// a lane in registers: 128 of them, nine more in scratch; 684 us for 256
+// columns.  The form with the pending update keeps 33 in scratch, with reloads
+// in the first blocks' columns: 755 us.
 #include "bsq_internal.hpp"
 #include "wave_ops.hpp"
 
