@@ -1341,6 +1341,7 @@ void decompress_host(Runtime &rt, const bitsqz_llm_array_t *c, float *d_dst) {
                             P.d_topk_val[0], has_out ? P.topk_k[0] : 0, rows, cols, d_dst, true, st);
     }
     BSQ_HIP(hipStreamSynchronize(st));
+    if (rt.factor_stream == st) rt.factor_stream = nullptr;  // nothing is in flight
 }
 
 template <typename F>
