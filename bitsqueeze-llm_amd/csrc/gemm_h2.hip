@@ -229,20 +229,13 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 
     float va[2][8];  // A values in flight
     float vs[TA ? 8 : 2];
-    // the scales of the next A slice: where the wait has no loads to spare
-    // they go out before the B transfers (with A^T their registers are not to
-    // be had that early: it spilled)
-    auto load_scales = [&]() __attribute__((always_inline)) {
-        asm volatile("" ::: "memory");
-        if constexpr (!TA) {
-#pragma unroll
-            for (int h = 0; h < 2; ++h) vs[h] = g.rs[min(ca.tm * T + 64 * h + (tid >> 2), g.M - 1)];
-        }
-    };
-    auto load_values = [&]() __attribute__((always_inline)) {
+    auto load_a = [&]() __attribute__((always_inline)) {
         const int m0 = ca.tm * T, k0 = ca.ks * BK;
         asm volatile("" ::: "memory");  // stays behind the DMA before it
         if constexpr (!TA) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) vs[h] = g.rs[min(m0 + 64 * h + (tid >> 2), g.M - 1)];
+            asm volatile("" ::: "memory");  // the scales first: the wait lets values alone stay in flight
             const int k = min(k0 + 8 * (tid & 3), g.K - 8);
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
@@ -348,20 +341,17 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         Frags f0, f1;
         fetch(f0, ac, bc, 0);
         stage_a(an);
-        load_scales();
         dma_b(bn);
-        load_values();
+        load_a();
         fetch(f1, ac, bc, 1);
         acc.multiply(f0);
         acc.multiply(f1);
     };
     if (n <= 0 || range >= g.ranges) return;  // uniform (ranges <= units and grid = ranges x tiles_n: does not occur)
-    load_scales();
-    load_values();
+    load_a();
     dma_b(b0);
     stage_a(a0);
-    load_scales();
-    load_values();
+    load_a();
     int left = n, c_pr = p0 - tile0 * g.pairs;
     for (int t = tile0; left > 0; ++t, c_pr = 0) {  // the range's tile rows
         const int here = min(g.pairs - c_pr, left);
