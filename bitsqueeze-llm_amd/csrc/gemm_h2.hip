@@ -13,7 +13,7 @@
 // PFLOP/s of f16 products (a large library bf16 product reaches 1.2 on this
 // card).  There the clock falls to 1.9 GHz (2.3 to 2.5 in the memory-bound and
 // one-workgroup kernels beside them) and the matrix cores are busy in 0.43 to
-// 0.48 of the cycles.
+// 0.5 of the cycles.
 //
 // Scales.  Row i of A is scaled so that its largest magnitude falls in
 // [2^14, 2^15) (row_scale_kernel, once per matrix).  With TA = false that is

@@ -1,7 +1,8 @@
-"""bsq_reconstruct_lowrank (recon.hip) at the edges of its kernels: ranks below
-32 (FP32 sums), slices of 32 with every kind of remainder, tiles of 128, rows
-of factors that start off 16 bytes, and the values whose two-piece form needs
-care: infinities, NaN, zero rows and rows of very different scale.
+"""bsq_reconstruct_lowrank (recon.hip) at the edges of its kernels: FP32 sums (at
+these sizes ranks to 128), the two-piece form above in slices of 32 with every
+kind of remainder, tiles of 64 and 128, rows of factors that start off 16 bytes,
+and the values whose two-piece form needs care: infinities, NaN, zero rows and
+rows of very different scale.
 
 Tolerance: an entry is a sum of k products of FP32 values, each carried to
 2^-22 of its row's scale at worst and summed in FP32: 2^-22 sqrt(k) of the
@@ -26,14 +27,15 @@ def exact(U, S, V):
 
 
 @pytest.mark.parametrize("m,n,k", [(1, 1, 1), (64, 64, 31), (65, 130, 17), (127, 129, 32), (129, 127, 33),
-                                   (128, 128, 63), (200, 261, 64), (261, 200, 95), (130, 259, 1030)])
+                                   (128, 128, 63), (200, 261, 64), (261, 200, 95), (129, 127, 129), (200, 261, 159), (261, 200, 160),
+                                   (130, 259, 1030)])
 def test_reconstruct_edges(m, n, k):
     U, S, V = factors(m, n, k, m + n + k)
     ref = exact(U, S, V)
     assert np.linalg.norm(B.reconstruct(U, S, V) - ref) <= 2e-6 * np.linalg.norm(ref)
 
 
-@pytest.mark.parametrize("k", [20, 40, 256])
+@pytest.mark.parametrize("k", [20, 40, 130, 131, 256])
 def test_reconstruct_non_finite_and_scales(k):
     U, S, V = factors(300, 200, k, k)
     U[7, 3], U[9, 5], U[20], V[30] = np.inf, np.nan, 0.0, 0.0
